@@ -307,13 +307,15 @@ def work(case: dict) -> dict:
 
 
 def tolerance(case: dict) -> dict:
+    # about four times the distance from exact() that was measured: fp32
+    # 2.8e-6 after 24 layers; bf16 modules 0.002-0.0046; bf16 models, whose
+    # layers carry on what earlier ones left, 0.007 after one layer, 0.014
+    # after two, 0.02 after four to seven, 0.03 after 24
     if case["dtype"] == "fp32":
         return {"rel": 1e-5}
-    # one bf16 rounding is 2^-9 at most; a layer rounds about ten times, and
-    # later layers carry what earlier ones left
     if case["kind"] in ("decode", "prefill"):
-        return {"rel": 1e-2 * math.sqrt(1 + case["layers"])}
-    return {"rel": 1e-2}
+        return {"rel": 2.5e-2 * math.sqrt(1 + case["layers"])}
+    return {"rel": 1.6e-2}
 
 
 def _linear64(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
