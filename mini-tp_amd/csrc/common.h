@@ -236,38 +236,79 @@ struct Partials {
   int64_t M, N;
 };
 
-// Sum over the splits of elements (row, col .. col + 7), added in split
+// Sum over the splits of elements (row, col .. col + W - 1), added in split
 // order (the order gemm_reduce_kernel uses), the loads of four splits in
-// flight at a time. col and N multiples of 4.
-__device__ __forceinline__ void sum_partials8(const Partials& q, int64_t row, int64_t col, float* v) {
+// flight at a time. W, col and N multiples of 4.
+template <int W>
+__device__ __forceinline__ void sum_partials(const Partials& q, int64_t row, int64_t col, float* v) {
   const int64_t mn = q.M * q.N, off = row * q.N + col;
   auto ld = [&](int s, float* o) {
-    const float4 a = *(const float4*)(q.p + s * mn + off), b = *(const float4*)(q.p + s * mn + off + 4);
-    o[0] = a.x;
-    o[1] = a.y;
-    o[2] = a.z;
-    o[3] = a.w;
-    o[4] = b.x;
-    o[5] = b.y;
-    o[6] = b.z;
-    o[7] = b.w;
+#pragma unroll
+    for (int h = 0; h < W / 4; ++h) {
+      const float4 a = *(const float4*)(q.p + s * mn + off + 4 * h);
+      o[4 * h] = a.x;
+      o[4 * h + 1] = a.y;
+      o[4 * h + 2] = a.z;
+      o[4 * h + 3] = a.w;
+    }
   };
   ld(0, v);
   int s = 1;
   for (; s + 4 <= q.S; s += 4) {
-    float t[4][8];
+    float t[4][W];
 #pragma unroll
     for (int u = 0; u < 4; ++u) ld(s + u, t[u]);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] += t[u][e];
+      for (int e = 0; e < W; ++e) v[e] += t[u][e];
   }
-  for (; s < q.S; ++s) {
-    float t[8];
-    ld(s, t);
+  // the last one to three splits, loaded together (a split past the end
+  // reads the last one again and is left out)
+  if (s >= q.S) return;
+  float t[3][W];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] += t[e];
+  for (int u = 0; u < 3; ++u) ld(s + u < q.S ? s + u : q.S - 1, t[u]);
+#pragma unroll
+  for (int u = 0; u < 3; ++u)
+    if (s + u < q.S)
+#pragma unroll
+      for (int e = 0; e < W; ++e) v[e] += t[u][e];
+}
+
+// W consecutive elements (W sizeof(T) a multiple of 8 bytes, aligned to it,
+// or to 16 when it is 16 or more) as floats, and back rounded to T.
+template <typename T, int W>
+__device__ __forceinline__ void load_vec(const T* p, float* v) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int h = 0; h < W / 4; ++h) {
+      const float4 a = *(const float4*)(p + 4 * h);
+      v[4 * h] = a.x;
+      v[4 * h + 1] = a.y;
+      v[4 * h + 2] = a.z;
+      v[4 * h + 3] = a.w;
+    }
+  } else if constexpr (W == 4) {
+    const uint2 a = *(const uint2*)p;
+    v[0] = __uint_as_float(a.x << 16);
+    v[1] = __uint_as_float(a.x & 0xffff0000u);
+    v[2] = __uint_as_float(a.y << 16);
+    v[3] = __uint_as_float(a.y & 0xffff0000u);
+  } else {
+    unpack16(*(const uint4*)p, v, (bf16*)nullptr);
+  }
+}
+template <typename T, int W>
+__device__ __forceinline__ void store_vec(T* p, const float* v) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int h = 0; h < W / 4; ++h) *(float4*)(p + 4 * h) = make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
+  } else if constexpr (W == 4) {
+    *(uint2*)p = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+  } else {
+    *(uint4*)p = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]),
+                            pack_bf16x2(v[6], v[7]));
   }
 }
 

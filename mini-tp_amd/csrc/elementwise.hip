@@ -164,11 +164,96 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const T* __restrict__ x, c
   }
 }
 
+// Rows of whole W-element pieces, one block per row: RMSNorm (NORM_PLAIN), or
+// the residual add first (x = dtype(x + delta) in place, layer.py:61-64) with
+// delta a row (NORM_ADD) or a split product's partials, their sum rounded to
+// the dtype as gemm_reduce_kernel stores it (NORM_ADD_PART). Each thread
+// reads and writes only its own elements, so out may alias delta. Rows of up
+// to 256 x KEEP pieces stay in registers between the sum of squares and the
+// scaling (no second read), the norm weights loaded before the reduction's
+// barrier. Memory-bound when rows are many (16,384 x 3,584 bf16, plain: 75 us
+// with scalar accesses and a second read, 46 us here, 5.1 TB/s), bound by its
+// load -> reduce -> store chain when they are few.
+enum { NORM_PLAIN = 0, NORM_ADD = 1, NORM_ADD_PART = 2 };
+template <typename T, int W, int MODE>
+__global__ __launch_bounds__(256) void norm_rows_kernel(const T* xin, T* x, const T* delta, Partials dp,
+                                                        const T* __restrict__ w, T* out, int64_t hidden, float eps) {
+  __shared__ float red[4];
+  constexpr int KEEP = 4;
+  const int64_t base = blockIdx.x * hidden;
+  const int n = (int)(hidden / W), tid = threadIdx.x;
+  float v[KEEP][W], wf[KEEP][W];
+  float ss = 0.f;
+  auto take = [&](int c, float* a) {
+    load_vec<T, W>((MODE == NORM_PLAIN ? xin : x) + base + c * W, a);
+    if constexpr (MODE != NORM_PLAIN) {
+      float d[W];
+      if constexpr (MODE == NORM_ADD_PART) {
+        sum_partials<W>(dp, blockIdx.x, c * W, d);
+#pragma unroll
+        for (int e = 0; e < W; ++e) d[e] = round_to<T>(d[e] + 0.f);
+      } else {
+        load_vec<T, W>(delta + base + c * W, d);
+      }
+#pragma unroll
+      for (int e = 0; e < W; ++e) a[e] = round_to<T>(add_rn(a[e], d[e]));
+      store_vec<T, W>(x + base + c * W, a);
+    }
+#pragma unroll
+    for (int e = 0; e < W; ++e) ss += mul_rn(a[e], a[e]);
+  };
+  auto give = [&](int c, const float* a, const float* g, float r) {
+    float o[W];
+#pragma unroll
+    for (int e = 0; e < W; ++e) o[e] = mul_rn(mul_rn(a[e], r), g[e]);
+    store_vec<T, W>(out + base + c * W, o);
+  };
+  const bool keep = n <= 256 * KEEP;
+  if (keep) {
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k)
+      if (tid + 256 * k < n) load_vec<T, W>(w + (tid + 256 * k) * W, wf[k]);
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k)
+      if (tid + 256 * k < n) take(tid + 256 * k, v[k]);
+  } else {
+    for (int c = tid; c < n; c += 256) take(c, v[0]);
+  }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  const float tot = (red[0] + red[1]) + (red[2] + red[3]);
+  const float r = __fdiv_rn(1.0f, __fsqrt_rn(add_rn(__fdiv_rn(tot, (float)hidden), eps)));
+  if (keep) {
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k)
+      if (tid + 256 * k < n) give(tid + 256 * k, v[k], wf[k], r);
+  } else {
+    for (int c = tid; c < n; c += 256) {
+      load_vec<T, W>((MODE == NORM_PLAIN ? xin : x) + base + c * W, v[0]);
+      load_vec<T, W>(w + c * W, wf[0]);
+      give(c, v[0], wf[0], r);
+    }
+  }
+}
+
+inline bool norm_vec_ok(int dtype, int64_t hidden, const void* a, const void* b, const void* c, const void* d) {
+  return hidden % (dtype == MINITP_F32 ? 4 : 8) == 0 && hidden < (1LL << 30) && aligned16(a) && aligned16(b) &&
+         aligned16(c) && aligned16(d);
+}
+
 int launch_rmsnorm(hipStream_t st, int dtype, const void* x, const void* w, void* out, int64_t rows, int64_t hidden,
                    float eps) {
   if (rows == 0) return MINITP_OK;
-  if (dtype == MINITP_F32)
+  const bool vec = norm_vec_ok(dtype, hidden, x, w, out, out);
+  if (dtype == MINITP_F32 && vec)
+    norm_rows_kernel<float, 4, NORM_PLAIN><<<(unsigned)rows, 256, 0, st>>>(
+        (const float*)x, nullptr, nullptr, Partials{}, (const float*)w, (float*)out, hidden, eps);
+  else if (dtype == MINITP_F32)
     rmsnorm_kernel<float><<<(unsigned)rows, 256, 0, st>>>((const float*)x, (const float*)w, (float*)out, hidden, eps);
+  else if (vec)
+    norm_rows_kernel<bf16, 8, NORM_PLAIN><<<(unsigned)rows, 256, 0, st>>>(
+        (const bf16*)x, nullptr, nullptr, Partials{}, (const bf16*)w, (bf16*)out, hidden, eps);
   else
     rmsnorm_kernel<bf16><<<(unsigned)rows, 256, 0, st>>>((const bf16*)x, (const bf16*)w, (bf16*)out, hidden, eps);
   MINITP_LAUNCH_CHECK();
@@ -202,66 +287,17 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(T* x, const T* delta, 
   }
 }
 
-// bf16 rows of hidden % 8 == 0: the same math in 16-byte pieces (8 elements per
-// load and store; a thread's elements are whole pieces).
-// PART: delta is the split-K partial product itself (the sum over the splits
-// rounded to bf16 as gemm_reduce_kernel stores it), not a bf16 row.
-template <bool PART>
-__global__ __launch_bounds__(256) void add_rmsnorm8_kernel(bf16* x, const bf16* delta, Partials dp,
-                                                           const bf16* __restrict__ w, bf16* out, int64_t hidden,
-                                                           float eps) {
-  __shared__ float red[4];
-  uint4* xr = reinterpret_cast<uint4*>(x + blockIdx.x * hidden);
-  const uint4* dr = reinterpret_cast<const uint4*>(delta + blockIdx.x * hidden);
-  uint4* orow = reinterpret_cast<uint4*>(out + blockIdx.x * hidden);
-  const uint4* wr = reinterpret_cast<const uint4*>(w);
-  const int64_t n8 = hidden / 8;
-  float ss = 0.f;
-  for (int64_t c = threadIdx.x; c < n8; c += 256) {
-    float a[8], d[8];
-    unpack16(xr[c], a, (bf16*)nullptr);
-    if constexpr (PART) {
-      float v[8];
-      sum_partials8(dp, blockIdx.x, c * 8, v);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) d[e] = round_to<bf16>(v[e] + 0.f);
-    } else {
-      unpack16(dr[c], d, (bf16*)nullptr);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      a[e] = round_to<bf16>(add_rn(a[e], d[e]));
-      ss += mul_rn(a[e], a[e]);
-    }
-    xr[c] = make_uint4(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(a[4], a[5]),
-                       pack_bf16x2(a[6], a[7]));
-  }
-  ss = wave_sum(ss);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  float tot = (red[0] + red[1]) + (red[2] + red[3]);
-  float r = __fdiv_rn(1.0f, __fsqrt_rn(add_rn(__fdiv_rn(tot, (float)hidden), eps)));
-  for (int64_t c = threadIdx.x; c < n8; c += 256) {
-    float a[8], wf[8], o[8];
-    unpack16(xr[c], a, (bf16*)nullptr);
-    unpack16(wr[c], wf, (bf16*)nullptr);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = mul_rn(mul_rn(a[e], r), wf[e]);
-    orow[c] = make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]),
-                         pack_bf16x2(o[6], o[7]));
-  }
-}
-
 int launch_add_rmsnorm(hipStream_t st, int dtype, void* x, const void* delta, const void* w, void* out, int64_t rows,
                        int64_t hidden, float eps) {
   if (rows == 0) return MINITP_OK;
-  if (dtype == MINITP_BF16 && hidden % 8 == 0 && aligned16(x) && aligned16(delta) && aligned16(w) && aligned16(out)) {
-    add_rmsnorm8_kernel<false><<<(unsigned)rows, 256, 0, st>>>((bf16*)x, (const bf16*)delta, Partials{}, (const bf16*)w,
-                                                               (bf16*)out, hidden, eps);
-    MINITP_LAUNCH_CHECK();
-    return MINITP_OK;
-  }
-  if (dtype == MINITP_F32)
+  const bool vec = norm_vec_ok(dtype, hidden, x, delta, w, out);
+  if (vec && dtype == MINITP_F32)
+    norm_rows_kernel<float, 4, NORM_ADD><<<(unsigned)rows, 256, 0, st>>>(
+        nullptr, (float*)x, (const float*)delta, Partials{}, (const float*)w, (float*)out, hidden, eps);
+  else if (vec)
+    norm_rows_kernel<bf16, 8, NORM_ADD><<<(unsigned)rows, 256, 0, st>>>(
+        nullptr, (bf16*)x, (const bf16*)delta, Partials{}, (const bf16*)w, (bf16*)out, hidden, eps);
+  else if (dtype == MINITP_F32)
     add_rmsnorm_kernel<float><<<(unsigned)rows, 256, 0, st>>>((float*)x, (const float*)delta, (const float*)w,
                                                               (float*)out, hidden, eps);
   else
@@ -304,49 +340,37 @@ __global__ void silu_mul_kernel(const T* gate, const T* up, int64_t ld_in, T* ou
   }
 }
 
-// bf16, 8 elements per thread through 16-byte loads and stores (rows of n % 8
-// == 0 elements, 16-byte aligned row starts); same math as silu_mul_kernel.
-// PART: gate and up are the split-K partial product of the [gate; up]
-// weight ([S][rows][2 n]), each sum rounded to bf16 as the GEMM stores it.
-template <bool PART>
-__global__ void silu_mul8_kernel(const bf16* gate, const bf16* up, int64_t ld_in, Partials gp, bf16* out,
-                                 int64_t ld_out, int64_t rows, int64_t n) {
-  const int64_t n8 = n / 8, total = rows * n8;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += stride) {
-    const int64_t r = i / n8, c = (i % n8) * 8;
-    float g[8], u[8], o[8];
-    if constexpr (PART) {
-      float vg[8], vu[8];
-      sum_partials8(gp, r, c, vg);
-      sum_partials8(gp, r, n + c, vu);
+// One 16-byte piece per thread (rows of whole pieces, 16-byte aligned row
+// starts; fewer than 2^31 pieces, so that the row division is 32-bit); same
+// math as silu_mul_kernel.
+template <typename T>
+__global__ __launch_bounds__(256) void silu_mulv_kernel(const T* gate, const T* up, int64_t ld_in, T* out,
+                                                        int64_t ld_out, int pieces, int total) {
+  constexpr int W = Vec<T>::N;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int64_t r = i / pieces, c = (i % pieces) * W;
+  float g[W], u[W], o[W];
+  load_vec<T, W>(gate + r * ld_in + c, g);
+  load_vec<T, W>(up + r * ld_in + c, u);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        g[e] = round_to<bf16>(vg[e] + 0.f);
-        u[e] = round_to<bf16>(vu[e] + 0.f);
-      }
-    } else {
-      const uint4 gv = *reinterpret_cast<const uint4*>(gate + r * ld_in + c);
-      const uint4 uv = *reinterpret_cast<const uint4*>(up + r * ld_in + c);
-      unpack16(gv, g, (bf16*)nullptr);
-      unpack16(uv, u, (bf16*)nullptr);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = swiglu<bf16>(g[e], u[e]);
-    *reinterpret_cast<uint4*>(out + r * ld_out + c) =
-        make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7]));
-  }
+  for (int e = 0; e < W; ++e) o[e] = swiglu<T>(g[e], u[e]);
+  store_vec<T, W>(out + r * ld_out + c, o);
 }
 
 int launch_silu_mul(hipStream_t st, int dtype, const void* gate, const void* up, int64_t ld_in, void* out,
                     int64_t ld_out, int64_t rows, int64_t n) {
   if (rows * n == 0) return MINITP_OK;
-  const bool vec = dtype == MINITP_BF16 && n % 8 == 0 && ld_in % 8 == 0 && ld_out % 8 == 0 && aligned16(gate) &&
-                   aligned16(up) && aligned16(out);
-  if (vec) {
-    const int grid8 = (int)std::min<int64_t>(cdiv(rows * (n / 8), 256), 65536);
-    silu_mul8_kernel<false><<<grid8, 256, 0, st>>>((const bf16*)gate, (const bf16*)up, ld_in, Partials{}, (bf16*)out,
-                                                   ld_out, rows, n);
+  const int64_t w = dtype == MINITP_F32 ? 4 : 8, total = rows * (n / w);
+  if (n % w == 0 && ld_in % w == 0 && ld_out % w == 0 && total < (1LL << 31) - 256 && aligned16(gate) &&
+      aligned16(up) && aligned16(out)) {
+    const unsigned grid = (unsigned)cdiv(total, 256);
+    if (dtype == MINITP_F32)
+      silu_mulv_kernel<float><<<grid, 256, 0, st>>>((const float*)gate, (const float*)up, ld_in, (float*)out, ld_out,
+                                                    (int)(n / w), (int)total);
+    else
+      silu_mulv_kernel<bf16><<<grid, 256, 0, st>>>((const bf16*)gate, (const bf16*)up, ld_in, (bf16*)out, ld_out,
+                                                   (int)(n / w), (int)total);
     MINITP_LAUNCH_CHECK();
     return MINITP_OK;
   }
@@ -361,28 +385,21 @@ int launch_silu_mul(hipStream_t st, int dtype, const void* gate, const void* up,
   return MINITP_OK;
 }
 
-int launch_add_rmsnorm_partials(hipStream_t st, void* x, const Partials& delta, const void* w, void* out,
+int launch_add_rmsnorm_partials(hipStream_t st, int dtype, void* x, const Partials& delta, const void* w, void* out,
                                 int64_t hidden, float eps) {
   if (delta.M == 0) return MINITP_OK;
-  if (delta.N != hidden || hidden % 8 != 0 || delta.S < 1 || !aligned16(x) || !aligned16(delta.p) || !aligned16(w) ||
-      !aligned16(out)) {
+  if (delta.N != hidden || delta.S < 1 || !norm_vec_ok(dtype, hidden, x, delta.p, w, out)) {
     set_error("add_rmsnorm from partials: hidden %lld, partial width %lld", (long long)hidden, (long long)delta.N);
     return MINITP_ERR_UNSUPPORTED;
   }
-  add_rmsnorm8_kernel<true><<<(unsigned)delta.M, 256, 0, st>>>((bf16*)x, nullptr, delta, (const bf16*)w, (bf16*)out,
-                                                              hidden, eps);
-  MINITP_LAUNCH_CHECK();
-  return MINITP_OK;
-}
-
-int launch_silu_mul_partials(hipStream_t st, const Partials& gu, void* out, int64_t ld_out, int64_t n) {
-  if (gu.M * n == 0) return MINITP_OK;
-  if (gu.N != 2 * n || n % 8 != 0 || ld_out % 8 != 0 || gu.S < 1 || !aligned16(gu.p) || !aligned16(out)) {
-    set_error("silu_mul from partials: n %lld, partial width %lld", (long long)n, (long long)gu.N);
-    return MINITP_ERR_UNSUPPORTED;
-  }
-  const int grid8 = (int)std::min<int64_t>(cdiv(gu.M * (n / 8), 256), 65536);
-  silu_mul8_kernel<true><<<grid8, 256, 0, st>>>(nullptr, nullptr, 0, gu, (bf16*)out, ld_out, gu.M, n);
+  // (4-element pieces of the partials: 0.5B rows then keep 224 of a block's
+  // threads loading instead of 112)
+  if (dtype == MINITP_F32)
+    norm_rows_kernel<float, 4, NORM_ADD_PART><<<(unsigned)delta.M, 256, 0, st>>>(
+        nullptr, (float*)x, nullptr, delta, (const float*)w, (float*)out, hidden, eps);
+  else
+    norm_rows_kernel<bf16, 4, NORM_ADD_PART><<<(unsigned)delta.M, 256, 0, st>>>(
+        nullptr, (bf16*)x, nullptr, delta, (const bf16*)w, (bf16*)out, hidden, eps);
   MINITP_LAUNCH_CHECK();
   return MINITP_OK;
 }

@@ -1,27 +1,33 @@
 // Prefill / batched linear layers: y[M, N] = epilogue(x[M, K] W[N, K]^T (+ bias)).
 //
-// MFMA tiling for CDNA (wave64): a 256-thread block owns a BM x BN output
-// tile (128 x 128 for large M, 64 x 64 when M is small); its 4 waves form a
-// 2 x 2 grid of wave tiles made of 32 x 32 MFMA accumulators (16 fp32
-// registers per lane each). Both operands are K-contiguous in memory (x rows
-// and W rows), the layout the MFMA A/B fragments want, so nothing is
-// transposed. K advances in chunks of 256 bytes per row staged in LDS; the
-// global loads of the next DEPTH chunks are in flight (in registers) while a
-// chunk's MFMAs run. The loads
-// are buffer loads whose lanes past the matrix (rows beyond M or N, K beyond
-// the split) get an out-of-range offset and read zeros: no load sits behind
-// a branch, so the compiler can count them precisely instead of waiting for
-// all of them before the next ones issue. Rows are padded by 16 bytes in LDS
-// to spread the MFMA fragment reads over the banks.
-//   bf16: v_mfma_f32_32x32x16_bf16 (A/B: 8 bf16 per lane, k = 8*(lane/32)+i)
-//   fp32: v_mfma_f32_32x32x2f32     (A/B: 1 float per lane, k = lane/32)
-// Accumulator layout: lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4,
-// column l%32.
+// MFMA tiling for CDNA4 (wave64). A block owns a BM x BN output tile (32 x 64
+// to 256 x 128) made of 64 x 64 wave tiles (2 x 2 MFMA accumulators of
+// 32 x 32; 32 x 64 wave tiles for few rows), with WK waves sharing each wave
+// tile's K: wave group g takes every WK-th
+// 16-byte substep of a stage and the groups' sums are added in group order at
+// the end (a fixed order). Both operands are K-contiguous in memory (x rows
+// and W rows), the layout the MFMA fragments want, so nothing is transposed:
+//   bf16: v_mfma_f32_32x32x16_bf16 (8 bf16 per lane and operand, k = 8*(lane/32)+i)
+//   fp32: 4 x v_mfma_f32_32x32x2f32 per 16 bytes (lane half h holds k 4h .. 4h+3
+//         of 8; MFMA i takes element i of both halves)
+// W is the MFMA's A operand and x its B operand, so lane l, register r is
+// output row l % 32 and column 8*(r/4) + 4*(l/32) + r%4: four consecutive
+// columns per register quad, stored as one piece.
 //
-// Small M (prefill of one short prompt, batched decode) leaves few output
-// tiles, so K is split over blockIdx.z: each split writes fp32 partial sums
-// to a workspace and gemm_reduce_kernel adds them in split order (a fixed
-// order, so results do not depend on timing) and applies the epilogue.
+// K advances in stages of 128 bytes per row, kept in a ring of STAGES LDS
+// buffers that global memory is loaded into directly (buffer_load_dwordx4 ...
+// lds: no registers, no LDS write instructions); each 16-byte chunk c of row r
+// sits at position c ^ (r / 2) % 8, so the lanes reading one fragment column
+// spread over all banks. STAGES - 1 stages are in flight: a wave waits for its own share of
+// the stage it reads next by count (vmcnt), and one barrier per stage both
+// publishes that stage and frees the previous one.
+//
+// Few output tiles (short prompts, batched decode) split K over blocks as
+// well: each split writes fp32 partial sums to a workspace, which
+// gemm_reduce_kernel, or the kernel that consumes the product, adds in split
+// order (fixed, so results do not depend on timing).
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -30,381 +36,530 @@ namespace minitp {
 namespace {
 
 constexpr int OUT_PARTIAL = 100;  // epilogue: fp32 split-K partials
-// epilogue: SwiGLU of a [gate; up] weight (2N rows): tile column bx holds
-// outputs [bx BN / 2, + BN / 2), its first BN / 2 B rows the gate rows and
-// the rest the matching up rows, so waves wn = 0 hold gate and wn = 1 up
+// epilogue: SwiGLU of a [gate; up] weight (2N rows): per 64 tile columns, 32
+// gate rows then the 32 matching up rows, so a wave's two column fragments
+// are a gate fragment and its up fragment
 constexpr int OUT_SWIGLU = 101;
-constexpr uint32_t OOB = 0xffffffffu;  // lane offset that reads zeros
-
-template <int AUX>
-__device__ __forceinline__ uint4 gemm_load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, AUX));
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-// weight loads of gemm_kernel: plain (non-temporal measured slower: 0.5B
-// 128-token TTFT 1.41-1.42 against 1.38 ms, 7B 512 tokens 11.55 against 11.28)
-#ifndef MINITP_GEMM_NT_LOADS
-#define MINITP_GEMM_NT_LOADS 0
-#endif
-constexpr int GEMM_W_AUX = MINITP_GEMM_NT_LOADS ? 2 : 0;
-// chunks in flight: register budget of the prefetch (LA + LB uint4 each)
-// (one chunk ahead measured best at the 0.5B prompt and 7B prefill shapes;
-// two to four chunks were slower, also in a form whose loop the compiler
-// counts exactly, waiting only for the chunk it stashes next)
-#ifndef MINITP_GEMM_DEPTH_LARGE
-#define MINITP_GEMM_DEPTH_LARGE 1
-#endif
-#ifndef MINITP_GEMM_DEPTH_SMALL
-#define MINITP_GEMM_DEPTH_SMALL 1
-#endif
-// output tile of the small-M GEMMs (M < 512)
-#ifndef MINITP_GEMM_SMALL_BM
-#define MINITP_GEMM_SMALL_BM 64
-#endif
-#ifndef MINITP_GEMM_SMALL_BN
-#define MINITP_GEMM_SMALL_BN 64
-#endif
-template <int BM>
-constexpr int depth() {
-  return BM >= 128 ? MINITP_GEMM_DEPTH_LARGE : MINITP_GEMM_DEPTH_SMALL;
-}
-// bytes of K per row per LDS chunk: 256 for 64 x 64 tiles, 128 for 128 x 128
-// (both operand tiles of a chunk stay under 40 KiB of LDS)
-template <int BM>
-constexpr int chunk_bytes() {
-  return BM >= 128 ? 128 : 256;
-}
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8_k __attribute__((ext_vector_type(8)));
 
 template <typename T>
-struct Mfma;
-
-typedef __bf16 bf16x8_k __attribute__((ext_vector_type(8)));
-// gfx950's 32x32x16: lane l holds A[l % 32][8 (l / 32) .. + 7] and the same
-// k range of B column l % 32, one 16-byte LDS read each
+__device__ __forceinline__ f32x16 mfma_step(const u32x4& a, const u32x4& b, f32x16 c);
 template <>
-struct Mfma<bf16> {
-  static constexpr int KSTEP = 16;  // k per instruction
-  __device__ static f32x16 step(const char* a_row, const char* b_row, int ks, int lane, f32x16 c) {
-    const int off = (ks * KSTEP + (lane >> 5) * 8) * 2;
-    const bf16x8_k a = *reinterpret_cast<const bf16x8_k*>(a_row + off);
-    const bf16x8_k b = *reinterpret_cast<const bf16x8_k*>(b_row + off);
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
+__device__ __forceinline__ f32x16 mfma_step<bf16>(const u32x4& a, const u32x4& b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_k, a), __builtin_bit_cast(bf16x8_k, b), c,
+                                                 0, 0, 0);
+}
+template <>
+__device__ __forceinline__ f32x16 mfma_step<float>(const u32x4& a, const u32x4& b, f32x16 c) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[i]), __uint_as_float(b[i]), c, 0, 0, 0);
+  return c;
+}
+
+// Lane offsets past a resource (the load writes zeros to LDS). ROW_OOB marks a
+// row past the matrix, and stays past any resource that ends below it with a
+// K offset added; K_OOB, never offset further, is past every resource (their
+// spans are multiples of 16 bytes below 4 GiB).
+constexpr uint32_t ROW_OOB = 0xF0000000u, K_OOB = 0xFFFFFFF0u;
+
+// 16 bytes per lane from the resource at voff straight into LDS: lane l's
+// bytes land at lds_addr + 16 l (wave-uniform, in m0). NT: non-temporal. asm, so that the
+// compiler does not wait for these loads at every LDS read: the kernel waits
+// for them itself, by count.
+template <bool NT>
+__device__ __forceinline__ void load16_lds(u32x4 r, uint32_t voff, uint32_t lds_addr) {
+  if constexpr (NT)
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen nt lds" ::"v"(voff), "s"(r), "{m0}"(lds_addr) : "memory");
+  else
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(lds_addr) : "memory");
+}
+
+__device__ __forceinline__ u32x4 rsrc_span(const void* base, uint32_t bytes) {
+  const uint64_t p = (uint64_t)base;
+  u32x4 r;
+  r.x = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)p);
+  r.y = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));  // stride 0
+  r.z = (uint32_t)__builtin_amdgcn_readfirstlane(bytes);
+  r.w = 0x00020000u;
+  return r;
+}
+
+// this wave's older stage loads have landed (all but the newest N) and its
+// LDS reads are done, then the block barrier
+template <int N>
+__device__ __forceinline__ void stage_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Tile shape of a launch: BM x BN outputs, WK waves per wave tile (64 columns,
+// 64 rows or all BM = 32), a ring of STAGES, non-temporal loads (NT).
+constexpr int KCH = 8;  // 16-byte chunks of K per row and stage
+template <int BM_, int BN_, int WK_, int STAGES_, bool NT_ = false>
+struct Tile {
+  static constexpr bool NT = NT_;
+  static constexpr int BM = BM_, BN = BN_, WK = WK_, STAGES = STAGES_;
+  static constexpr int FM = BM >= 64 ? 2 : 1;  // 32-row fragments per wave tile
+  static constexpr int WM = BM / (32 * FM), WN = BN / 64, NW = WM * WN * WK, THREADS = 64 * NW;
+  static constexpr int ROWB = KCH * 16;
+  static constexpr int STAGE_BYTES = (BM + BN) * ROWB;
+  static constexpr int RING_BYTES = STAGES * STAGE_BYTES, XCH_BYTES = WM * WN * (WK - 1) * FM * 8192;
+  static constexpr int LDS_BYTES = RING_BYTES > XCH_BYTES ? RING_BYTES : XCH_BYTES;
+  static constexpr int PIECE_ROWS = 64 / KCH;                   // rows of one 1 KiB load
+  static constexpr int PPW = (BM + BN) / PIECE_ROWS / NW;       // loads per wave and stage
+  static_assert((BM + BN) % (PIECE_ROWS * NW) == 0, "a stage splits evenly over the waves");
+  static_assert((STAGES - 2) * PPW < 64, "vmcnt counts six bits");
+  static_assert((KCH / 2) % WK == 0, "substeps split evenly over the wave groups");
 };
 
-template <>
-struct Mfma<float> {
-  static constexpr int KSTEP = 2;
-  __device__ static f32x16 step(const char* a_row, const char* b_row, int ks, int lane, f32x16 c) {
-    const int off = (ks * KSTEP + (lane >> 5)) * 4;
-    float a = *reinterpret_cast<const float*>(a_row + off);
-    float b = *reinterpret_cast<const float*>(b_row + off);
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-};
-
-// Block (bx, by, z): output tile (by * BM, bx * BN), K range [z kper, (z + 1)
-// kper). kper is a multiple of the chunk (KCB bytes).
-template <typename T, int BM, int BN, int OUT>
-__global__ __launch_bounds__(256) void gemm_kernel(const T* __restrict__ x, int64_t ldx, const T* __restrict__ w,
-                                                   const T* __restrict__ bias, T* y, int64_t ldy, const T* aux,
-                                                   float* part, int64_t M, int64_t N, int64_t K, int64_t kper,
-                                                   const StepState* state) {
+// Block b: split b / (tiles), tile b % tiles in XCD-aware order. Blocks go to
+// the 8 XCDs round-robin and each XCD has its own L2, so XCD b % 8 takes a
+// contiguous range of (split, tile) items, row tiles fastest inside groups of
+// 8: the row tiles that share a W panel run on one XCD at the same time.
+template <typename T, typename C, int OUT>
+__global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ x, int64_t ldx,
+                                                          const T* __restrict__ w, const T* __restrict__ bias, T* y,
+                                                          int64_t ldy, const T* aux, float* part, int M, int N, int K,
+                                                          int kper, int tiles_m, int tiles_n, int items,
+                                                          const StepState* state) {
+  constexpr int BM = C::BM, BN = C::BN, WK = C::WK, STAGES = C::STAGES, PPW = C::PPW;
+  constexpr int FM = C::FM, WN = C::WN, ROWB = C::ROWB, ES = (int)sizeof(T), V = 16 / ES, TK = KCH * V;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
   if (state != nullptr) y = (T*)state->args.logits;
-  constexpr int KCB = chunk_bytes<BM>(), ROWB = KCB + 16;
-  constexpr int V = Vec<T>::N;          // elements per 16 B
-  constexpr int KCE = KCB / sizeof(T);  // elements of K per chunk
-  constexpr int CPR = KCB / 16;         // 16-byte pieces per row per chunk
-  constexpr int LA = BM * CPR / 256, LB = BN * CPR / 256;  // pieces per thread
-  constexpr int FM = BM / 64, FN = BN / 64;                // 32 x 32 fragments per wave
-  __shared__ __attribute__((aligned(16))) char As[BM * ROWB];
-  __shared__ __attribute__((aligned(16))) char Bs[BN * ROWB];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
-  const int64_t kb = (int64_t)blockIdx.z * kper;
-  const int64_t ke = kb + kper < K ? kb + kper : K;
+  const int per_xcd = (items + 7) >> 3;
+  const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || item >= items) return;
+  const int tiles = tiles_m * tiles_n;
+  const int z = item / tiles, t = item - z * tiles;
+  const int group = t / (8 * tiles_n), first_m = group * 8, gsz = min(tiles_m - first_m, 8);
+  const int in_group = t - group * 8 * tiles_n;
+  const int m0 = (first_m + in_group % gsz) * BM, tn = in_group / gsz;
+  const int kb = z * kper, ke = min(kb + kper, K);
 
-  f32x16 acc[FM][FN];
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave / (C::WM * WN), wm = wave / WN % C::WM, wn = wave % WN;
+
+  // the tile's rows of x and of W as buffers; W row r of the tile
+  constexpr int BNO = OUT == OUT_SWIGLU ? BN / 2 : BN;  // output columns
+  const int n0 = tn * BNO;
+  auto w_row = [&](int r) -> int64_t {  // relative to n0, -1: past the matrix
+    if (OUT == OUT_SWIGLU) {
+      const int c = (r >> 6) * 32 + (r & 31);
+      return n0 + c < N ? ((r & 32) ? (int64_t)N + c : c) : -1;
+    }
+    return n0 + r < N ? r : -1;
+  };
+  const int x_rows = min(M - m0, BM);
+  const int64_t w_rows = OUT == OUT_SWIGLU ? (int64_t)2 * N - n0 : min(N - n0, BN);
+  const uint32_t x_bytes = (uint32_t)(((int64_t)(x_rows - 1) * ldx + K) * ES);
+  const uint32_t w_bytes = (uint32_t)(w_rows * K * ES);
+  const u32x4 xq = rsrc_span(x + (int64_t)m0 * ldx, x_bytes);
+  const u32x4 wq = rsrc_span(w + (int64_t)n0 * K, w_bytes);
+  // rows past the matrix read zeros; where a tile spans nearly 4 GiB, its
+  // last row again (their outputs are not stored either way)
+  const uint32_t x_pad = x_bytes <= ROW_OOB ? ROW_OOB : (uint32_t)((int64_t)(x_rows - 1) * ldx * ES);
+  const uint32_t w_pad = w_bytes <= ROW_OOB ? ROW_OOB : 0u;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  constexpr int A_BYTES = BM * ROWB;
+  auto swz = [](int r) { return (r >> 1) & 7; };
+  uint32_t voff[PPW];  // byte offset of the lane's chunk at k = 0
+  int kc[PPW];         // its first k
+#pragma unroll
+  for (int j = 0; j < PPW; ++j) {
+    const int p = wave * PPW + j;
+    const bool is_w = p >= BM / C::PIECE_ROWS;
+    const int r = C::PIECE_ROWS * (is_w ? p - BM / C::PIECE_ROWS : p) + lane / KCH;
+    const int c = (lane % KCH) ^ swz(r);
+    kc[j] = c * V;
+    if (!is_w) {
+      voff[j] = r < x_rows ? (uint32_t)(((int64_t)r * ldx + c * V) * ES) : x_pad;
+    } else {
+      const int64_t wr = w_row(r);
+      voff[j] = wr >= 0 ? (uint32_t)((wr * K + c * V) * ES) : w_pad;
+    }
+  }
+  const int nk = (ke - kb + TK - 1) / TK;
+  // (chunks past the split's end read zeros: steps past the last load nothing,
+  // so that every step issues the same number of loads and the waits can
+  // count them)
+  auto issue = [&](int step, int stage) {
+    const int k0 = kb + step * TK;
+    const uint32_t base = lds0 + stage * C::STAGE_BYTES + wave * PPW * 1024;
+#pragma unroll
+    for (int j = 0; j < PPW; ++j)
+      load16_lds<C::NT>(wave * PPW + j >= BM / C::PIECE_ROWS ? wq : xq, k0 + kc[j] < ke ? voff[j] + (uint32_t)(k0 * ES) : K_OOB,
+                 (uint32_t)__builtin_amdgcn_readfirstlane(base + j * 1024));
+  };
+
+  f32x16 acc[FM][2];  // [x fragment][W fragment]
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  constexpr int DEPTH = depth<BM>();
-  constexpr int ES = (int)sizeof(T);
-  // x rows [0, M) and W rows [0, N) as buffers; a lane's piece is read only
-  // when its row exists and its K lies inside this block's split
-  const __amdgpu_buffer_rsrc_t xr = span_rsrc(x, (uint32_t)(((M - 1) * ldx + K) * ES));
-  const __amdgpu_buffer_rsrc_t wr = span_rsrc(w, (uint32_t)((OUT == OUT_SWIGLU ? 2 : 1) * N * K * ES));
-  uint4 ra[DEPTH][LA], rb[DEPTH][LB];
-  auto load = [&](int64_t k0, uint4(&a)[LA], uint4(&bb)[LB]) {
+  const int ar = wm * (32 * FM) + (lane & 31), br = wn * 64 + (lane & 31);
+  // (rows 32 apart share the swizzle)
+  const int a_off = ar * ROWB, b_off = A_BYTES + br * ROWB, a_swz = swz(ar), b_swz = swz(br);
+  constexpr int KS = KCH / 2 / WK;  // substeps of a stage per wave group
+#pragma unroll 1
+  for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
+  int rd = 0, wr_stage = STAGES - 1;
+  for (int kt = 0; kt < nk; ++kt) {
+    stage_barrier<(STAGES - 2) * PPW>();
+    issue(kt + STAGES - 1, wr_stage);
+    const char* st = lds + rd * C::STAGE_BYTES;
+    u32x4 av[2][FM], bv[2][2];
+    auto fetch = [&](int s, u32x4(&a)[FM], u32x4(&b)[2]) {
+      const int c = (s * WK + wk) * 2 + half;
 #pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      const int c = tid + i * 256, row = c / CPR, pc = c % CPR;
-      const int64_t k = k0 + pc * V;
-      const bool ok = m0 + row < M && k < ke;
-      a[i] = gemm_load16<0>(xr, ok ? (uint32_t)(((m0 + row) * ldx + k) * ES) : OOB);
-    }
+      for (int i = 0; i < FM; ++i) a[i] = *(const u32x4*)(st + a_off + i * 32 * ROWB + ((c ^ a_swz) << 4));
 #pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int c = tid + i * 256, row = c / CPR, pc = c % CPR;
-      const int64_t k = k0 + pc * V;
-      int64_t wrow = n0 + row;
-      bool ok = wrow < N && k < ke;
-      if constexpr (OUT == OUT_SWIGLU) {
-        const int64_t j = (int64_t)blockIdx.x * (BN / 2) + row % (BN / 2);
-        wrow = row < BN / 2 ? j : N + j;
-        ok = j < N && k < ke;
-      }
-      bb[i] = gemm_load16<GEMM_W_AUX>(wr, ok ? (uint32_t)((wrow * K + k) * ES) : OOB);
-    }
-  };
-  auto stash = [&](const uint4(&a)[LA], const uint4(&bb)[LB]) {
+      for (int j = 0; j < 2; ++j) b[j] = *(const u32x4*)(st + b_off + j * 32 * ROWB + ((c ^ b_swz) << 4));
+    };
+    fetch(0, av[0], bv[0]);
 #pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      const int c = tid + i * 256, row = c / CPR, pc = c % CPR;
-      *reinterpret_cast<uint4*>(As + row * ROWB + pc * 16) = a[i];
-    }
-#pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int c = tid + i * 256, row = c / CPR, pc = c % CPR;
-      *reinterpret_cast<uint4*>(Bs + row * ROWB + pc * 16) = bb[i];
-    }
-  };
-
-  // chunk c of the split lives in register slot c % DEPTH (loads past the
-  // split read zeros and are never stashed)
-#pragma unroll
-  for (int d = 0; d < DEPTH; ++d) load(kb + (int64_t)d * KCE, ra[d], rb[d]);
-  for (int64_t k0 = kb; k0 < ke; k0 += (int64_t)DEPTH * KCE) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      const int64_t kc = k0 + (int64_t)d * KCE;
-      if (kc >= ke) break;
-      stash(ra[d], rb[d]);
-      __syncthreads();
-      if (kc + DEPTH * KCE < ke) load(kc + (int64_t)DEPTH * KCE, ra[d], rb[d]);  // in flight for later chunks
-#pragma unroll
-      for (int ks = 0; ks < KCE / Mfma<T>::KSTEP; ++ks) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) {
-            const char* a_row = As + (wm * (BM / 2) + i * 32 + (lane & 31)) * ROWB;
-            const char* b_row = Bs + (wn * (BN / 2) + j * 32 + (lane & 31)) * ROWB;
-            acc[i][j] = Mfma<T>::step(a_row, b_row, ks, lane, acc[i][j]);
-          }
-      }
-      __syncthreads();
-    }
-  }
-
-  if constexpr (OUT == OUT_SWIGLU) {
-    // the up waves hand their accumulators to the gate waves through LDS
-    // (free after the last chunk's barrier): [wm][i][j][r][lane]
-    float* xch = reinterpret_cast<float*>(As);
-    static_assert(2 * FM * FN * 16 * 64 * 4 <= BM * ROWB, "exchange fits the A tile");
-    if (wn == 1) {
+    for (int s = 0; s < KS; ++s) {
+      if (s + 1 < KS) fetch(s + 1, av[(s + 1) & 1], bv[(s + 1) & 1]);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_step<T>(bv[s & 1][j], av[s & 1][i], acc[i][j]);
+    }
+    rd = rd + 1 == STAGES ? 0 : rd + 1;
+    wr_stage = wr_stage + 1 == STAGES ? 0 : wr_stage + 1;
+  }
+
+  // (the steps past the last wrote zeros into the ring: let them land before
+  // this block's LDS is reused or given back)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // the wave groups' sums of a tile, added in group order: group g finishes
+  // the register quads q with q WK / 4 == g of every fragment and hands over
+  // the others
+  if constexpr (WK > 1) {
+    __syncthreads();  // (the ring is free: every wave's last reads and loads are done)
+    u32x4* xch = (u32x4*)lds;
+    const int wt = wave % (C::WM * WN);
+    auto slot = [&](int f, int g, int q) { return (((wt * 2 * FM + f) * (WK - 1) + g) * 4 + q) * 64 + lane; };
 #pragma unroll
-          for (int r = 0; r < 16; ++r) xch[(((wm * FM + i) * FN + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+    for (int q = 0; q < 4; ++q) {
+      const int owner = q * WK / 4;
+      if (owner == wk) continue;
+      const int g = wk < owner ? wk : wk - 1;
+#pragma unroll
+      for (int f = 0; f < 2 * FM; ++f) {
+        const f32x16& a = acc[f >> 1][f & 1];
+        xch[slot(f, g, q)] = u32x4{__float_as_uint(a[4 * q]), __float_as_uint(a[4 * q + 1]),
+                                   __float_as_uint(a[4 * q + 2]), __float_as_uint(a[4 * q + 3])};
+      }
     }
     __syncthreads();
-    if (wn == 1) return;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int q = 0; q < 4; ++q) {
+      if (q * WK / 4 != wk) continue;
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int64_t col = (int64_t)blockIdx.x * (BN / 2) + j * 32 + (lane & 31);
-        if (col >= N) continue;
+      for (int f = 0; f < 2 * FM; ++f) {
+        float v[4];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t row = m0 + wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-          if (row >= M) continue;
-          const float g = round_to<T>(acc[i][j][r] + 0.f);
-          const float u = round_to<T>(xch[(((wm * FM + i) * FN + j) * 16 + r) * 64 + lane] + 0.f);
-          store_f32<T>(y, row * ldy + col, swiglu<T>(g, u));
+        for (int g = 0; g < WK; ++g) {
+          float p[4];
+          if (g == wk) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p[e] = acc[f >> 1][f & 1][4 * q + e];
+          } else {
+            const u32x4 u = xch[slot(f, g < wk ? g : g - 1, q)];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p[e] = __uint_as_float(u[e]);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = g == 0 ? p[e] : v[e] + p[e];
         }
-      }
-    return;
-  }
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int64_t col = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
-      if (col >= N) continue;
-      const float bcol = (OUT == MINITP_EPI_NONE && bias != nullptr) ? load_f32<T>(bias, col) : 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t row = m0 + wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row >= M) continue;
-        const float v = acc[i][j][r];
-        if constexpr (OUT == OUT_PARTIAL)
-          part[((int64_t)blockIdx.z * M + row) * N + col] = v;
-        else if constexpr (OUT == MINITP_EPI_RESID)
-          store_f32<T>(y, row * ldy + col, add_rn(load_f32<T>(aux, row * ldy + col), round_to<T>(v)));
-        else
-          store_f32<T>(y, row * ldy + col, v + bcol);
+        for (int e = 0; e < 4; ++e) acc[f >> 1][f & 1][4 * q + e] = v[e];
       }
     }
+  }
+
+  // outputs of lane l, fragment (i, j), register 4 q + e: row i 32 + l % 32,
+  // column j 32 + 8 q + 4 (l / 32) + e. Whole quads go out as one store when
+  // rows and base allow it (else element by element).
+  using O = typename std::conditional<OUT == OUT_PARTIAL, float, T>::type;
+  O* const out = OUT == OUT_PARTIAL ? (O*)(part + (int64_t)z * M * N) : (O*)y;
+  const int64_t ldo = OUT == OUT_PARTIAL ? N : ldy;
+  const bool quads = N % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)out & (4 * sizeof(O) - 1)) == 0;
+  auto finish = [&](int i, int j, int q, int64_t row, int col, float* v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = acc[i][j][4 * q + e];
+      if constexpr (OUT == OUT_SWIGLU)
+        v[e] = swiglu<T>(round_to<T>(a + 0.f), round_to<T>(acc[i][1][4 * q + e] + 0.f));
+      else if constexpr (OUT == MINITP_EPI_RESID)
+        v[e] = col + e < N ? add_rn(load_f32<T>(aux, row * ldy + col + e), round_to<T>(a)) : 0.f;
+      else if constexpr (OUT == MINITP_EPI_NONE)
+        v[e] = a + (bias != nullptr && col + e < N ? load_f32<T>(bias, col + e) : 0.f);
+      else
+        v[e] = a;
+    }
+  };
+  constexpr int FJ = OUT == OUT_SWIGLU ? 1 : 2;
+  const int col0 = n0 + wn * (32 * FJ) + 4 * half;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (WK > 1 && q * WK / 4 != wk) continue;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int64_t row = m0 + wm * (32 * FM) + i * 32 + (lane & 31);
+      if (row >= M) continue;
+#pragma unroll
+      for (int j = 0; j < FJ; ++j) {
+        const int col = col0 + j * 32 + 8 * q;
+        float v[4];
+        if (col >= N) continue;
+        finish(i, j, q, row, col, v);
+        O* o = out + row * ldo + col;
+        if (quads) {
+          if constexpr (sizeof(O) == 4)
+            *(float4*)o = make_float4(v[0], v[1], v[2], v[3]);
+          else
+            *(uint2*)o = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        } else {
+#pragma unroll 1
+          for (int e = 0; e < 4 && col + e < N; ++e) store_f32<O>(o, e, e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3]);
+        }
+      }
+    }
+  }
 }
 
-// y = epilogue(sum over the S splits of part[s][M][N]), splits added in order.
-template <typename T, int EPI>
+// y = epilogue(sum over the S splits of part[s][M][N]), splits added in order;
+// PER (4 when N is a multiple of 4) consecutive elements of a row per thread.
+template <typename T, int EPI, int PER>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int S, const T* bias, T* y,
                                                           int64_t ldy, const T* aux, int64_t M, int64_t N,
                                                           const StepState* state) {
   if (state != nullptr) y = (T*)state->args.logits;
-  const int64_t MN = M * N;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < MN; e += (int64_t)gridDim.x * blockDim.x) {
-    float v = part[e];
-    for (int s = 1; s < S; ++s) v += part[s * MN + e];
-    const int64_t row = e / N, col = e % N;
-    if constexpr (EPI == MINITP_EPI_RESID)
-      store_f32<T>(y, row * ldy + col, add_rn(load_f32<T>(aux, row * ldy + col), round_to<T>(v)));
-    else
-      store_f32<T>(y, row * ldy + col, v + (bias != nullptr ? load_f32<T>(bias, col) : 0.f));
+  const int64_t MN = M * N, stride = (int64_t)gridDim.x * blockDim.x * PER;
+  for (int64_t e0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * PER; e0 < MN; e0 += stride) {
+    float v[PER];
+    for (int s = 0; s < S; ++s) {
+      float p[PER];
+      if constexpr (PER == 4) {
+        const float4 t = *(const float4*)(part + s * MN + e0);
+        p[0] = t.x;
+        p[1] = t.y;
+        p[2] = t.z;
+        p[3] = t.w;
+      } else {
+        p[0] = part[s * MN + e0];
+      }
+#pragma unroll
+      for (int u = 0; u < PER; ++u) v[u] = s == 0 ? p[u] : v[u] + p[u];
+    }
+    const int64_t row = e0 / N, col = e0 % N;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      if constexpr (EPI == MINITP_EPI_RESID)
+        store_f32<T>(y, row * ldy + col + u, add_rn(load_f32<T>(aux, row * ldy + col + u), round_to<T>(v[u])));
+      else
+        store_f32<T>(y, row * ldy + col + u, v[u] + (bias != nullptr ? load_f32<T>(bias, col + u) : 0.f));
+    }
   }
 }
 
-// blocks a split-K product aims at: the reduce-kernel form (fp32, direct
-// calls) fills the CUs twice; the form whose partials the next kernel adds
-// (bf16 prompt forwards) once: 128-token 0.5B TTFT 1.62 ms at 512 blocks,
-// 1.49 at 256 (128: 1.53, 192: 1.51, 384: 1.56; per-product mixes of 192-1024
-// no better), 512-token 7B 12.67 -> 12.16 ms
-#ifndef MINITP_SPLIT_BLOCKS
-#define MINITP_SPLIT_BLOCKS 512
-#endif
-#ifndef MINITP_PARTIALS_SPLIT_BLOCKS
-#define MINITP_PARTIALS_SPLIT_BLOCKS 256
-#endif
-// the same on 128 x 128 tiles (prompts of 512 rows and more): 7B 512-token
-// TTFT 11.13 ms at 384 blocks, 11.30 at 320, 11.43-11.46 at 192-256
-#ifndef MINITP_PARTIALS_SPLIT_BLOCKS_LARGE
-#define MINITP_PARTIALS_SPLIT_BLOCKS_LARGE 384
-#endif
-// Splits of K (and K elements per split) for an M x N x K product on BM x BN
-// tiles: enough blocks to fill the CUs twice, each at least one chunk deep,
-// and partials that fit the workspace.
-template <typename T, int BM, int BN>
-int64_t split_plan(int64_t M, int64_t N, int64_t K, const float* ws, int64_t ws_bytes, int64_t* kper_out,
-                   int64_t target = MINITP_SPLIT_BLOCKS) {
-  constexpr int64_t KCE = chunk_bytes<BM>() / sizeof(T);
-  const int64_t tiles = cdiv(N, BN) * cdiv(M, BM);
-  const int64_t nchunk = cdiv(K, KCE);
-  int64_t S = 1;
-  if (ws != nullptr) {
-    S = std::min<int64_t>(cdiv(target, tiles), nchunk);
-    while (S > 1 && S * M * N * (int64_t)sizeof(float) > ws_bytes) --S;
+// The tile shapes and what a launch on them costs: measured in a graph between
+// other kernels, cold weights, as FIXED_US + rounds x (stages x stage_us +
+// round_us), a round being one block per CU (blocks sharing a CU add up their
+// times within a few percent) and a stage 128 bytes of K.
+//   256 x 128, 16 waves, 144 KiB of LDS: 2000 x 3584 x 3584      53.7 us (957 TFLOP/s)
+//   128 x 128,  8 waves, 128 KiB: 433 x 3584 x 3584 in 2 splits  20.7 us
+//    64 x 128,  8 waves,  96 KiB: 433 x 4608 x 3584              27.8 us
+//    64 x  64,  4 waves,  64 KiB: 1099 x 896 x 4864              19.4 us
+//    32 x  64,  4 waves,  72 KiB: 8 x 37888 x 3584               46.7 us (5.8 TB/s)
+// against 77.8, 31.0, 32.6, 68.1 and 76.0 us for register-staged 64 x 64 and
+// 128 x 128 tiles without the ring. A product of one row tile reads every
+// weight once: non-temporal loads (8 x 37888 x 3584: 52.8 us without). Rings: 3 stages of 64 x 64 are 3-10 %
+// slower than 4 in bf16, 8 no faster. fp32 (bound by its MFMAs) always takes
+// 64 x 64 with 3 stages (32 x 64 up to 32 rows): the fastest or within 3 % at
+// every shape measured (999 x 9728 x 896: 153 us against 164-169 and 8 stages
+// 204; 30 x 151936 x 896: 114 us against 158 on 64 x 64).
+using TileXL = Tile<256, 128, 2, 3>;
+using TileL = Tile<128, 128, 2, 4>;
+using TileN = Tile<64, 128, 4, 4>;
+using TileS = Tile<64, 64, 4, 4>;
+using TileSnt = Tile<64, 64, 4, 4, true>;
+using TileXS = Tile<32, 64, 4, 6, true>;
+using TileS32 = Tile<64, 64, 4, 3>;
+using TileXS32 = Tile<32, 64, 4, 3, true>;
+
+struct TileCost {
+  int bm, bn;
+  float stage_us, round_us;
+};
+constexpr TileCost TILE_COST[] = {
+    {256, 128, 0.90f, 4.5f}, {128, 128, 0.60f, 3.f}, {64, 128, 0.42f, 2.f}, {64, 64, 0.25f, 0.5f}, {32, 64, 0.22f, 0.5f}};
+constexpr TileCost F32_COST[] = {{64, 64, 0.56f, 1.f}, {32, 64, 0.33f, 0.5f}};
+constexpr TileCost TILE256_COST = {256, 256, 1.33f, 5.f};
+enum { KIND_XL = 0, KIND_L = 1, KIND_N = 2, KIND_S = 3, KIND_XS = 4 };
+constexpr int64_t XS_ROWS = 32, S_NT_ROWS = 64;
+constexpr float FIXED_US = 3.3f, REDUCE_US = 3.f;
+constexpr float PARTIALS_PER_US = 1e6f;   // fp32 partials written and read back
+constexpr int64_t SPLIT_MIN_STAGES = 2;   // stages a split runs at least
+
+struct GemmPlan {
+  int kind;
+  int64_t S, kper;
+  float us;
+};
+
+// The cheapest tile shape and number of K splits of an M x N x K product by
+// the costs above. ws_bytes: room for the partials (0: no splits); split_us:
+// what a split adds (the reduction launch). swiglu: W has 2N rows.
+GemmPlan gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, bool swiglu, int64_t ws_bytes, float split_us) {
+  const bool f32 = dtype == MINITP_F32;
+  const int64_t tk = f32 ? 32 : 64, stages = cdiv(K, tk), cus = device_cus();
+  GemmPlan best{-1, 1, stages * tk, 0.f};
+  for (int kind = M <= XS_ROWS ? KIND_XS : f32 ? KIND_S : KIND_XL; kind <= (M <= XS_ROWS ? KIND_XS : KIND_S); ++kind) {
+    const TileCost& c = f32 ? F32_COST[kind - KIND_S] : TILE_COST[kind];
+    const int64_t tiles = cdiv(M, c.bm) * cdiv(swiglu ? 2 * N : N, c.bn);
+    for (int64_t s = 1; s <= 16; ++s) {
+      if (s > 1 && (s * M * N * 4 > ws_bytes || stages < s * SPLIT_MIN_STAGES || tiles * (s - 1) >= 2 * cus)) break;
+      const int64_t per = cdiv(stages, s);
+      if (cdiv(stages, per) != s) continue;
+      const float us = FIXED_US + (float)cdiv(tiles * s, cus) * ((float)per * c.stage_us + c.round_us) +
+                       (s > 1 ? split_us + (float)(s * M * N) / PARTIALS_PER_US : 0.f);
+      if (best.kind < 0 || us < best.us) best = GemmPlan{kind, s, per * tk, us};
+    }
   }
-  const int64_t kper = cdiv(nchunk, S) * KCE;
-  *kper_out = kper;
-  return cdiv(K, kper);
+  return best;
 }
 
+// Rows of x past 4 GiB from a tile's first row, or a [gate; up] weight past
+// it, are out of a buffer resource's reach.
 inline bool gemm_operands_fit(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t es) {
-  return N * K * es <= 0xffffffffLL && ((M - 1) * ldx + K) * es <= 0xffffffffLL;
+  return N * K * es <= 0xffffffffLL && ((M - 1) * ldx + K) * es <= 0xffffffffLL && M < (1LL << 31) &&
+         N < (1LL << 30) && K < (1LL << 26);
 }
 
-template <typename T, int BM, int BN>
-int gemm_launch(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
-                int64_t N, int64_t K, int epi, const T* aux, const StepState* state, float* ws, int64_t ws_bytes) {
-  if (!gemm_operands_fit(M, N, K, ldx, sizeof(T))) {
-    set_error("gemm: operands over 4 GiB (M=%lld N=%lld K=%lld)", (long long)M, (long long)N, (long long)K);
-    return MINITP_ERR_UNSUPPORTED;
-  }
-  int64_t kper = 0;
-  const int64_t S = split_plan<T, BM, BN>(M, N, K, ws, ws_bytes, &kper);
-  const dim3 grid((unsigned)cdiv(N, BN), (unsigned)cdiv(M, BM), (unsigned)S);
-  if (S > 1) {
-    hipLaunchKernelGGL((gemm_kernel<T, BM, BN, OUT_PARTIAL>), grid, dim3(256), 0, st, x, ldx, w, bias, y, ldy, aux,
-                       ws, M, N, K, kper, state);
-    MINITP_LAUNCH_CHECK();
-    const int rgrid = (int)std::min<int64_t>(cdiv(M * N, 256), 2048);
-    if (epi == MINITP_EPI_RESID)
-      hipLaunchKernelGGL((gemm_reduce_kernel<T, MINITP_EPI_RESID>), dim3(rgrid), dim3(256), 0, st, ws, (int)S, bias,
-                         y, ldy, aux, M, N, state);
-    else
-      hipLaunchKernelGGL((gemm_reduce_kernel<T, MINITP_EPI_NONE>), dim3(rgrid), dim3(256), 0, st, ws, (int)S, bias, y,
-                         ldy, aux, M, N, state);
-  } else if (epi == MINITP_EPI_RESID) {
-    hipLaunchKernelGGL((gemm_kernel<T, BM, BN, MINITP_EPI_RESID>), grid, dim3(256), 0, st, x, ldx, w, bias, y, ldy,
-                       aux, ws, M, N, K, kper, state);
+template <typename T, typename C, int OUT>
+int launch_cfg(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
+               int64_t N, int64_t K, const T* aux, const StepState* state, float* part, const GemmPlan& p) {
+  if (const int rc = ensure_lds_limit((const void*)gemm_kernel<T, C, OUT>, C::LDS_BYTES)) return rc;
+  const int tiles_m = (int)cdiv(M, C::BM), tiles_n = (int)cdiv(OUT == OUT_SWIGLU ? 2 * N : N, C::BN);
+  const int64_t items = (int64_t)tiles_m * tiles_n * p.S;
+  const dim3 grid((unsigned)(8 * cdiv(items, 8)));
+  hipLaunchKernelGGL((gemm_kernel<T, C, OUT>), grid, dim3(C::THREADS), C::LDS_BYTES, st, x, ldx, w, bias, y, ldy, aux,
+                     part, (int)M, (int)N, (int)K, (int)p.kper, tiles_m, tiles_n, (int)items, state);
+  MINITP_LAUNCH_CHECK();
+  return MINITP_OK;
+}
+
+template <typename T, int OUT>
+int launch_plan(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
+                int64_t N, int64_t K, const T* aux, const StepState* state, float* part, const GemmPlan& p) {
+  auto go = [&](auto cfg) {
+    return launch_cfg<T, decltype(cfg), OUT>(st, x, ldx, w, bias, y, ldy, M, N, K, aux, state, part, p);
+  };
+  if constexpr (sizeof(T) == 2) {
+    if (p.kind == KIND_XL) return go(TileXL{});
+    if (p.kind == KIND_L) return go(TileL{});
+    if (p.kind == KIND_N) return go(TileN{});
+    if (p.kind == KIND_XS) return go(TileXS{});
+    return M <= S_NT_ROWS ? go(TileSnt{}) : go(TileS{});
   } else {
-    hipLaunchKernelGGL((gemm_kernel<T, BM, BN, MINITP_EPI_NONE>), grid, dim3(256), 0, st, x, ldx, w, bias, y, ldy,
-                       aux, ws, M, N, K, kper, state);
+    return p.kind == KIND_XS ? go(TileXS32{}) : go(TileS32{});
+  }
+}
+
+template <typename T, int EPI>
+int launch_reduce(hipStream_t st, const float* ws, int64_t S, const T* bias, T* y, int64_t ldy, const T* aux,
+                  int64_t M, int64_t N, const StepState* state) {
+  if (N % 4 == 0 && aligned16(ws)) {
+    const int grid = (int)std::min<int64_t>(cdiv(M * N / 4, 256), 2048);
+    hipLaunchKernelGGL((gemm_reduce_kernel<T, EPI, 4>), dim3(grid), dim3(256), 0, st, ws, (int)S, bias, y, ldy, aux, M,
+                       N, state);
+  } else {
+    const int grid = (int)std::min<int64_t>(cdiv(M * N, 256), 2048);
+    hipLaunchKernelGGL((gemm_reduce_kernel<T, EPI, 1>), dim3(grid), dim3(256), 0, st, ws, (int)S, bias, y, ldy, aux, M,
+                       N, state);
   }
   MINITP_LAUNCH_CHECK();
   return MINITP_OK;
 }
 
 template <typename T>
-int gemm_typed(hipStream_t st, const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy,
-               int64_t M, int64_t N, int64_t K, int epi, const void* aux, const StepState* state, void* ws,
-               int64_t ws_bytes) {
-  // large M: 128 x 128 tiles already fill the chip; small M: 64 x 64 tiles and split K
-  if (M >= 512)
-    return gemm_launch<T, 128, 128>(st, (const T*)x, ldx, (const T*)w, (const T*)bias, (T*)y, ldy, M, N, K, epi,
-                                    (const T*)aux, state, (float*)ws, ws_bytes);
-  return gemm_launch<T, MINITP_GEMM_SMALL_BM, MINITP_GEMM_SMALL_BN>(st, (const T*)x, ldx, (const T*)w,
-                                                                    (const T*)bias, (T*)y, ldy, M, N, K, epi,
-                                                                    (const T*)aux, state, (float*)ws, ws_bytes);
+int gemm_typed(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
+               int64_t N, int64_t K, int epi, const T* aux, const StepState* state, float* ws, int64_t ws_bytes) {
+  if (!gemm_operands_fit(M, N, K, ldx, sizeof(T))) {
+    set_error("gemm: operands over 4 GiB (M=%lld N=%lld K=%lld)", (long long)M, (long long)N, (long long)K);
+    return MINITP_ERR_UNSUPPORTED;
+  }
+  const GemmPlan p = gemm_plan(sizeof(T) == 4 ? MINITP_F32 : MINITP_BF16, M, N, K, false, ws ? ws_bytes : 0, REDUCE_US);
+  const bool resid = epi == MINITP_EPI_RESID;
+  if (p.S > 1) {
+    const int rc = launch_plan<T, OUT_PARTIAL>(st, x, ldx, w, bias, y, ldy, M, N, K, aux, state, ws, p);
+    if (rc) return rc;
+    return resid ? launch_reduce<T, MINITP_EPI_RESID>(st, ws, p.S, bias, y, ldy, aux, M, N, state)
+                 : launch_reduce<T, MINITP_EPI_NONE>(st, ws, p.S, bias, y, ldy, aux, M, N, state);
+  }
+  return resid ? launch_plan<T, MINITP_EPI_RESID>(st, x, ldx, w, bias, y, ldy, M, N, K, aux, state, ws, p)
+               : launch_plan<T, MINITP_EPI_NONE>(st, x, ldx, w, bias, y, ldy, M, N, K, aux, state, ws, p);
 }
 
 }  // namespace
 
+bool gemm_prefers_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu, int64_t ws_bytes,
+                       float split_us) {
+  if (!gemm_tile_supported(M, N, K, ldx, ldy, swiglu)) return false;
+  const int64_t tiles = cdiv(M, 256) * cdiv(swiglu ? 2 * N : N, 256), cus = device_cus(), rem = tiles % cus;
+  // (a last round at most half full is split over K when the caller brings the workspace)
+  const float rounds = (float)(tiles / cus) + (rem == 0 ? 0.f : tiles > cus && 2 * rem <= cus && ws_bytes ? 0.6f : 1.f);
+  const float us = FIXED_US + rounds * ((float)cdiv(K, 64) * TILE256_COST.stage_us + TILE256_COST.round_us);
+  return us <= gemm_plan(MINITP_BF16, M, N, K, swiglu, swiglu ? 0 : ws_bytes, split_us).us;
+}
+
 int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
-                       int64_t M, int64_t N, int64_t K) {
+                       int64_t M, int64_t N, int64_t K, TileTail tail) {
   if (M == 0 || N == 0) return MINITP_OK;
-  if (dtype != MINITP_BF16 || M >= 512 || ldy < N || !aligned16(x) || !aligned16(w) ||
-      !gemm_operands_fit(M, 2 * N, K, ldx, 2)) {
+  const int64_t es = dtype == MINITP_F32 ? 4 : 2;
+  if (dtype == MINITP_BF16 && aligned16(x) && aligned16(w) &&
+      gemm_prefers_tile(M, N, K, ldx, ldy, true, tail.part != nullptr ? TILE_TAIL_BYTES : 0, 0.f))
+    return launch_gemm_tile(st, x, ldx, w, nullptr, y, ldy, M, N, K, true, tail);
+  if (ldy < N || K * es % 16 != 0 || !aligned16(x) || !aligned16(w) || 2 * N * K * es >= (int64_t)ROW_OOB ||
+      !gemm_operands_fit(M, 2 * N, K, ldx, es)) {
     set_error("gemm: SwiGLU form M=%lld N=%lld K=%lld not served", (long long)M, (long long)N, (long long)K);
     return MINITP_ERR_UNSUPPORTED;
   }
-  constexpr int BM = MINITP_GEMM_SMALL_BM, BN = MINITP_GEMM_SMALL_BN;
-  const dim3 grid((unsigned)cdiv(N, BN / 2), (unsigned)cdiv(M, BM), 1u);
-  hipLaunchKernelGGL((gemm_kernel<bf16, BM, BN, OUT_SWIGLU>), grid, dim3(256), 0, st, (const bf16*)x, ldx,
-                     (const bf16*)w, nullptr, (bf16*)y, ldy, nullptr, nullptr, M, N, K, K, nullptr);
-  MINITP_LAUNCH_CHECK();
-  return MINITP_OK;
+  const GemmPlan p = gemm_plan(dtype, M, N, K, true, 0, 0.f);
+  return dtype == MINITP_F32
+             ? launch_plan<float, OUT_SWIGLU>(st, (const float*)x, ldx, (const float*)w, nullptr, (float*)y, ldy, M, N,
+                                              K, nullptr, nullptr, nullptr, p)
+             : launch_plan<bf16, OUT_SWIGLU>(st, (const bf16*)x, ldx, (const bf16*)w, nullptr, (bf16*)y, ldy, M, N, K,
+                                             nullptr, nullptr, nullptr, p);
 }
 
 int launch_gemm_partials(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, int64_t M, int64_t N,
-                         int64_t K, void* ws, int64_t ws_bytes, Partials* out, int64_t target_blocks) {
-  if (target_blocks <= 0) target_blocks = M >= 512 ? MINITP_PARTIALS_SPLIT_BLOCKS_LARGE : MINITP_PARTIALS_SPLIT_BLOCKS;
-  // the product launch_gemm would split (bf16, not on the tile kernel)
-  if (dtype != MINITP_BF16 || M <= 0 || N % 8 != 0 || ws == nullptr || !aligned16(ws) || !aligned16(x) ||
-      !aligned16(w) || gemm_tile_supported(M, N, K, ldx, N, false) || !gemm_operands_fit(M, N, K, ldx, 2))
+                         int64_t K, void* ws, int64_t ws_bytes, Partials* out) {
+  const int64_t es = dtype == MINITP_F32 ? 4 : 2;
+  if (M <= 0 || N % 8 != 0 || ws == nullptr || !aligned16(ws) || !aligned16(x) || !aligned16(w) ||
+      !gemm_operands_fit(M, N, K, ldx, es) ||
+      (dtype == MINITP_BF16 && gemm_prefers_tile(M, N, K, ldx, N, false, ws_bytes, 0.f)))
     return MINITP_ERR_UNSUPPORTED;
-  int64_t kper = 0, S;
-  dim3 grid;
-  const bf16 *xb = (const bf16*)x, *wb = (const bf16*)w;
-  float* part = (float*)ws;
-  if (M >= 512) {
-    S = split_plan<bf16, 128, 128>(M, N, K, part, ws_bytes, &kper, target_blocks);
-    if (S < 2) return MINITP_ERR_UNSUPPORTED;
-    grid = dim3((unsigned)cdiv(N, 128), (unsigned)cdiv(M, 128), (unsigned)S);
-    hipLaunchKernelGGL((gemm_kernel<bf16, 128, 128, OUT_PARTIAL>), grid, dim3(256), 0, st, xb, ldx, wb, nullptr,
-                       nullptr, N, nullptr, part, M, N, K, kper, nullptr);
-  } else {
-    constexpr int BM = MINITP_GEMM_SMALL_BM, BN = MINITP_GEMM_SMALL_BN;
-    S = split_plan<bf16, BM, BN>(M, N, K, part, ws_bytes, &kper, target_blocks);
-    if (S < 2) return MINITP_ERR_UNSUPPORTED;
-    grid = dim3((unsigned)cdiv(N, BN), (unsigned)cdiv(M, BM), (unsigned)S);
-    hipLaunchKernelGGL((gemm_kernel<bf16, BM, BN, OUT_PARTIAL>), grid, dim3(256), 0, st, xb, ldx, wb, nullptr, nullptr,
-                       N, nullptr, part, M, N, K, kper, nullptr);
-  }
-  MINITP_LAUNCH_CHECK();
-  *out = Partials{part, (int)S, M, N};
+  const GemmPlan p = gemm_plan(dtype, M, N, K, false, ws_bytes, 0.f);
+  if (p.S < 2) return MINITP_ERR_UNSUPPORTED;
+  const int rc =
+      dtype == MINITP_F32
+          ? launch_plan<float, OUT_PARTIAL>(st, (const float*)x, ldx, (const float*)w, nullptr, nullptr, N, M, N, K,
+                                            nullptr, nullptr, (float*)ws, p)
+          : launch_plan<bf16, OUT_PARTIAL>(st, (const bf16*)x, ldx, (const bf16*)w, nullptr, nullptr, N, M, N, K,
+                                           nullptr, nullptr, (float*)ws, p);
+  if (rc) return rc;
+  *out = Partials{(const float*)ws, (int)p.S, M, N};
   return MINITP_OK;
 }
 
@@ -418,10 +573,13 @@ int launch_gemm(hipStream_t st, int dtype, const void* x, int64_t ldx, const voi
   }
   // bf16 products large enough to fill the chip with 256 x 256 tiles
   if (dtype == MINITP_BF16 && epi == MINITP_EPI_NONE && state == nullptr && aligned16(x) && aligned16(w) &&
-      gemm_tile_supported(M, N, K, ldx, ldy, false))
+      gemm_prefers_tile(M, N, K, ldx, ldy, false, ws != nullptr ? ws_bytes : 0, REDUCE_US))
     return launch_gemm_tile(st, x, ldx, w, bias, y, ldy, M, N, K, false, tail);
-  return dtype == MINITP_F32 ? gemm_typed<float>(st, x, ldx, w, bias, y, ldy, M, N, K, epi, aux, state, ws, ws_bytes)
-                             : gemm_typed<bf16>(st, x, ldx, w, bias, y, ldy, M, N, K, epi, aux, state, ws, ws_bytes);
+  return dtype == MINITP_F32
+             ? gemm_typed<float>(st, (const float*)x, ldx, (const float*)w, (const float*)bias, (float*)y, ldy, M, N,
+                                 K, epi, (const float*)aux, state, (float*)ws, ws_bytes)
+             : gemm_typed<bf16>(st, (const bf16*)x, ldx, (const bf16*)w, (const bf16*)bias, (bf16*)y, ldy, M, N, K,
+                                epi, (const bf16*)aux, state, (float*)ws, ws_bytes);
 }
 
 }  // namespace minitp

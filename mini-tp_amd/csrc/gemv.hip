@@ -27,8 +27,6 @@
 
 namespace minitp {
 
-static int device_cus();
-
 namespace {
 
 constexpr int P = 2;  // pairs per tuple (R = 4 rows)
@@ -2158,7 +2156,7 @@ bool gemv_part_supported(int dtype, int64_t K, int nparts) {
 }
 
 // Compute units of the current device (cached per device).
-static int device_cus() {
+int device_cus() {
   static std::mutex mu;
   static int cus[64] = {0};
   int dev = 0;

@@ -98,6 +98,8 @@ struct GemvArgs {
   int max_grid;  // register form: cap on the grid (0: the default)
 };
 
+int device_cus();  // compute units of the current device (gemv.hip)
+
 // gemv.hip
 // The partial-sum prologue's limits: at most PART_MAX_PARTS partial rows of
 // K <= PART_MAX_K elements (one row).
@@ -144,18 +146,24 @@ int launch_gemm(hipStream_t st, int dtype, const void* x, int64_t ldx, const voi
                 int64_t ldy, int64_t M, int64_t N, int64_t K, int epi, const void* aux,
                 const StepState* state = nullptr, void* ws = nullptr, int64_t ws_bytes = 0,
                 TileTail tail = TileTail{nullptr, nullptr});
-// The first half of a bf16 product that launch_gemm would split over K: the
+// The first half of a product that launch_gemm would split over K: the
 // split GEMM alone, its fp32 partials [S][M][N] in ws (described in *out),
 // for a consumer kernel to add up in split order with its own epilogue
 // (the *_partials launchers). MINITP_ERR_UNSUPPORTED when the product is
-// not split (tile kernel, one split, fp32): the caller runs launch_gemm.
+// not split (tile kernel, one split): the caller runs launch_gemm.
 int launch_gemm_partials(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, int64_t M, int64_t N,
-                         int64_t K, void* ws, int64_t ws_bytes, Partials* out, int64_t target_blocks = 0);
-// bf16 y[M, N] = swiglu(x W_gate^T, x W_up^T) for W = [gate; up] ([2N, K]) on
-// the small tiles, unsplit (M < 512), gate and up rounded to bf16 first as
-// launch_gemm + launch_silu_mul would store and read them
-int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
-                       int64_t M, int64_t N, int64_t K);
+                         int64_t K, void* ws, int64_t ws_bytes, Partials* out);
+// y[M, N] = swiglu(x W_gate^T, x W_up^T) for W = [gate; up] ([2N, K]), gate
+// and up rounded to the dtype first as launch_gemm + launch_silu_mul would
+// store and read them
+int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int64_t M,
+                       int64_t N, int64_t K, TileTail tail = TileTail{nullptr, nullptr});
+// Whether launch_gemm, launch_gemm_swiglu and launch_gemm_partials run a bf16
+// product on the 256 x 256 tiles (the faster choice by the measured stage
+// costs); ws_bytes: room for split partials (0: none), split_us: what a split
+// adds on top of them.
+bool gemm_prefers_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu, int64_t ws_bytes,
+                       float split_us);
 
 // gemm_tile.hip: 256 x 256 MFMA tiles (32x32x16 bf16) for prompt-sized
 // bf16 products; swiglu: W is [2N, K] = [gate; up] and y = silu(gate) * up
@@ -164,13 +172,6 @@ int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, co
 bool gemm_tile_supported(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu);
 int launch_gemm_tile(hipStream_t st, const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy,
                      int64_t M, int64_t N, int64_t K, bool swiglu, TileTail tail = TileTail{nullptr, nullptr});
-// The same tiles for products with too few of them (M a multiple of 256,
-// fewer tiles than half the CUs) and a long K: every tile split over K into
-// parts that its last block adds (needs the forward's tail buffers)
-bool gemm_tile_split_supported(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu);
-int launch_gemm_tile_split(hipStream_t st, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
-                           int64_t ldy, int64_t M, int64_t N, int64_t K, bool swiglu, TileTail tail);
-
 // elementwise.hip
 int launch_fill_normal(hipStream_t st, int dtype, void* dst, int64_t count, uint64_t seed, uint64_t sid,
                        double std_dev);
@@ -186,12 +187,11 @@ int launch_silu_mul(hipStream_t st, int dtype, const void* gate, const void* up,
 int launch_cast_f32_bf16(hipStream_t st, const float* in, void* out, int64_t n);
 int launch_add_rmsnorm(hipStream_t st, int dtype, void* x, const void* delta, const void* w, void* out, int64_t rows,
                        int64_t hidden, float eps);
-// bf16 launch_add_rmsnorm / launch_silu_mul whose delta / [gate, up] input is
-// a split product's partials (the sums rounded to bf16 as launch_gemm
-// stores them, so the results are the same bits)
-int launch_add_rmsnorm_partials(hipStream_t st, void* x, const Partials& delta, const void* w, void* out,
+// launch_add_rmsnorm whose delta input is a split product's partials (the
+// sums rounded to the dtype as launch_gemm stores them, so the results are
+// the same bits)
+int launch_add_rmsnorm_partials(hipStream_t st, int dtype, void* x, const Partials& delta, const void* w, void* out,
                                 int64_t hidden, float eps);
-int launch_silu_mul_partials(hipStream_t st, const Partials& gu, void* out, int64_t ld_out, int64_t n);
 
 // rope.hip
 int launch_rope(hipStream_t st, int dtype, const void* q, const void* k, void* q_out, void* k_out, const float* cos_tab,
@@ -204,9 +204,9 @@ int launch_rope_kv_write(hipStream_t st, int dtype, const void* qkv, int64_t ld_
                          int64_t max_pos, int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t S,
                          int64_t cache_len, int32_t* error_flag, const StepState* state = nullptr,
                          int layer = 0);
-// bf16 launch_rope_kv_write of a QKV projection given as its split partials
-// plus the bias (positions, cache length and caches from the step state)
-int launch_rope_kv_write_partials(hipStream_t st, const Partials& qkv, const void* bias, void* q_out,
+// launch_rope_kv_write of a QKV projection given as its split partials plus
+// the bias (positions, cache length and caches from the step state)
+int launch_rope_kv_write_partials(hipStream_t st, int dtype, const Partials& qkv, const void* bias, void* q_out,
                                   const float* cos_tab, const float* sin_tab, int64_t max_pos, int64_t B, int64_t T,
                                   int64_t Hq, int64_t Hkv, int64_t D, int64_t S, const StepState* state, int layer);
 

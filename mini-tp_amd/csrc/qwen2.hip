@@ -8,11 +8,14 @@
 // therefore never needs re-capture: each replay patches only the first
 // node's by-value argument.
 //
-// Rows M = B * T <= 4 take the fused GEMV path, 5 kernels per layer:
+// Rows M = B * T that the GEMV forms serve take the fused path, 5 kernels per
+// layer:
 //   [RMSNorm -> QKV + bias -> RoPE -> q, KV write] [attention]
 //   [o_proj + residual] [RMSNorm -> gate/up -> SwiGLU] [down + residual]
-// and the final RMSNorm -> LM head -> argmax is one more kernel. Larger M
-// runs MFMA GEMMs with separate norm / RoPE / SwiGLU kernels.
+// and the final RMSNorm -> LM head -> argmax is one more kernel. Other rows
+// run MFMA GEMMs, 7 kernels per layer: the split products' partials are added
+// by the kernel that consumes them (RoPE + KV write, residual add + RMSNorm),
+// SwiGLU runs in the gate/up product's epilogue.
 #include <cmath>
 #include <cstddef>
 #include <mutex>
@@ -21,13 +24,6 @@
 
 #include "common.h"
 #include "kernels.h"
-
-#ifndef MINITP_DOWN_TILE_SPLIT
-#define MINITP_DOWN_TILE_SPLIT 1
-#endif
-#ifndef MINITP_GEMM_SWIGLU_EPI
-#define MINITP_GEMM_SWIGLU_EPI 1
-#endif
 
 namespace minitp {
 
@@ -204,12 +200,17 @@ struct Qwen2Program {
   // reads the per-call values from the step state: all of them with the last
   // position's logits; with every position's logits, those whose LM head runs
   // launch_gemm (logits pointer from the state), not the GEMV form (few rows)
-  // or the tile kernel (M >= 256), which store to the pointer they are given.
+  // or the tile kernel (many), which store to the pointer they are given.
   bool prompt_graphable(const minitp_qwen2_step& s) const {
     if (!prefill_graphs || s.tokens <= 1 || c.dtype != MINITP_BF16) return false;
     if (!s.logits_all) return true;
     const int64_t M = s.batch * s.tokens;
-    return !fused(M) && !gemm_tile_supported(M, c.vocab, c.hidden, c.hidden, c.vocab, false);
+    return !fused(M) && !head_on_tile(M);
+  }
+
+  // the LM head of M prompt rows (every position's logits) on the tile kernel
+  bool head_on_tile(int64_t M) const {
+    return c.dtype == MINITP_BF16 && gemm_prefers_tile(M, c.vocab, c.hidden, c.hidden, c.vocab, false, 0, 0.f);
   }
 
   bool fused(int64_t M) const {
@@ -246,13 +247,14 @@ struct Qwen2Program {
     const bool fo = fz && T == 1 && fuse_oproj && attn_oproj_supported(c.dtype, as, H, OPROJ_SLICES) &&
                     gemv_part_supported(c.dtype, H, c.heads);
     const int64_t layer_elems = B * c.kv_heads * s.max_seq * D;
-    // bf16 prompts: plain GEMMs (the 256 x 256 MFMA tile kernel where the
-    // shape fills the chip, else the split-K one), gate/up with SwiGLU in
-    // the tile kernel's epilogue. The residual adds go with the next RMSNorm
-    // (one fused kernel, the reference's rounding order), the projections
-    // that feed them writing into the normed-input buffer h, free at that
-    // point.
-    const bool blas = c.dtype == MINITP_BF16 && !fz && T > 1;
+    // Rows past the GEMV forms: plain GEMMs (the 256 x 256 MFMA tile kernel
+    // or the smaller tiles, by the measured costs), gate/up with SwiGLU in the
+    // epilogue. The residual adds go with the next RMSNorm (one fused kernel,
+    // the reference's rounding order), the projections that feed them writing
+    // into the normed-input buffer h, free at that point. (33-48 decode rows
+    // of the 0.5B shape: 11 kernels a layer with separate reductions, norms
+    // and SwiGLU before, 7 now.)
+    const bool gemm = !fz;
     // the tile GEMM's split last round: partials after the split-K region,
     // arrival words in the step state (zeroed by the embedding kernel)
     const TileTail tail{(float*)((char*)w.gemm_ws + GEMM_SPLIT_BYTES), w.split_count};
@@ -261,14 +263,13 @@ struct Qwen2Program {
       return launch_gemm(st, c.dtype, xin, ldx, wt, b, y, ldy, M, n, k, MINITP_EPI_NONE, nullptr, nullptr, w.gemm_ws,
                          GEMM_SPLIT_BYTES, tail);
     };
-    if (blas && (rc = launch_rmsnorm(st, c.dtype, w.x, L(0, MINITP_W_LN1), w.h, M, H, c.eps))) return rc;
-    // Prompt products that the split-K GEMM serves hand their partials to
-    // the kernel after them (RoPE + KV write, residual add + RMSNorm,
-    // SwiGLU), which adds them up in split order: no reduction launch, and
-    // the same bits as reduce-then-consume. The partials may take the whole
+    if (gemm && (rc = launch_rmsnorm(st, c.dtype, w.x, L(0, MINITP_W_LN1), w.h, M, H, c.eps))) return rc;
+    // Products that the split-K GEMM serves hand their partials to the kernel
+    // after them (RoPE + KV write, residual add + RMSNorm), which adds them up
+    // in split order: no reduction launch, and the same bits as
+    // reduce-then-consume. The partials may take the whole
     // GEMM workspace (nothing else in it is live between the two launches).
-    const bool fuse_split = blas && D % 16 == 0 && H % 8 == 0 && I % 8 == 0 &&
-                            aligned16(cos_tab) && aligned16(sin_tab);
+    const bool fuse_split = gemm && D % 16 == 0 && H % 8 == 0 && aligned16(cos_tab) && aligned16(sin_tab);
     auto partials = [&](const void* xin, int64_t ldx, const void* wt, int64_t n, int64_t k, Partials* p) -> int {
       if (!fuse_split) return MINITP_ERR_UNSUPPORTED;
       return launch_gemm_partials(st, c.dtype, xin, ldx, wt, M, n, k, w.gemm_ws, GEMM_WS_BYTES, p);
@@ -279,13 +280,13 @@ struct Qwen2Program {
       g.split_count = w.split_count;
     };
     for (int l = 0; l < c.num_layers; ++l) {
-      if (blas) {
+      if (gemm) {
         // h holds input_layernorm(x) of this layer
         Partials pp{};
         rc = partials(w.h, H, L(l, MINITP_W_QKV), qkv_rows(), H, &pp);
         if (rc == MINITP_OK) {
-          rc = launch_rope_kv_write_partials(st, pp, L(l, MINITP_W_QKV_BIAS), w.q, cos_tab, sin_tab, c.max_pos, B, T,
-                                             c.heads, c.kv_heads, D, s.max_seq, w.st, l);
+          rc = launch_rope_kv_write_partials(st, c.dtype, pp, L(l, MINITP_W_QKV_BIAS), w.q, cos_tab, sin_tab, c.max_pos,
+                                             B, T, c.heads, c.kv_heads, D, s.max_seq, w.st, l);
         } else if (rc == MINITP_ERR_UNSUPPORTED) {
           rc = lin(w.h, H, L(l, MINITP_W_QKV), L(l, MINITP_W_QKV_BIAS), w.qkv, qkv_rows(), qkv_rows(), H);
           if (!rc)
@@ -295,47 +296,31 @@ struct Qwen2Program {
         if (rc) return rc;
         const char* kc = (const char*)s.k_cache + l * layer_elems * es();
         const char* vc = (const char*)s.v_cache + l * layer_elems * es();
-        if ((rc = launch_prefill_attention(st, c.dtype, w.q, kc, vc, w.attn, as, s.cache_len, w.st, l))) return rc;
+        rc = T == 1 ? launch_decode_attention(st, c.dtype, w.q, nullptr, nullptr, w.attn, as, s.cache_len, w.st, l,
+                                              w.attn_ws, w.attn_ws_bytes)
+                    : launch_prefill_attention(st, c.dtype, w.q, kc, vc, w.attn, as, s.cache_len, w.st, l);
+        if (rc) return rc;
         // x += o_proj(attn), h = post_attention_layernorm(x)
         rc = partials(w.attn, q_rows(), L(l, MINITP_W_O), H, q_rows(), &pp);
         if (rc == MINITP_OK) {
-          rc = launch_add_rmsnorm_partials(st, w.x, pp, L(l, MINITP_W_LN2), w.h, H, c.eps);
+          rc = launch_add_rmsnorm_partials(st, c.dtype, w.x, pp, L(l, MINITP_W_LN2), w.h, H, c.eps);
         } else if (rc == MINITP_ERR_UNSUPPORTED) {
           rc = lin(w.attn, q_rows(), L(l, MINITP_W_O), nullptr, w.h, H, H, q_rows());
           if (!rc) rc = launch_add_rmsnorm(st, c.dtype, w.x, w.h, L(l, MINITP_W_LN2), w.h, M, H, c.eps);
         }
         if (rc) return rc;
-        if (gemm_tile_supported(M, I, H, H, I, true)) {
-          if ((rc = launch_gemm_tile(st, w.h, H, L(l, MINITP_W_GATE_UP), nullptr, w.act, I, M, I, H, true, tail)))
-            return rc;
-        } else {
-          rc = partials(w.h, H, L(l, MINITP_W_GATE_UP), 2 * I, H, &pp);
-          if (rc == MINITP_OK) {
-            rc = launch_silu_mul_partials(st, pp, w.act, I, I);
-          } else if (rc == MINITP_ERR_UNSUPPORTED && MINITP_GEMM_SWIGLU_EPI) {
-            // unsplit: SwiGLU in the GEMM's epilogue
-            rc = launch_gemm_swiglu(st, c.dtype, w.h, H, L(l, MINITP_W_GATE_UP), w.act, I, M, I, H);
-          }
-          if (rc == MINITP_ERR_UNSUPPORTED) {
-            rc = lin(w.h, H, L(l, MINITP_W_GATE_UP), nullptr, w.gu, 2 * I, 2 * I, H);
-            const char* up = (const char*)w.gu + I * es();
-            if (!rc) rc = launch_silu_mul(st, c.dtype, w.gu, up, 2 * I, w.act, I, M, I);
-          }
-          if (rc) return rc;
+        rc = launch_gemm_swiglu(st, c.dtype, w.h, H, L(l, MINITP_W_GATE_UP), w.act, I, M, I, H, tail);
+        if (rc == MINITP_ERR_UNSUPPORTED) {
+          rc = lin(w.h, H, L(l, MINITP_W_GATE_UP), nullptr, w.gu, 2 * I, 2 * I, H);
+          const char* up = (const char*)w.gu + I * es();
+          if (!rc) rc = launch_silu_mul(st, c.dtype, w.gu, up, 2 * I, w.act, I, M, I);
         }
+        if (rc) return rc;
         // x += down(act), h = the next layer's input_layernorm(x) (the final norm after the last)
         const void* next_norm = l + 1 < c.num_layers ? L(l + 1, MINITP_W_LN1) : final_norm;
-        // (a long K over too few tiles, e.g. 7B at 512 tokens: the tile kernel
-        // with every tile split over K, then the residual add + norm)
-        if (MINITP_DOWN_TILE_SPLIT && gemm_tile_split_supported(M, H, I, I, H, false)) {
-          rc = launch_gemm_tile_split(st, w.act, I, L(l, MINITP_W_DOWN), nullptr, w.h, H, M, H, I, false, tail);
-          if (!rc) rc = launch_add_rmsnorm(st, c.dtype, w.x, w.h, next_norm, w.h, M, H, c.eps);
-          if (rc) return rc;
-          continue;
-        }
         rc = partials(w.act, I, L(l, MINITP_W_DOWN), H, I, &pp);
         if (rc == MINITP_OK) {
-          rc = launch_add_rmsnorm_partials(st, w.x, pp, next_norm, w.h, H, c.eps);
+          rc = launch_add_rmsnorm_partials(st, c.dtype, w.x, pp, next_norm, w.h, H, c.eps);
         } else if (rc == MINITP_ERR_UNSUPPORTED) {
           rc = lin(w.act, I, L(l, MINITP_W_DOWN), nullptr, w.h, H, H, I);
           if (!rc) rc = launch_add_rmsnorm(st, c.dtype, w.x, w.h, next_norm, w.h, M, H, c.eps);
@@ -344,35 +329,25 @@ struct Qwen2Program {
         continue;
       }
       // ---- attention block --------------------------------------------------
-      if (fz) {
-        GemvArgs g{};
-        g.x = w.x;
-        g.ldx = H;
-        g.norm_w = L(l, MINITP_W_LN1);
-        g.eps = c.eps;
-        g.w = L(l, MINITP_W_QKV);
-        g.bias = L(l, MINITP_W_QKV_BIAS);
-        g.y = w.q;
-        g.ldy = q_rows();
-        g.M = M;
-        g.N = qkv_rows();
-        g.K = H;
-        g.st = w.st;
-        g.cos_tab = cos_tab;
-        g.sin_tab = sin_tab;
-        g.max_pos = c.max_pos;
-        g.layer = l;
-        g.a = as;
-        if ((rc = launch_gemv(st, c.dtype, PRO_NORM, EPI_QKV_ROPE, g))) return rc;
-      } else {
-        if ((rc = launch_rmsnorm(st, c.dtype, w.x, L(l, MINITP_W_LN1), w.h, M, H, c.eps))) return rc;
-        if ((rc = launch_gemm(st, c.dtype, w.h, H, L(l, MINITP_W_QKV), L(l, MINITP_W_QKV_BIAS), w.qkv, qkv_rows(), M,
-                              qkv_rows(), H, MINITP_EPI_NONE, nullptr, nullptr, w.gemm_ws, GEMM_SPLIT_BYTES)))
-          return rc;
-        if ((rc = launch_rope_kv_write(st, c.dtype, w.qkv, qkv_rows(), w.q, nullptr, nullptr, cos_tab, sin_tab, nullptr,
-                                       c.max_pos, B, T, c.heads, c.kv_heads, D, s.max_seq, 0, nullptr, w.st, l)))
-          return rc;
-      }
+      GemvArgs p{};
+      p.x = w.x;
+      p.ldx = H;
+      p.norm_w = L(l, MINITP_W_LN1);
+      p.eps = c.eps;
+      p.w = L(l, MINITP_W_QKV);
+      p.bias = L(l, MINITP_W_QKV_BIAS);
+      p.y = w.q;
+      p.ldy = q_rows();
+      p.M = M;
+      p.N = qkv_rows();
+      p.K = H;
+      p.st = w.st;
+      p.cos_tab = cos_tab;
+      p.sin_tab = sin_tab;
+      p.max_pos = c.max_pos;
+      p.layer = l;
+      p.a = as;
+      if ((rc = launch_gemv(st, c.dtype, PRO_NORM, EPI_QKV_ROPE, p))) return rc;
       if (fo) {
         const OprojArgs o{L(l, MINITP_W_O), H, attn_oproj_rows(c.dtype, as, H, OPROJ_SLICES), w.opart};
         if ((rc = launch_decode_attention_oproj(st, c.dtype, w.q, as, w.st, l, o))) return rc;
@@ -385,9 +360,7 @@ struct Qwen2Program {
         const char* vc = (const char*)s.v_cache + l * layer_elems * es();
         if ((rc = launch_prefill_attention(st, c.dtype, w.q, kc, vc, w.attn, as, s.cache_len, w.st, l))) return rc;
       }
-      if (fo) {
-        // (o_proj ran in the attention kernel)
-      } else if (fz) {
+      if (!fo) {  // (else o_proj ran in the attention kernel)
         GemvArgs g{};
         g.x = w.attn;
         g.ldx = q_rows();
@@ -402,58 +375,42 @@ struct Qwen2Program {
         // split form's three extra at K = 896)
         if (!gemv_mfma_rows(c.dtype, M)) split_bufs(g);
         if ((rc = launch_gemv(st, c.dtype, PRO_NONE, EPI_RESID, g))) return rc;
-      } else {
-        if ((rc = launch_gemm(st, c.dtype, w.attn, q_rows(), L(l, MINITP_W_O), nullptr, w.x, H, M, H, q_rows(),
-                              MINITP_EPI_RESID, w.x, nullptr, w.gemm_ws, GEMM_SPLIT_BYTES)))
-          return rc;
       }
       // ---- MLP block ----------------------------------------------------------
-      if (fz) {
-        GemvArgs g{};
-        g.x = w.x;
-        g.ldx = H;
-        g.norm_w = L(l, MINITP_W_LN2);
-        g.eps = c.eps;
-        g.w = L(l, MINITP_W_GATE_UP);
-        g.y = w.act;
-        g.ldy = I;
-        g.M = M;
-        g.N = I;
-        g.K = H;
-        if (fo) {
-          // x + o_proj (the attention's partials) -> h, then as above
-          g.part = w.opart;
-          g.nparts = c.heads;
-          g.x_out = w.h;
-          if ((rc = launch_gemv_part_swiglu(st, c.dtype, g))) return rc;
-        } else if ((rc = launch_gemv(st, c.dtype, PRO_NORM, EPI_SWIGLU, g))) {
-          return rc;
-        }
-        // the down projection's long K splits over blocks (register form
-        // past 8,192, MFMA form at 5..32 rows)
-        GemvArgs d{};
-        d.x = w.act;
-        d.ldx = I;
-        d.w = L(l, MINITP_W_DOWN);
-        d.y = w.x;
-        d.ldy = H;
-        d.aux = fo ? w.h : w.x;
-        d.M = M;
-        d.N = H;
-        d.K = I;
-        split_bufs(d);
-        if ((rc = launch_gemv(st, c.dtype, PRO_NONE, EPI_RESID, d))) return rc;
-      } else {
-        if ((rc = launch_rmsnorm(st, c.dtype, w.x, L(l, MINITP_W_LN2), w.h, M, H, c.eps))) return rc;
-        if ((rc = launch_gemm(st, c.dtype, w.h, H, L(l, MINITP_W_GATE_UP), nullptr, w.gu, 2 * I, M, 2 * I, H,
-                              MINITP_EPI_NONE, nullptr, nullptr, w.gemm_ws, GEMM_SPLIT_BYTES)))
-          return rc;
-        const char* up = (const char*)w.gu + I * es();
-        if ((rc = launch_silu_mul(st, c.dtype, w.gu, up, 2 * I, w.act, I, M, I))) return rc;
-        if ((rc = launch_gemm(st, c.dtype, w.act, I, L(l, MINITP_W_DOWN), nullptr, w.x, H, M, H, I, MINITP_EPI_RESID,
-                              w.x, nullptr, w.gemm_ws, GEMM_SPLIT_BYTES)))
-          return rc;
+      GemvArgs g{};
+      g.x = w.x;
+      g.ldx = H;
+      g.norm_w = L(l, MINITP_W_LN2);
+      g.eps = c.eps;
+      g.w = L(l, MINITP_W_GATE_UP);
+      g.y = w.act;
+      g.ldy = I;
+      g.M = M;
+      g.N = I;
+      g.K = H;
+      if (fo) {
+        // x + o_proj (the attention's partials) -> h, then as above
+        g.part = w.opart;
+        g.nparts = c.heads;
+        g.x_out = w.h;
+        if ((rc = launch_gemv_part_swiglu(st, c.dtype, g))) return rc;
+      } else if ((rc = launch_gemv(st, c.dtype, PRO_NORM, EPI_SWIGLU, g))) {
+        return rc;
       }
+      // the down projection's long K splits over blocks (register form
+      // past 8,192, MFMA form at 5..32 rows)
+      GemvArgs d{};
+      d.x = w.act;
+      d.ldx = I;
+      d.w = L(l, MINITP_W_DOWN);
+      d.y = w.x;
+      d.ldy = H;
+      d.aux = fo ? w.h : w.x;
+      d.M = M;
+      d.N = H;
+      d.K = I;
+      split_bufs(d);
+      if ((rc = launch_gemv(st, c.dtype, PRO_NONE, EPI_RESID, d))) return rc;
     }
     // ---- final norm, LM head, greedy pick ----------------------------------------
     if (!s.logits_all && gemv_supported(c.dtype, B, H) && !gemv_mfma_rows(c.dtype, B)) {
@@ -508,10 +465,10 @@ struct Qwen2Program {
                              (T - 1) * V);
       return MINITP_OK;
     }
-    if (!blas && (rc = launch_rmsnorm(st, c.dtype, w.x, final_norm, w.h, M, H, c.eps))) return rc;
-    if (s.logits_all) {  // (with blas, h already holds norm(x))
+    if (!gemm && (rc = launch_rmsnorm(st, c.dtype, w.x, final_norm, w.h, M, H, c.eps))) return rc;
+    if (s.logits_all) {  // (on the GEMM path h already holds norm(x))
       rc = MINITP_ERR_UNSUPPORTED;
-      if (blas && gemm_tile_supported(M, V, H, H, V, false))
+      if (head_on_tile(M))
         rc = launch_gemm_tile(st, w.h, H, lm_head, nullptr, s.logits, V, M, V, H, false, tail);
       if (rc == MINITP_ERR_UNSUPPORTED)
         rc = launch_gemm(st, c.dtype, w.h, H, lm_head, nullptr, nullptr, V, M, V, H, MINITP_EPI_NONE, nullptr, w.st);

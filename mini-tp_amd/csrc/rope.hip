@@ -129,95 +129,98 @@ __global__ void rope_kv_write_kernel(const T* qkv, int64_t ld, T* q_out, T* k_ca
   }
 }
 
-__device__ __forceinline__ void store8_bf16(bf16* dst, const float* v) {
-  if (((uintptr_t)dst & 15u) == 0) {
-    *reinterpret_cast<uint4*>(dst) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
-                                                pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) store_f32<bf16>(dst, e, v[e]);
-  }
-}
-
-// The same as rope_kv_write_kernel<bf16> for D / 2 % 8 == 0, eight pairs per
-// thread: 16-byte loads of the qkv row (the caller checks its alignment) and
-// of the fp32 tables, 16-byte stores wherever the destination allows them.
+// The same as rope_kv_write_kernel with W pairs per thread (D / 2 % W == 0):
+// vector loads of the qkv row (the caller checks its alignment) and of the
+// fp32 tables, vector stores wherever the destination allows them. One block
+// per token, so the only divisions are 32-bit ones by the pieces of a head.
 // PART: the projection is the split-K partial product (qp) plus the bias,
-// rounded to bf16 as gemm_reduce_kernel stores it, instead of a qkv row.
-template <bool PART>
-__global__ void rope_kv_write8_kernel(const bf16* qkv, int64_t ld, Partials qp, const bf16* bias, bf16* q_out,
-                                      bf16* k_cache, bf16* v_cache, const float* cos_tab, const float* sin_tab,
-                                      const int64_t* positions, int64_t max_pos, int64_t B, int64_t T_, int64_t Hq,
-                                      int64_t Hkv, int64_t D, int64_t S, int64_t cache_len, int32_t* error_flag,
-                                      const StepState* state, int layer) {
+// rounded to the dtype as gemm_reduce_kernel stores it, instead of a qkv row.
+template <typename T, int W, bool PART>
+__global__ __launch_bounds__(256) void rope_kv_writev_kernel(const T* qkv, int64_t ld, Partials qp, const T* bias,
+                                                             T* q_out, T* k_cache, T* v_cache, const float* cos_tab,
+                                                             const float* sin_tab, const int64_t* positions,
+                                                             int64_t max_pos, int64_t B, int T_, int Hq, int Hkv,
+                                                             int D, int64_t S, int64_t cache_len, int32_t* error_flag,
+                                                             const StepState* state, int layer) {
+  int halted = 0;
   if (state != nullptr) {
     const int64_t layer_off = (int64_t)layer * B * Hkv * S * D;
     positions = state->args.positions;
     cache_len = state->args.cache_len;
-    k_cache = (bf16*)state->args.k_cache + layer_off;
-    v_cache = (bf16*)state->args.v_cache + layer_off;
+    k_cache = (T*)state->args.k_cache + layer_off;
+    v_cache = (T*)state->args.v_cache + layer_off;
     error_flag = (int32_t*)&state->error;
+    halted = state->halted;
   }
-  const int64_t half = D / 2, groups = half / 8, heads = Hq + 2 * Hkv;
-  int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (idx >= B * T_ * heads * groups) return;
-  const int64_t i = (idx % groups) * 8;
-  const int64_t head = (idx / groups) % heads;
-  if (state != nullptr && state->halted && head >= Hq) return;
-  const int64_t n = idx / (groups * heads);
-  const int64_t b = n / T_, t = n % T_;
-  float xa[8], xb[8], oa[8], ob[8];
-  if constexpr (PART) {
-    const int64_t col = head * D + i;
-    float va[8], vb[8], ba[8], bb[8];
-    sum_partials8(qp, n, col, va);
-    sum_partials8(qp, n, col + half, vb);
-    unpack16(*reinterpret_cast<const uint4*>(bias + col), ba, (bf16*)nullptr);
-    unpack16(*reinterpret_cast<const uint4*>(bias + col + half), bb, (bf16*)nullptr);
+  const int64_t n = blockIdx.x;
+  const int b = (int)(blockIdx.x / (unsigned)T_), t = (int)(blockIdx.x % (unsigned)T_);
+  const int64_t pos = positions[t];
+  const bool pos_ok = pos >= 0 && pos < max_pos;
+  const int half = D / 2, groups = half / W, heads = Hq + 2 * Hkv;
+  for (int idx = threadIdx.x; idx < heads * groups; idx += blockDim.x) {
+    const int head = idx / groups, i = (idx % groups) * W;
+    if (halted && head >= Hq) return;
+    float xa[W], xb[W], oa[W], ob[W];
+    if constexpr (PART) {
+      const int64_t col = (int64_t)head * D + i;
+      float ba[W], bb[W];
+      load_vec<T, W>(bias + col, ba);
+      load_vec<T, W>(bias + col + half, bb);
+      sum_partials<W>(qp, n, col, xa);
+      sum_partials<W>(qp, n, col + half, xb);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      xa[e] = round_to<bf16>(va[e] + ba[e]);
-      xb[e] = round_to<bf16>(vb[e] + bb[e]);
-    }
-  } else {
-    const bf16* src = qkv + n * ld + head * D;
-    unpack16(*reinterpret_cast<const uint4*>(src + i), xa, (bf16*)nullptr);
-    unpack16(*reinterpret_cast<const uint4*>(src + i + half), xb, (bf16*)nullptr);
-  }
-  bf16* dst;
-  if (head < Hq + Hkv) {
-    const int64_t pos = positions[t];
-    if (pos < 0 || pos >= max_pos) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) oa[e] = ob[e] = __builtin_nanf("");
-      if (error_flag) *error_flag = 1;
+      for (int e = 0; e < W; ++e) {
+        xa[e] = round_to<T>(xa[e] + ba[e]);
+        xb[e] = round_to<T>(xb[e] + bb[e]);
+      }
     } else {
-      const float4* cr = reinterpret_cast<const float4*>(cos_tab + pos * D + i);
-      const float4* sr = reinterpret_cast<const float4*>(sin_tab + pos * D + i);
-      const float4 c0 = cr[0], c1 = cr[1], s0 = sr[0], s1 = sr[1];
-      const float4 c2 = cr[half / 4], c3 = cr[half / 4 + 1], s2 = sr[half / 4], s3 = sr[half / 4 + 1];
-      const float ca[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-      const float sa[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-      const float cb[8] = {c2.x, c2.y, c2.z, c2.w, c3.x, c3.y, c3.z, c3.w};
-      const float sb[8] = {s2.x, s2.y, s2.z, s2.w, s3.x, s3.y, s3.z, s3.w};
+      const T* src = qkv + n * ld + head * D;
+      load_vec<T, W>(src + i, xa);
+      load_vec<T, W>(src + i + half, xb);
+    }
+    T* dst;
+    if (head < Hq + Hkv) {
+      if (!pos_ok) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        oa[e] = add_rn(mul_rn(xa[e], ca[e]), -mul_rn(xb[e], sa[e]));
-        ob[e] = add_rn(mul_rn(xb[e], cb[e]), mul_rn(xa[e], sb[e]));
+        for (int e = 0; e < W; ++e) oa[e] = ob[e] = __builtin_nanf("");
+        if (error_flag) *error_flag = 1;
+      } else {
+        float ca[W], sa[W], cb[W], sb[W];
+        load_vec<float, W>(cos_tab + pos * D + i, ca);
+        load_vec<float, W>(sin_tab + pos * D + i, sa);
+        load_vec<float, W>(cos_tab + pos * D + i + half, cb);
+        load_vec<float, W>(sin_tab + pos * D + i + half, sb);
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+          oa[e] = add_rn(mul_rn(xa[e], ca[e]), -mul_rn(xb[e], sa[e]));
+          ob[e] = add_rn(mul_rn(xb[e], cb[e]), mul_rn(xa[e], sb[e]));
+        }
+      }
+      dst = head < Hq ? q_out + (n * Hq + head) * D
+                      : k_cache + (((int64_t)b * Hkv + (head - Hq)) * S + cache_len + t) * D;
+    } else {
+#pragma unroll
+      for (int e = 0; e < W; ++e) {
+        oa[e] = xa[e];
+        ob[e] = xb[e];
+      }
+      dst = v_cache + (((int64_t)b * Hkv + (head - Hq - Hkv)) * S + cache_len + t) * D;
+    }
+    if (((uintptr_t)dst & 15u) == 0) {
+      store_vec<T, W>(dst + i, oa);
+      store_vec<T, W>(dst + i + half, ob);
+    } else {
+#pragma unroll
+      for (int e = 0; e < W; ++e) {
+        store_f32<T>(dst, i + e, oa[e]);
+        store_f32<T>(dst, i + e + half, ob[e]);
       }
     }
-    dst = head < Hq ? q_out + (n * Hq + head) * D : k_cache + ((b * Hkv + (head - Hq)) * S + cache_len + t) * D;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      oa[e] = xa[e];
-      ob[e] = xb[e];
-    }
-    dst = v_cache + ((b * Hkv + (head - Hq - Hkv)) * S + cache_len + t) * D;
   }
-  store8_bf16(dst + i, oa);
-  store8_bf16(dst + i + half, ob);
 }
+
+// threads of a block of rope_kv_writev_kernel: its pieces, in whole waves
+inline unsigned rope_threads(int64_t pieces) { return (unsigned)std::min<int64_t>(256, cdiv(pieces, 64) * 64); }
 
 int launch_rope_kv_write(hipStream_t st, int dtype, const void* qkv, int64_t ld_qkv, void* q_out, void* k_cache,
                          void* v_cache, const float* cos_tab, const float* sin_tab, const int64_t* positions,
@@ -225,11 +228,18 @@ int launch_rope_kv_write(hipStream_t st, int dtype, const void* qkv, int64_t ld_
                          int64_t cache_len, int32_t* error_flag, const StepState* state, int layer) {
   const int64_t n = B * T_ * (Hq + 2 * Hkv) * (D / 2);
   if (n == 0) return MINITP_OK;
-  if (dtype == MINITP_BF16 && D % 16 == 0 && ld_qkv % 8 == 0 && aligned16(qkv) && aligned16(cos_tab) &&
-      aligned16(sin_tab)) {
-    rope_kv_write8_kernel<false><<<(unsigned)cdiv(n / 8, 256), 256, 0, st>>>(
-        (const bf16*)qkv, ld_qkv, Partials{}, nullptr, (bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, cos_tab, sin_tab,
-        positions, max_pos, B, T_, Hq, Hkv, D, S, cache_len, error_flag, state, layer);
+  const int64_t w = dtype == MINITP_F32 ? 4 : 8, heads = Hq + 2 * Hkv;
+  if (D % (2 * w) == 0 && ld_qkv % w == 0 && B * T_ < (1LL << 31) && heads * D < (1LL << 31) && aligned16(qkv) &&
+      aligned16(cos_tab) && aligned16(sin_tab)) {
+    const unsigned threads = rope_threads(heads * (D / 2 / w));
+    if (dtype == MINITP_F32)
+      rope_kv_writev_kernel<float, 4, false><<<(unsigned)(B * T_), threads, 0, st>>>(
+          (const float*)qkv, ld_qkv, Partials{}, nullptr, (float*)q_out, (float*)k_cache, (float*)v_cache, cos_tab,
+          sin_tab, positions, max_pos, B, (int)T_, (int)Hq, (int)Hkv, (int)D, S, cache_len, error_flag, state, layer);
+    else
+      rope_kv_writev_kernel<bf16, 8, false><<<(unsigned)(B * T_), threads, 0, st>>>(
+          (const bf16*)qkv, ld_qkv, Partials{}, nullptr, (bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, cos_tab,
+          sin_tab, positions, max_pos, B, (int)T_, (int)Hq, (int)Hkv, (int)D, S, cache_len, error_flag, state, layer);
     MINITP_LAUNCH_CHECK();
     return MINITP_OK;
   }
@@ -246,19 +256,29 @@ int launch_rope_kv_write(hipStream_t st, int dtype, const void* qkv, int64_t ld_
   return MINITP_OK;
 }
 
-int launch_rope_kv_write_partials(hipStream_t st, const Partials& qkv, const void* bias, void* q_out,
+int launch_rope_kv_write_partials(hipStream_t st, int dtype, const Partials& qkv, const void* bias, void* q_out,
                                   const float* cos_tab, const float* sin_tab, int64_t max_pos, int64_t B, int64_t T_,
                                   int64_t Hq, int64_t Hkv, int64_t D, int64_t S, const StepState* state, int layer) {
-  const int64_t n = B * T_ * (Hq + 2 * Hkv) * (D / 2);
+  const int64_t heads = Hq + 2 * Hkv, n = B * T_ * heads * (D / 2);
   if (n == 0) return MINITP_OK;
-  if (state == nullptr || bias == nullptr || D % 16 != 0 || qkv.M != B * T_ || qkv.N != (Hq + 2 * Hkv) * D ||
-      qkv.S < 1 || !aligned16(qkv.p) || !aligned16(bias) || !aligned16(cos_tab) || !aligned16(sin_tab)) {
+  if (state == nullptr || bias == nullptr || D % 16 != 0 || qkv.M != B * T_ || qkv.N != heads * D || qkv.S < 1 ||
+      B * T_ >= (1LL << 31) || heads * D >= (1LL << 31) || !aligned16(qkv.p) || !aligned16(bias) ||
+      !aligned16(cos_tab) || !aligned16(sin_tab)) {
     set_error("rope_kv_write from partials: D %lld, partial width %lld", (long long)D, (long long)qkv.N);
     return MINITP_ERR_UNSUPPORTED;
   }
-  rope_kv_write8_kernel<true><<<(unsigned)cdiv(n / 8, 256), 256, 0, st>>>(
-      nullptr, 0, qkv, (const bf16*)bias, (bf16*)q_out, nullptr, nullptr, cos_tab, sin_tab, nullptr, max_pos, B, T_, Hq,
-      Hkv, D, S, 0, nullptr, state, layer);
+  // (four pairs a thread: 128 tokens of the 0.5B shape then load their
+  // partials from 128 blocks of 192 threads; as 36 blocks of 256 threads of
+  // eight pairs with 64-bit index divisions this launch took 6.5 us, now 4.4)
+  const unsigned threads = rope_threads(heads * (D / 8));
+  if (dtype == MINITP_F32)
+    rope_kv_writev_kernel<float, 4, true><<<(unsigned)(B * T_), threads, 0, st>>>(
+        nullptr, 0, qkv, (const float*)bias, (float*)q_out, nullptr, nullptr, cos_tab, sin_tab, nullptr, max_pos, B,
+        (int)T_, (int)Hq, (int)Hkv, (int)D, S, 0, nullptr, state, layer);
+  else
+    rope_kv_writev_kernel<bf16, 4, true><<<(unsigned)(B * T_), threads, 0, st>>>(
+        nullptr, 0, qkv, (const bf16*)bias, (bf16*)q_out, nullptr, nullptr, cos_tab, sin_tab, nullptr, max_pos, B,
+        (int)T_, (int)Hq, (int)Hkv, (int)D, S, 0, nullptr, state, layer);
   MINITP_LAUNCH_CHECK();
   return MINITP_OK;
 }

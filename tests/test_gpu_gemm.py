@@ -1,0 +1,96 @@
+"""The MFMA GEMM of prompts and batched decode (csrc/gemm.hip) at the edges of
+its tiles: rows and columns just below, at and past each tile shape, K tails
+shorter than a stage and shorter than the ring, and shapes on both sides of
+the tile-choice rule (64 x 64 up to 256 x 128).
+
+Bar: against float64 products. fp32 sums of K terms in any order are off by
+at most K 2^-24 sum |x_k w_k| (twice that for fp32 operands, whose products
+round too), and a bf16 output is off by half a step more (2^-9 relative);
+both are doubled here.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+SHAPES = [
+    (33, 64, 8),          # one stage, one chunk of it
+    (63, 130, 72),        # ragged columns (not a multiple of 4), K tail of one chunk
+    (64, 896, 896),
+    (65, 1152, 200),
+    (100, 77, 264),       # odd width
+    (129, 4608, 1000),
+    (194, 9728, 896),
+    (257, 640, 4864),     # long K on few tiles
+    (433, 3584, 1096),    # 64 x 128 and 128 x 128 tiles at 7B widths
+    (700, 9728, 520),
+    (2000, 3584, 384),    # 256 x 128 tiles
+]
+
+
+def _bound(ref, x, w, dtype, k):
+    mag = x.double().abs() @ w.double().abs().t()
+    eps = 2.0 ** -24 * k * (2 if dtype == torch.float32 else 1)
+    return 2 * (eps * mag + (2.0 ** -9 * ref.abs() if dtype == torch.bfloat16 else 2.0 ** -24 * ref.abs())) + 1e-30
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_linear_matches_float64(m, n, k, dtype):
+    """Plain product, with and without bias, from rows inside a wider buffer
+    whose other columns are NaN (nothing past K may reach a sum)."""
+    from minitp import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(m * 7 + n + k)
+    wide = torch.full((m, k + 64), float("nan"), dtype=dtype, device=DEV)
+    wide[:, :k] = torch.randn(m, k, generator=g, device=DEV).to(dtype)
+    x = wide[:, :k]
+    w = (torch.randn(n, k, generator=g, device=DEV) * 0.05).to(dtype)
+    bias = torch.randn(n, generator=g, device=DEV).to(dtype)
+    ref = x.double() @ w.double().t()
+    for b, r in ((None, ref), (bias, ref + bias.double())):
+        got = K.linear(x, w, b).double()
+        assert torch.isfinite(got).all()
+        over = ((got - r).abs() - _bound(r, x, w, dtype, k)).max().item()
+        assert over <= 0, (b is not None, over)
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 1152, 200), (433, 3584, 1096)])
+def test_linear_resid_matches_float64(m, n, k):
+    from minitp import _native as N
+    from minitp import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=DEV) * 0.05).bfloat16()
+    aux = torch.randn(m, n, generator=g, device=DEV).bfloat16()
+    prod = x.double() @ w.double().t()
+    got = K.linear(x, w, epilogue=N.EPI_RESID, aux=aux).double()
+    ref = prod + aux.double()
+    bar = _bound(prod, x, w, torch.bfloat16, k) + 2 * 2.0 ** -9 * ref.abs()
+    assert ((got - ref).abs() <= bar).all()
+
+
+@pytest.mark.parametrize("tokens", [33, 65, 129, 200, 321])
+def test_swiglu_forms_agree_with_the_module(tokens):
+    """A prompt's gate/up product with SwiGLU in the GEMM's epilogue (the
+    native forward) against the module path (product, then SwiGLU), one
+    layer at the 0.5B widths: logits and cache rows."""
+    import dataclasses
+
+    from minitp import synthetic
+    from minitp.generation import make_kv_cache
+
+    cfg = dataclasses.replace(synthetic.QWEN05B, num_hidden_layers=2, vocab_size=4096)
+    model = synthetic.build_synthetic_model(cfg, dtype=torch.bfloat16, device=DEV, seed=0)
+    ids = synthetic.synthetic_prompt(cfg.vocab_size, 1, tokens, seed=1, device=DEV)
+    out = []
+    for rotary in (True, False):  # False: the module path
+        model.use_rotary_cache = rotary
+        kv = make_kv_cache(model, 1, tokens, init="zeros")
+        out.append((model(ids, kv_cache=kv).float(), kv.k[1].float()))
+    model.use_rotary_cache = True
+    for a, b in zip(*out):
+        torch.testing.assert_close(a, b, atol=0.05, rtol=0.02)
