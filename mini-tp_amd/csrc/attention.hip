@@ -742,82 +742,163 @@ struct PrefillKV {
 };
 
 // ---------------------------------------------------------------------------
-// Prefill: flash-style causal attention, fp32 FMA. Block = (b * Hq + h,
-// 64-query tile); 4 lanes per query, each owning D/4 dims; key tiles of K
-// and V (64 keys, 32 at D = 128) staged in LDS as fp32.
+// Prefill, fp32, on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 products
+// and sums). Block = (b * Hq + h, 64-query tile), wave w = the 16-query strip
+// 16 w of it. Per tile of KT keys staged in LDS the products run transposed:
+// S^T = K Q^T leaves lane (quad, r) = (l / 16, l % 16) holding keys
+// 4 quad .. 4 quad + 3 of query r, which register by register is the B operand
+// of O^T = V^T P^T (MFMA e takes key 4 quad + e from both operands), so the
+// probabilities never leave the registers and each lane's softmax state is
+// its own query's.
+// A lane's operands are 16-byte LDS reads: MFMA i of a K chunk takes dims
+// 16 c + 4 quad + i (Q alike), MFMA j of a V row dims E r + j (E = D / 16,
+// at most 4; a second half from 64 on at D = 128), so an output register's
+// E dims are consecutive in memory. Rows are padded by 16 bytes: the 16 rows
+// of a K read, and the four rows of a V read, fall in different banks.
+// The next tile's loads are in flight during a tile's math. Bound by the
+// fp32 MFMAs and the softmax's latency chain on few blocks: 3 x 333 tokens,
+// 14 heads of 64 (252 blocks) 241 us on fp32 FMAs with one query per four
+// lanes, 24 us here.
 constexpr int QT = 64;
 
-template <typename T, int D>
-__global__ __launch_bounds__(256) void prefill_attn_kernel(const T* q, const T* kc, const T* vc, T* out, AttnShape s,
-                                                           int64_t cache_len, float scale, PrefillKV kv) {
+template <int D>
+__global__ __launch_bounds__(256) void prefill_attn_f32_kernel(const float* q, const float* kc, const float* vc,
+                                                               float* out, AttnShape s, int64_t cache_len, float scale,
+                                                               PrefillKV kv) {
   kv.resolve(kc, vc, cache_len);
-  constexpr int DQ = D / 4;
-  constexpr int KT = D >= 128 ? 32 : 64;
-  __shared__ float Ks[KT][D + 1];
-  __shared__ float Vs[KT][D + 1];
+  typedef float f32x4_t __attribute__((ext_vector_type(4)));
+  constexpr int KT = D >= 128 ? 32 : 64;         // keys per tile
+  constexpr int KB = KT / 16;                    // 16-key blocks per tile
+  constexpr int KC = D / 16;                     // 16-dim chunks of a score
+  constexpr int E = D / 16 < 4 ? D / 16 : 4;     // dims of a V row per lane and half
+  constexpr int HALVES = D / 16 / E;
+  constexpr int ROW = D + 4;                     // LDS floats per row
+  constexpr int PIECES = KT * D / 4, PER = (PIECES + 255) / 256;
+  __shared__ __attribute__((aligned(16))) float Ks[KT * ROW];
+  __shared__ __attribute__((aligned(16))) float Vs[KT * ROW];
   const int G = s.Hq / s.Hkv;
   const int bh = blockIdx.x, b = bh / s.Hq, h = bh % s.Hq, g = h / G;
-  const int tid = threadIdx.x, qi = tid / 4, quarter = tid % 4;
-  const int64_t t = (int64_t)blockIdx.y * QT + qi;  // query index in this forward
-  const bool q_ok = t < s.T;
-  const T* kbase = kc + ((int64_t)b * s.Hkv + g) * s.S * D;
-  const T* vbase = vc + ((int64_t)b * s.Hkv + g) * s.S * D;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lr = lane % 16, lq = lane / 16;
+  // the longest query tiles first
+  const int64_t tile0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * QT;
+  const int64_t t0 = tile0 + wave * 16, t = t0 + lr;
+  const float* kbase = kc + ((int64_t)b * s.Hkv + g) * s.S * D;
+  const float* vbase = vc + ((int64_t)b * s.Hkv + g) * s.S * D;
 
-  float qv[DQ], o[DQ];
+  f32x4_t qa[KC];
+  {
+    const float* qrow = q + (((int64_t)b * s.T + (t < s.T ? t : 0)) * s.Hq + h) * D;
 #pragma unroll
-  for (int i = 0; i < DQ; ++i) {
-    qv[i] = q_ok ? load_f32<T>(q, (((int64_t)b * s.T + t) * s.Hq + h) * D + quarter * DQ + i) : 0.f;
-    o[i] = 0.f;
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) qa[c][i] = qrow[16 * c + 4 * lq + i];
   }
-  float m = -__builtin_inff(), l = 0.f;
-  const int64_t limit = cache_len + t;  // last key this query may see
-  const int64_t t_last = std::min<int64_t>((int64_t)blockIdx.y * QT + QT, s.T) - 1;
-  const int64_t key_end = cache_len + t_last + 1;  // keys needed by the tile
+  f32x4_t o[HALVES][E];
+#pragma unroll
+  for (int hf = 0; hf < HALVES; ++hf)
+#pragma unroll
+    for (int j = 0; j < E; ++j) o[hf][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -__builtin_inff(), lsum = 0.f;  // this lane's query; lsum over its own keys
+  const int64_t tb_last = std::min<int64_t>(tile0 + QT, s.T) - 1;
+  const int64_t key_end = cache_len + tb_last + 1;  // keys the block's queries may see
 
+  const uint32_t kv_bytes = (uint32_t)(key_end * D * 4);
+  const __amdgpu_buffer_rsrc_t krs = span_rsrc(kbase, kv_bytes), vrs = span_rsrc(vbase, kv_bytes);
+  uint4 kr[PER], vr[PER];
+  auto load_tile = [&](int64_t k0) {  // rows past key_end read zeros
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = tid + 256 * u;
+      const int64_t key = k0 + i / (D / 4);
+      const uint32_t off = i < PIECES && key < key_end ? (uint32_t)((key * D + i % (D / 4) * 4) * 4) : kv_bytes;
+      kr[u] = attn_load16(krs, off);
+      vr[u] = attn_load16(vrs, off);
+    }
+  };
+  load_tile(0);
   for (int64_t k0 = 0; k0 < key_end; k0 += KT) {
-    __syncthreads();
-    for (int i = tid; i < KT * D; i += 256) {
-      const int j = i / D, d = i % D;
-      const bool ok = k0 + j < key_end;
-      Ks[j][d] = ok ? load_f32<T>(kbase, (k0 + j) * D + d) : 0.f;
-      Vs[j][d] = ok ? load_f32<T>(vbase, (k0 + j) * D + d) : 0.f;
+    __syncthreads();  // the previous tile is consumed
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = tid + 256 * u;
+      if (i < PIECES) {
+        const int at = i / (D / 4) * ROW + i % (D / 4) * 4;
+        *(uint4*)(Ks + at) = kr[u];
+        *(uint4*)(Vs + at) = vr[u];
+      }
     }
     __syncthreads();
-    float sc[KT];
-    float tile_max = -__builtin_inff();
-#pragma unroll 8
-    for (int j = 0; j < KT; ++j) {
-      float p = 0.f;
+    if (k0 + KT < key_end) load_tile(k0 + KT);
+    if (t0 >= s.T || k0 > cache_len + t0 + 15) continue;  // this strip sees none of the tile
+    const int64_t limit = cache_len + t - k0;             // last key of the tile this query may see
+    float sc[KB][4];
+    float mx = -__builtin_inff();
 #pragma unroll
-      for (int i = 0; i < DQ; ++i) p = fmaf(qv[i], Ks[j][quarter * DQ + i], p);
-      p += __shfl_xor(p, 1, 64);
-      p += __shfl_xor(p, 2, 64);
-      const bool ok = k0 + j <= limit;
-      sc[j] = ok ? p * scale : -__builtin_inff();
-      tile_max = fmaxf(tile_max, sc[j]);
+    for (int kb = 0; kb < KB; ++kb) {
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const f32x4_t kv4 = *(const f32x4_t*)(Ks + (kb * 16 + lr) * ROW + 16 * c + 4 * lq);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv4[i], qa[c][i], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sc[kb][e] = kb * 16 + 4 * lq + e <= limit ? acc[e] * scale : -__builtin_inff();
+        mx = fmaxf(mx, sc[kb][e]);
+      }
     }
-    const float m_new = fmaxf(m, tile_max);
-    if (m_new == -__builtin_inff()) continue;  // nothing visible yet
-    const float alpha = expf(m - m_new);
-    l *= alpha;
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mn = fmaxf(m, mx);
+    const float alpha = mn == -__builtin_inff() ? 1.f : expf(m - mn);
+    m = mn;
+    lsum *= alpha;
 #pragma unroll
-    for (int i = 0; i < DQ; ++i) o[i] *= alpha;
-#pragma unroll 8
-    for (int j = 0; j < KT; ++j) {
-      const float p = expf(sc[j] - m_new);
-      l += p;
+    for (int hf = 0; hf < HALVES; ++hf)
 #pragma unroll
-      for (int i = 0; i < DQ; ++i) o[i] = fmaf(p, Vs[j][quarter * DQ + i], o[i]);
+      for (int j = 0; j < E; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[hf][j][e] *= alpha;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float p = sc[kb][e] == -__builtin_inff() ? 0.f : expf(sc[kb][e] - mn);
+        lsum += p;
+        const float* vrow = Vs + (kb * 16 + 4 * lq + e) * ROW + E * lr;
+#pragma unroll
+        for (int hf = 0; hf < HALVES; ++hf) {
+          float v[E];
+          if constexpr (E == 4) {
+            const f32x4_t v4 = *(const f32x4_t*)(vrow + 64 * hf);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = v4[j];
+          } else {
+#pragma unroll
+            for (int j = 0; j < E; ++j) v[j] = vrow[j];
+          }
+#pragma unroll
+          for (int j = 0; j < E; ++j) o[hf][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], p, o[hf][j], 0, 0, 0);
+        }
+      }
     }
-    m = m_new;
   }
-  if (q_ok) {
+  if (t0 >= s.T) return;
+  float l = lsum;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (t >= s.T) return;
+  // o[hf][j][e]: row 4 lq + e of the MFMA's 16, dim 64 hf + E (4 lq + e) + j
+  float* orow = out + (((int64_t)b * s.T + t) * s.Hq + h) * D;
 #pragma unroll
-    for (int i = 0; i < DQ; ++i)
-      store_f32<T>(out, (((int64_t)b * s.T + t) * s.Hq + h) * D + quarter * DQ + i, o[i] / l);
-  }
+  for (int hf = 0; hf < HALVES; ++hf)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int j = 0; j < E; ++j) orow[64 * hf + E * (4 * lq + e) + j] = o[hf][j][e] / l;
 }
-
 
 // Prefill on matrix cores (bf16): block = (b * Hq + h, PQ-query tile), wave
 // w = the 16-query strip t0 = PQ y + 16 w (all strips share each staged tile). Per 64-key tile staged in LDS (K
@@ -1328,8 +1409,8 @@ int prefill_dispatch(hipStream_t st, const void* q, const void* k, const void* v
       hipLaunchKernelGGL((prefill_attn_mfma_kernel<D, 4>), dim3(s.B * s.Hq, (unsigned)cdiv(s.T, 64)), dim3(256), 0,
                          st, (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, s, cache_len, scale, kv);
   } else
-    hipLaunchKernelGGL((prefill_attn_kernel<T, D>), dim3(s.B * s.Hq, (unsigned)cdiv(s.T, QT)), dim3(256), 0, st,
-                       (const T*)q, (const T*)k, (const T*)v, (T*)out, s, cache_len, scale, kv);
+    hipLaunchKernelGGL((prefill_attn_f32_kernel<D>), dim3(s.B * s.Hq, (unsigned)cdiv(s.T, QT)), dim3(256), 0, st,
+                       (const float*)q, (const float*)k, (const float*)v, (float*)out, s, cache_len, scale, kv);
   MINITP_LAUNCH_CHECK();
   return MINITP_OK;
 }

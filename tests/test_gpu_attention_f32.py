@@ -1,0 +1,57 @@
+"""fp32 prompt attention on the matrix cores (csrc/attention.hip) at the edges
+of its 16-query strips, 64-query blocks and 32- / 64-key tiles, for every head
+dim it serves, with the cache rows past the last key poisoned.
+
+Bar: rounding errors taken as independent, a score of D products carries
+about 2^-24 sqrt(D) (7e-7 at D = 128), so each probability that relative
+error plus two roundings of the exponential, and an output of values of order
+1 the same; five standard deviations over the outputs, twice: 1e-5.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+@pytest.mark.parametrize("t,cache_len", [(2, 0), (15, 1), (16, 16), (17, 31), (33, 33), (63, 64), (64, 0), (65, 127),
+                                         (130, 5), (333, 0), (200, 700)])
+def test_prefill_attention_f32_matches_float64(t, cache_len, d):
+    from minitp import kernels as K
+
+    b, hq, hkv = 2, 6, 2
+    g = torch.Generator(device=DEV).manual_seed(t * 31 + cache_len + d)
+    q = torch.randn(b, t, hq, d, generator=g, device=DEV)
+    n = cache_len + t
+    kc = torch.full((b, hkv, n + 5, d), float("nan"), device=DEV)
+    vc = torch.full_like(kc, float("nan"))
+    kc[:, :, :n] = torch.randn(b, hkv, n, d, generator=g, device=DEV)
+    vc[:, :, :n] = torch.randn(b, hkv, n, d, generator=g, device=DEV)
+    out = K.attention(q, kc, vc, cache_len).view(b, t, hq, d).double()
+    kk = kc[:, :, :n].double().repeat_interleave(hq // hkv, 1)
+    vv = vc[:, :, :n].double().repeat_interleave(hq // hkv, 1)
+    s = (q.double().transpose(1, 2) @ kk.transpose(-1, -2).contiguous()) / d ** 0.5
+    mask = torch.arange(n, device=DEV)[None, :] > cache_len + torch.arange(t, device=DEV)[:, None]
+    ref = (s.masked_fill(mask, float("-inf")).softmax(-1) @ vv).transpose(1, 2)
+    assert torch.isfinite(out).all()
+    assert (out - ref).abs().max().item() <= 1e-5
+
+
+def test_prefill_attention_f32_large_scores():
+    """Scores far past the exponential's range, one key per query dominating."""
+    from minitp import kernels as K
+
+    t, d = 40, 64
+    g = torch.Generator(device=DEV).manual_seed(5)
+    q = torch.randn(1, t, 1, d, generator=g, device=DEV) * 40
+    k = torch.randn(1, 1, t, d, generator=g, device=DEV) * 40
+    v = torch.randn(1, 1, t, d, generator=g, device=DEV)
+    out = K.attention(q, k, v, 0).view(t, d)
+    s = (q[0, :, 0].double() @ k[0, 0].double().t().contiguous()) / d ** 0.5
+    s = s.masked_fill(torch.triu(torch.ones(t, t, device=DEV, dtype=torch.bool), 1), float("-inf"))
+    ref = s.softmax(-1) @ v[0, 0].double()
+    # scores of order 13,000 carry an absolute error of up to 13,000 x 2^-24 x 8
+    assert torch.isfinite(out).all()
+    assert (out.double() - ref).abs().max().item() <= 0.05
