@@ -94,6 +94,23 @@ int minitp_cast_f32_bf16(void* stream, const float* in, void* out, int64_t n);
 int minitp_linear(void* stream, int dtype, const void* x, int64_t ldx, const void* w,
                   const void* bias, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
                   int epilogue, const void* aux);
+
+/* minitp_linear with scratch for its split-K products: some shapes (few
+ * output tiles, long K) split K over blocks when `workspace` holds at least
+ * minitp_linear_workspace_bytes bytes (0: this shape does not split), fp32
+ * partials added in split order by a second kernel. A smaller or NULL
+ * workspace runs the unsplit form. The workspace needs no initial value and
+ * holds nothing after the call's kernels have run. */
+int64_t minitp_linear_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int epilogue);
+int minitp_linear_ws(void* stream, int dtype, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
+                     int64_t ldy, int64_t M, int64_t N, int64_t K, int epilogue, const void* aux, void* workspace,
+                     int64_t workspace_bytes);
+
+/* y[M, N] = silu(gate) * up of x W^T for W = [gate; up] ([2N, K]) at any
+ * row count, gate and up rounded to dtype first (mlp.py:34-38,
+ * fused.py:102-104): minitp_linear + minitp_silu_mul in one kernel. */
+int minitp_gate_up_swiglu(void* stream, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
+                          int64_t M, int64_t N, int64_t K);
 /* RMSNorm (layer.py:39-42) feeding a linear (the decoder layer's
  * input_layernorm -> qkv_proj and post_attention_layernorm -> gate_up_proj,
  * layer.py:60-67) in one pass over W: every block normalises the x rows it

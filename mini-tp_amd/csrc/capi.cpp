@@ -174,6 +174,10 @@ GemvArgs gemv_args(const void* x, int64_t ldx, const void* w, const void* bias, 
   return g;
 }
 
+// The GEMV forms finish whole SwiGLU tuples: pairs of outputs, eight on the
+// MFMA form (a narrower remainder would be left unwritten).
+bool gemv_swiglu_width(int dtype, int64_t M, int64_t N) { return N % (gemv_mfma_rows(dtype, M) ? 8 : 2) == 0; }
+
 int gemv_epilogue(int epilogue) {
   return epilogue == MINITP_EPI_RESID ? EPI_RESID : epilogue == MINITP_EPI_SWIGLU ? EPI_SWIGLU : EPI_STORE;
 }
@@ -182,10 +186,27 @@ int gemv_epilogue(int epilogue) {
 
 int minitp_linear(void* stream, int dtype, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
                   int64_t ldy, int64_t M, int64_t N, int64_t K, int epilogue, const void* aux) {
+  return minitp_linear_ws(stream, dtype, x, ldx, w, bias, y, ldy, M, N, K, epilogue, aux, nullptr, 0);
+}
+
+int64_t minitp_linear_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int epilogue) {
+  if (!dtype_ok(dtype) || M < 0 || N < 0 || K <= 0 || epilogue < MINITP_EPI_NONE || epilogue > MINITP_EPI_SWIGLU)
+    return -1;
+  if (M == 0 || N == 0 || epilogue == MINITP_EPI_SWIGLU || gemv_supported(dtype, M, K)) return 0;
+  return gemm_split_bytes(dtype, M, N, K, epilogue == MINITP_EPI_NONE);
+}
+
+int minitp_linear_ws(void* stream, int dtype, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
+                     int64_t ldy, int64_t M, int64_t N, int64_t K, int epilogue, const void* aux, void* workspace,
+                     int64_t workspace_bytes) {
   int rc = linear_checks(dtype, x, ldx, w, bias, y, ldy, M, N, K, epilogue, aux);
   if (rc || M == 0 || N == 0) return rc;
+  MINITP_CHECK_ARG(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0) && aligned16(workspace),
+                   "linear: workspace %p of %lld bytes", workspace, (long long)workspace_bytes);
   hipStream_t st = S(stream);
-  if (gemv_supported(dtype, M, K))
+  if (epilogue == MINITP_EPI_SWIGLU && gemv_entry_rows(dtype, M, K) && !gemv_swiglu_width(dtype, M, N))
+    return launch_gemm_swiglu(st, dtype, x, ldx, w, y, ldy, M, N, K);
+  if (epilogue == MINITP_EPI_SWIGLU ? gemv_entry_rows(dtype, M, K) : gemv_supported(dtype, M, K))
     return launch_gemv(st, dtype, PRO_NONE, gemv_epilogue(epilogue), gemv_args(x, ldx, w, bias, y, ldy, M, N, K, aux));
   if (epilogue == MINITP_EPI_SWIGLU) {
     if (dtype == MINITP_BF16 && bias == nullptr && aligned16(x) && aligned16(w) &&
@@ -195,7 +216,17 @@ int minitp_linear(void* stream, int dtype, const void* x, int64_t ldx, const voi
               "least 96 256 x 128 output tiles; use NONE + minitp_silu_mul");
     return MINITP_ERR_UNSUPPORTED;
   }
-  return launch_gemm(st, dtype, x, ldx, w, bias, y, ldy, M, N, K, epilogue, aux);
+  return launch_gemm(st, dtype, x, ldx, w, bias, y, ldy, M, N, K, epilogue, aux, nullptr, workspace, workspace_bytes);
+}
+
+int minitp_gate_up_swiglu(void* stream, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
+                          int64_t M, int64_t N, int64_t K) {
+  int rc = linear_checks(dtype, x, ldx, w, nullptr, y, ldy, M, N, K, MINITP_EPI_NONE, nullptr);
+  if (rc || M == 0 || N == 0) return rc;
+  hipStream_t st = S(stream);
+  if (gemv_supported(dtype, M, K) && gemv_swiglu_width(dtype, M, N))
+    return launch_gemv(st, dtype, PRO_NONE, EPI_SWIGLU, gemv_args(x, ldx, w, nullptr, y, ldy, M, N, K, nullptr));
+  return launch_gemm_swiglu(st, dtype, x, ldx, w, y, ldy, M, N, K);
 }
 
 int minitp_rmsnorm_linear(void* stream, int dtype, const void* x, int64_t ldx, const void* norm_w, float eps,
@@ -205,7 +236,7 @@ int minitp_rmsnorm_linear(void* stream, int dtype, const void* x, int64_t ldx, c
   if (rc || M == 0 || N == 0) return rc;
   MINITP_CHECK_ARG(norm_w != nullptr, "rmsnorm_linear: NULL norm weight");
   MINITP_CHECK_ARG(epilogue != MINITP_EPI_RESID || aux != x, "rmsnorm_linear: RESID aux must not alias x");
-  if (!gemv_norm_supported(dtype, M, K)) {
+  if (!gemv_entry_rows(dtype, M, K) || !gemv_norm_supported(dtype, M, K)) {
     set_error("rmsnorm_linear: M=%lld K=%lld is not a decode shape; use minitp_rmsnorm + minitp_linear",
               (long long)M, (long long)K);
     return MINITP_ERR_UNSUPPORTED;

@@ -169,19 +169,20 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const T* __restrict__ x, c
 // delta a row (NORM_ADD) or a split product's partials, their sum rounded to
 // the dtype as gemm_reduce_kernel stores it (NORM_ADD_PART). Each thread
 // reads and writes only its own elements, so out may alias delta. Rows of up
-// to 256 x KEEP pieces stay in registers between the sum of squares and the
-// scaling (no second read), the norm weights loaded before the reduction's
-// barrier. Memory-bound when rows are many (16,384 x 3,584 bf16, plain: 75 us
-// with scalar accesses and a second read, 46 us here, 5.1 TB/s), bound by its
-// load -> reduce -> store chain when they are few.
+// to KEEP pieces a thread stay in registers between the sum of squares and
+// the scaling (no second read), the norm weights loaded before the
+// reduction's barrier. Memory-bound when rows are many (16,384 x 3,584 bf16,
+// plain: 75 us with scalar accesses and a second read, 49 us here), bound by
+// its load -> reduce -> store chain when they are few.
 enum { NORM_PLAIN = 0, NORM_ADD = 1, NORM_ADD_PART = 2 };
+constexpr int NORM_THREADS = 512;  // at most; a block has one thread a piece up to there
 template <typename T, int W, int MODE>
-__global__ __launch_bounds__(256) void norm_rows_kernel(const T* xin, T* x, const T* delta, Partials dp,
+__global__ __launch_bounds__(NORM_THREADS) void norm_rows_kernel(const T* xin, T* x, const T* delta, Partials dp,
                                                         const T* __restrict__ w, T* out, int64_t hidden, float eps) {
-  __shared__ float red[4];
-  constexpr int KEEP = 4;
+  __shared__ float red[NORM_THREADS / 64];
+  constexpr int KEEP = 2;
   const int64_t base = blockIdx.x * hidden;
-  const int n = (int)(hidden / W), tid = threadIdx.x;
+  const int n = (int)(hidden / W), tid = threadIdx.x, nt = blockDim.x;
   float v[KEEP][W], wf[KEEP][W];
   float ss = 0.f;
   auto take = [&](int c, float* a) {
@@ -208,33 +209,38 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const T* xin, T* x, cons
     for (int e = 0; e < W; ++e) o[e] = mul_rn(mul_rn(a[e], r), g[e]);
     store_vec<T, W>(out + base + c * W, o);
   };
-  const bool keep = n <= 256 * KEEP;
+  const bool keep = n <= nt * KEEP;
   if (keep) {
 #pragma unroll
     for (int k = 0; k < KEEP; ++k)
-      if (tid + 256 * k < n) load_vec<T, W>(w + (tid + 256 * k) * W, wf[k]);
+      if (tid + nt * k < n) load_vec<T, W>(w + (tid + nt * k) * W, wf[k]);
 #pragma unroll
     for (int k = 0; k < KEEP; ++k)
-      if (tid + 256 * k < n) take(tid + 256 * k, v[k]);
+      if (tid + nt * k < n) take(tid + nt * k, v[k]);
   } else {
-    for (int c = tid; c < n; c += 256) take(c, v[0]);
+    for (int c = tid; c < n; c += nt) take(c, v[0]);
   }
   ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
-  const float tot = (red[0] + red[1]) + (red[2] + red[3]);
+  float tot = red[0];
+  for (int i = 1; i < nt / 64; ++i) tot += red[i];
   const float r = __fdiv_rn(1.0f, __fsqrt_rn(add_rn(__fdiv_rn(tot, (float)hidden), eps)));
   if (keep) {
 #pragma unroll
     for (int k = 0; k < KEEP; ++k)
-      if (tid + 256 * k < n) give(tid + 256 * k, v[k], wf[k], r);
+      if (tid + nt * k < n) give(tid + nt * k, v[k], wf[k], r);
   } else {
-    for (int c = tid; c < n; c += 256) {
+    for (int c = tid; c < n; c += nt) {
       load_vec<T, W>((MODE == NORM_PLAIN ? xin : x) + base + c * W, v[0]);
       load_vec<T, W>(w + c * W, wf[0]);
       give(c, v[0], wf[0], r);
     }
   }
+}
+
+inline unsigned norm_threads(int64_t pieces) {
+  return (unsigned)std::min<int64_t>(NORM_THREADS, cdiv(pieces, 64) * 64);
 }
 
 inline bool norm_vec_ok(int dtype, int64_t hidden, const void* a, const void* b, const void* c, const void* d) {
@@ -247,12 +253,12 @@ int launch_rmsnorm(hipStream_t st, int dtype, const void* x, const void* w, void
   if (rows == 0) return MINITP_OK;
   const bool vec = norm_vec_ok(dtype, hidden, x, w, out, out);
   if (dtype == MINITP_F32 && vec)
-    norm_rows_kernel<float, 4, NORM_PLAIN><<<(unsigned)rows, 256, 0, st>>>(
+    norm_rows_kernel<float, 4, NORM_PLAIN><<<(unsigned)rows, norm_threads(hidden / 4), 0, st>>>(
         (const float*)x, nullptr, nullptr, Partials{}, (const float*)w, (float*)out, hidden, eps);
   else if (dtype == MINITP_F32)
     rmsnorm_kernel<float><<<(unsigned)rows, 256, 0, st>>>((const float*)x, (const float*)w, (float*)out, hidden, eps);
   else if (vec)
-    norm_rows_kernel<bf16, 8, NORM_PLAIN><<<(unsigned)rows, 256, 0, st>>>(
+    norm_rows_kernel<bf16, 8, NORM_PLAIN><<<(unsigned)rows, norm_threads(hidden / 8), 0, st>>>(
         (const bf16*)x, nullptr, nullptr, Partials{}, (const bf16*)w, (bf16*)out, hidden, eps);
   else
     rmsnorm_kernel<bf16><<<(unsigned)rows, 256, 0, st>>>((const bf16*)x, (const bf16*)w, (bf16*)out, hidden, eps);
@@ -292,10 +298,10 @@ int launch_add_rmsnorm(hipStream_t st, int dtype, void* x, const void* delta, co
   if (rows == 0) return MINITP_OK;
   const bool vec = norm_vec_ok(dtype, hidden, x, delta, w, out);
   if (vec && dtype == MINITP_F32)
-    norm_rows_kernel<float, 4, NORM_ADD><<<(unsigned)rows, 256, 0, st>>>(
+    norm_rows_kernel<float, 4, NORM_ADD><<<(unsigned)rows, norm_threads(hidden / 4), 0, st>>>(
         nullptr, (float*)x, (const float*)delta, Partials{}, (const float*)w, (float*)out, hidden, eps);
   else if (vec)
-    norm_rows_kernel<bf16, 8, NORM_ADD><<<(unsigned)rows, 256, 0, st>>>(
+    norm_rows_kernel<bf16, 8, NORM_ADD><<<(unsigned)rows, norm_threads(hidden / 8), 0, st>>>(
         nullptr, (bf16*)x, (const bf16*)delta, Partials{}, (const bf16*)w, (bf16*)out, hidden, eps);
   else if (dtype == MINITP_F32)
     add_rmsnorm_kernel<float><<<(unsigned)rows, 256, 0, st>>>((float*)x, (const float*)delta, (const float*)w,
@@ -395,10 +401,10 @@ int launch_add_rmsnorm_partials(hipStream_t st, int dtype, void* x, const Partia
   // (4-element pieces of the partials: 0.5B rows then keep 224 of a block's
   // threads loading instead of 112)
   if (dtype == MINITP_F32)
-    norm_rows_kernel<float, 4, NORM_ADD_PART><<<(unsigned)delta.M, 256, 0, st>>>(
+    norm_rows_kernel<float, 4, NORM_ADD_PART><<<(unsigned)delta.M, norm_threads(hidden / 4), 0, st>>>(
         nullptr, (float*)x, nullptr, delta, (const float*)w, (float*)out, hidden, eps);
   else
-    norm_rows_kernel<bf16, 4, NORM_ADD_PART><<<(unsigned)delta.M, 256, 0, st>>>(
+    norm_rows_kernel<bf16, 4, NORM_ADD_PART><<<(unsigned)delta.M, norm_threads(hidden / 4), 0, st>>>(
         nullptr, (bf16*)x, nullptr, delta, (const bf16*)w, (bf16*)out, hidden, eps);
   MINITP_LAUNCH_CHECK();
   return MINITP_OK;

@@ -344,31 +344,30 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
                                                           int64_t ldy, const T* aux, int64_t M, int64_t N,
                                                           const StepState* state) {
   if (state != nullptr) y = (T*)state->args.logits;
-  const int64_t MN = M * N, stride = (int64_t)gridDim.x * blockDim.x * PER;
-  for (int64_t e0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * PER; e0 < MN; e0 += stride) {
-    float v[PER];
-    for (int s = 0; s < S; ++s) {
-      float p[PER];
-      if constexpr (PER == 4) {
-        const float4 t = *(const float4*)(part + s * MN + e0);
-        p[0] = t.x;
-        p[1] = t.y;
-        p[2] = t.z;
-        p[3] = t.w;
-      } else {
-        p[0] = part[s * MN + e0];
-      }
+  const int64_t e0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * PER;
+  if (e0 >= M * N) return;
+  // (32-bit division where it reaches: a 64-bit one costs more than the loads)
+  const int64_t row = e0 < (1LL << 31) ? (int64_t)((uint32_t)e0 / (uint32_t)N) : e0 / N, col = e0 - row * N;
+  float v[PER];
+  if constexpr (PER == 4) {
+    sum_partials<4>(Partials{part, S, M, N}, row, col, v);
+  } else {
+    v[0] = part[e0];
+    for (int s = 1; s < S; ++s) v[0] += part[s * M * N + e0];
+  }
 #pragma unroll
-      for (int u = 0; u < PER; ++u) v[u] = s == 0 ? p[u] : v[u] + p[u];
-    }
-    const int64_t row = e0 / N, col = e0 % N;
+  for (int u = 0; u < PER; ++u) {
+    if constexpr (EPI == MINITP_EPI_RESID)
+      v[u] = add_rn(load_f32<T>(aux, row * ldy + col + u), round_to<T>(v[u]));
+    else
+      v[u] += bias != nullptr ? load_f32<T>(bias, col + u) : 0.f;
+  }
+  T* o = y + row * ldy + col;
+  if (PER == 4 && ((uintptr_t)o & (4 * sizeof(T) - 1)) == 0) {
+    store_vec<T, 4>(o, v);
+  } else {
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      if constexpr (EPI == MINITP_EPI_RESID)
-        store_f32<T>(y, row * ldy + col + u, add_rn(load_f32<T>(aux, row * ldy + col + u), round_to<T>(v[u])));
-      else
-        store_f32<T>(y, row * ldy + col + u, v[u] + (bias != nullptr ? load_f32<T>(bias, col + u) : 0.f));
-    }
+    for (int u = 0; u < PER; ++u) store_f32<T>(o, u, v[u]);
   }
 }
 
@@ -403,7 +402,10 @@ struct TileCost {
 };
 constexpr TileCost TILE_COST[] = {
     {256, 128, 0.90f, 4.5f}, {128, 128, 0.60f, 3.f}, {64, 128, 0.42f, 2.f}, {64, 64, 0.25f, 0.5f}, {32, 64, 0.22f, 0.5f}};
-constexpr TileCost F32_COST[] = {{64, 64, 0.56f, 1.f}, {32, 64, 0.33f, 0.5f}};
+// fp32: one block alone on a CU leaves its MFMAs idle between stages (0.64 us
+// a stage of 64 x 64), blocks that share one fill in for each other (0.53)
+constexpr TileCost F32_COST[] = {{64, 64, 0.53f, 1.f}, {32, 64, 0.33f, 0.5f}};
+constexpr float F32_ALONE = 1.2f;
 constexpr TileCost TILE256_COST = {256, 256, 1.33f, 5.f};
 enum { KIND_XL = 0, KIND_L = 1, KIND_N = 2, KIND_S = 3, KIND_XS = 4 };
 constexpr int64_t XS_ROWS = 32, S_NT_ROWS = 64;
@@ -431,7 +433,8 @@ GemmPlan gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, bool swiglu, int6
       if (s > 1 && (s * M * N * 4 > ws_bytes || stages < s * SPLIT_MIN_STAGES || tiles * (s - 1) >= 2 * cus)) break;
       const int64_t per = cdiv(stages, s);
       if (cdiv(stages, per) != s) continue;
-      const float us = FIXED_US + (float)cdiv(tiles * s, cus) * ((float)per * c.stage_us + c.round_us) +
+      const float alone = f32 && tiles * s <= cus ? F32_ALONE : 1.f;
+      const float us = FIXED_US + (float)cdiv(tiles * s, cus) * ((float)per * c.stage_us * alone + c.round_us) +
                        (s > 1 ? split_us + (float)(s * M * N) / PARTIALS_PER_US : 0.f);
       if (best.kind < 0 || us < best.us) best = GemmPlan{kind, s, per * tk, us};
     }
@@ -480,11 +483,11 @@ template <typename T, int EPI>
 int launch_reduce(hipStream_t st, const float* ws, int64_t S, const T* bias, T* y, int64_t ldy, const T* aux,
                   int64_t M, int64_t N, const StepState* state) {
   if (N % 4 == 0 && aligned16(ws)) {
-    const int grid = (int)std::min<int64_t>(cdiv(M * N / 4, 256), 2048);
+    const unsigned grid = (unsigned)cdiv(M * N / 4, 256);
     hipLaunchKernelGGL((gemm_reduce_kernel<T, EPI, 4>), dim3(grid), dim3(256), 0, st, ws, (int)S, bias, y, ldy, aux, M,
                        N, state);
   } else {
-    const int grid = (int)std::min<int64_t>(cdiv(M * N, 256), 2048);
+    const unsigned grid = (unsigned)cdiv(M * N, 256);
     hipLaunchKernelGGL((gemm_reduce_kernel<T, EPI, 1>), dim3(grid), dim3(256), 0, st, ws, (int)S, bias, y, ldy, aux, M,
                        N, state);
   }
@@ -521,6 +524,12 @@ bool gemm_prefers_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy
   const float rounds = (float)(tiles / cus) + (rem == 0 ? 0.f : tiles > cus && 2 * rem <= cus && ws_bytes ? 0.6f : 1.f);
   const float us = FIXED_US + rounds * ((float)cdiv(K, 64) * TILE256_COST.stage_us + TILE256_COST.round_us);
   return us <= gemm_plan(MINITP_BF16, M, N, K, swiglu, swiglu ? 0 : ws_bytes, split_us).us;
+}
+
+int64_t gemm_split_bytes(int dtype, int64_t M, int64_t N, int64_t K, bool plain) {
+  if (dtype == MINITP_BF16 && plain && gemm_prefers_tile(M, N, K, K, N, false, GEMM_WS_BYTES, REDUCE_US)) return 0;
+  const GemmPlan p = gemm_plan(dtype, M, N, K, false, GEMM_WS_BYTES, REDUCE_US);
+  return p.S > 1 ? p.S * M * N * 4 : 0;
 }
 
 int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,

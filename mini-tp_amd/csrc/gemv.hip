@@ -34,6 +34,7 @@ constexpr int R = 2 * P;
 constexpr int U = 2;  // gemv_lds_kernel chunk unroll
 constexpr int MAX_GRID = 2048;
 constexpr int64_t REG_MAX_CHUNKS = 1024;
+constexpr int64_t F32_NORM_CHUNKS = 256, F32_MAX_CHUNKS = 1280;  // fp32 rows 2..4 (gemv_supported)
 // Split-K form: chunks per lane and row in one segment, and the row length
 // (in 16-byte chunks) above which single-row products take it.
 #ifndef MINITP_SPLIT_JMAX
@@ -2094,6 +2095,15 @@ int pick_k(hipStream_t st, const GemvArgs& a) {
   if constexpr (MM == 1 && PRO == PRO_NONE && (EPI == EPI_STORE || EPI == EPI_RESID || EPI == EPI_SWIGLU))
     if (use_split<T, PRO, EPI>(a)) return launch_split<T, MM, EPI>(st, a);
   if (nchunk <= 128) return launch_reg<T, MM, 1, 2, PRO, EPI>(st, a);
+  if constexpr (MM == 4 && sizeof(T) == 4) {
+    if (nchunk <= F32_NORM_CHUNKS) return launch_reg<T, MM, 2, 2, PRO, EPI>(st, a);
+  }
+  if constexpr (MM > 1 && sizeof(T) == 4 && PRO == PRO_NONE &&
+                (EPI == EPI_STORE || EPI == EPI_RESID || EPI == EPI_SWIGLU)) {
+    // (two rows a tuple: the input rows take 80 of the registers)
+    if (nchunk > (MM == 2 ? REG_MAX_CHUNKS : F32_NORM_CHUNKS))
+      return launch_reg_pp<T, MM, 4, 5, PRO, EPI, 1>(st, a);
+  }
   if constexpr (MM <= 2) {
     // up to 512 chunks: bf16 rows split K over four waves, one tuple a block
     // (at the 7B decode the 1,152 QKV and 896 o_proj tuples then spread over
@@ -2195,7 +2205,9 @@ int64_t gemv_argmax_partials(int64_t N) { return std::min<int64_t>(cdiv(cdiv(N, 
 // The register path keeps the input rows in registers (M * JMAX chunks per
 // lane): M <= 4 up to 128 chunks per row, M <= 2 up to 1024; M == 1 beyond
 // that stages the input in LDS (up to 80 KiB). Other shapes run the GEMM.
-bool gemv_supported(int dtype, int64_t M, int64_t K) {
+// The rows minitp_rmsnorm_linear and minitp_linear's SwiGLU epilogue serve
+// (the forms below reach further inside a forward and for plain products).
+bool gemv_entry_rows(int dtype, int64_t M, int64_t K) {
   const int v = dtype == MINITP_F32 ? 4 : 8;
   // bf16 rows MF_MIN_ROWS..32 run the MFMA form (K a multiple of 8, rows under 2 GiB)
   if (gemv_mfma_rows(dtype, M)) return K % v == 0 && K * 2 < (1LL << 31);
@@ -2206,11 +2218,21 @@ bool gemv_supported(int dtype, int64_t M, int64_t K) {
   return M == 1 && K * 4 <= 80 * 1024;
 }
 
+// fp32 rows 2..4 past those: up to 256 chunks on two waves a row, up to 1,280
+// (no norm prologue) on four, five chunks a lane. The 0.5B shape's decode at
+// batch 2-4 then runs the five fused kernels a layer (K = 896: 224 chunks,
+// the down projection's 4,864: 1,216) instead of seven on 32-row GEMM tiles:
+// batch 3, 777 positions, 24 layers 1,418 -> 945 us a step.
+bool gemv_supported(int dtype, int64_t M, int64_t K) {
+  if (gemv_entry_rows(dtype, M, K)) return true;
+  return dtype == MINITP_F32 && M >= 2 && M <= 4 && K % 4 == 0 && K / 4 <= F32_MAX_CHUNKS;
+}
+
 // The RMSNorm prologue holds a wave's whole K range: on the MFMA form that
 // is K <= 4 waves x 8 steps x 32.
 bool gemv_norm_supported(int dtype, int64_t M, int64_t K) {
-  if (!gemv_supported(dtype, M, K)) return false;
-  return !gemv_mfma_rows(dtype, M) || K <= 4 * 32 * MF_ONE;
+  if (gemv_entry_rows(dtype, M, K)) return !gemv_mfma_rows(dtype, M) || K <= 4 * 32 * MF_ONE;
+  return gemv_supported(dtype, M, K) && K / 4 <= F32_NORM_CHUNKS;
 }
 
 int launch_gemv(hipStream_t st, int dtype, int pro, int epi, const GemvArgs& a) {

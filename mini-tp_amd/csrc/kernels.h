@@ -111,6 +111,7 @@ int launch_gemv_part_swiglu(hipStream_t st, int dtype, const GemvArgs& a);
 int64_t gemv_argmax_partials(int64_t N);
 int launch_gemv(hipStream_t st, int dtype, int pro, int epi, const GemvArgs& a);
 bool gemv_supported(int dtype, int64_t M, int64_t K);
+bool gemv_entry_rows(int dtype, int64_t M, int64_t K);
 // bf16 rows MF_MIN_ROWS..32 run the MFMA forms (16-row operand tiles, rows
 // past M read as zeros); fewer rows and fp32 the register forms. At 3 and 4
 // rows the register forms' per-lane row budget leaves long rows (the 0.5B
@@ -158,6 +159,10 @@ int launch_gemm_partials(hipStream_t st, int dtype, const void* x, int64_t ldx, 
 // store and read them
 int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int64_t M,
                        int64_t N, int64_t K, TileTail tail = TileTail{nullptr, nullptr});
+// Workspace with which launch_gemm would split an M x N x K product over K
+// (0: it runs unsplit at any size); plain: MINITP_EPI_NONE, which the tile
+// kernel may serve.
+int64_t gemm_split_bytes(int dtype, int64_t M, int64_t N, int64_t K, bool plain);
 // Whether launch_gemm, launch_gemm_swiglu and launch_gemm_partials run a bf16
 // product on the 256 x 256 tiles (the faster choice by the measured stage
 // costs); ws_bytes: room for split partials (0: none), split_us: what a split

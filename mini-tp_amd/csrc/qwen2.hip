@@ -413,7 +413,9 @@ struct Qwen2Program {
       if ((rc = launch_gemv(st, c.dtype, PRO_NONE, EPI_RESID, d))) return rc;
     }
     // ---- final norm, LM head, greedy pick ----------------------------------------
-    if (!s.logits_all && gemv_supported(c.dtype, B, H) && !gemv_mfma_rows(c.dtype, B)) {
+    // (fp32 rows past the entry forms' keep their LM head on the GEMM: 0.5B
+    // batch 3 91 us, 147 on the register GEMV)
+    if (!s.logits_all && gemv_entry_rows(c.dtype, B, H) && !gemv_mfma_rows(c.dtype, B)) {
       GemvArgs g{};
       g.x = (const char*)w.x + (T - 1) * H * es();  // last position of each row
       g.ldx = T * H;
@@ -494,7 +496,7 @@ struct Qwen2Program {
     MINITP_CHECK_ARG(s->logits != nullptr || s->next_tok != nullptr, "step produces nothing (no logits, no next_tok)");
     // Only the fused LM-head GEMV + argmax (last position, batch <= 4) can
     // skip the logits store; the other LM-head paths always write them.
-    const bool fused_head = !s->logits_all && s->batch <= 4 && gemv_supported(c.dtype, s->batch, c.hidden);
+    const bool fused_head = !s->logits_all && s->batch <= 4 && gemv_entry_rows(c.dtype, s->batch, c.hidden);
     MINITP_CHECK_ARG(fused_head || s->logits != nullptr,
                      "logits buffer required (batch %lld, logits_all %d: the LM head stores logits before the argmax)",
                      (long long)s->batch, (int)s->logits_all);

@@ -6,6 +6,8 @@ caller passes them. Launches go to torch's current stream.
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from minitp import _native as N
@@ -144,9 +146,35 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
         ldy = n_out
     else:
         ldy = out.stride(-2) if out.dim() > 1 else n_out
-    N.check(_lib().minitp_linear(N.stream(), N.dtype_code(x.dtype), xr.data_ptr(), ldx, w.data_ptr(),
-                                 N.ptr(bias.contiguous() if bias is not None else None), out.data_ptr(), ldy, m,
-                                 n_out, w.shape[1], epilogue, N.ptr(aux)), "linear")
+    dt = N.dtype_code(x.dtype)
+    bias = bias.contiguous() if bias is not None else None
+    # (up to 32 bf16 rows and 1 fp32 row run as GEMVs, which need none)
+    need = _split_bytes(x.device, dt, m, n_out, w.shape[1], epilogue) if m > (1 if dt == N.F32 else 32) else 0
+    # (scratch of the call: from the caching allocator, on the current stream)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need > 0 else None
+    N.check(_lib().minitp_linear_ws(N.stream(), dt, xr.data_ptr(), ldx, w.data_ptr(), N.ptr(bias), out.data_ptr(), ldy,
+                                    m, n_out, w.shape[1], epilogue, N.ptr(aux), N.ptr(ws), max(need, 0)), "linear")
+    return out
+
+
+@functools.lru_cache(maxsize=4096)
+def _split_bytes(device: torch.device, dtype: int, m: int, n: int, k: int, epilogue: int) -> int:
+    """Scratch with which a product of these sizes splits over K (0: it does not)."""
+    return _lib().minitp_linear_workspace_bytes(dtype, m, n, k, epilogue)
+
+
+def gate_up_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of linear(x, w) for w = [gate; up], as ``linear`` then
+    ``silu_mul`` round them, in one kernel."""
+    N.require_gpu(x, w, what="gate_up_swiglu")
+    if x.dtype != w.dtype:
+        raise TypeError(f"gate_up_swiglu: dtype mismatch x={x.dtype} w={w.dtype}")
+    w = w.contiguous()
+    xr, m, ldx = _as_rows(x)
+    n = w.shape[0] // 2
+    out = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
+    N.check(_lib().minitp_gate_up_swiglu(N.stream(), N.dtype_code(x.dtype), xr.data_ptr(), ldx, w.data_ptr(),
+                                         out.data_ptr(), n, m, n, w.shape[1]), "gate_up_swiglu")
     return out
 
 

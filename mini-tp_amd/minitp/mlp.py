@@ -22,6 +22,9 @@ class TPQwen2MLP(nn.Module):
         self.use_fused_gateup = True  # ablation toggle (mlp.py:32)
 
     def forward(self, x):
-        y = self.gate_up_proj.project(x, fused=self.use_fused_gateup)
         n = self.intermediate_local
+        gu = self.gate_up_proj
+        if self.use_fused_gateup and gu.bias is None and 2 * gu.weight.numel() * gu.weight.element_size() < 1 << 32:
+            return self.down_proj(K.gate_up_swiglu(x, gu.weight))
+        y = gu.project(x, fused=self.use_fused_gateup)
         return self.down_proj(K.silu_mul(y[..., :n], y[..., n:]))

@@ -27,6 +27,16 @@ SHAPES = [
     (433, 3584, 1096),    # 64 x 128 and 128 x 128 tiles at 7B widths
     (700, 9728, 520),
     (2000, 3584, 384),    # 256 x 128 tiles
+    (40, 3584, 18944),    # split over K: few tiles, long K
+    (100, 896, 4864),
+    (17, 130, 4864),      # (fp32: split, ragged columns)
+    (3, 896, 904),        # (fp32: the register GEMVs of 2-4 rows, to their last chunk)
+    (4, 897, 1024),
+    (3, 70, 1032),
+    (2, 96, 4104),
+    (4, 896, 4864),
+    (2, 1153, 5120),
+    (3, 64, 5128),
 ]
 
 
@@ -57,7 +67,7 @@ def test_linear_matches_float64(m, n, k, dtype):
         assert over <= 0, (b is not None, over)
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 1152, 200), (433, 3584, 1096)])
+@pytest.mark.parametrize("m,n,k", [(65, 1152, 200), (433, 3584, 1096), (40, 1792, 9480)])
 def test_linear_resid_matches_float64(m, n, k):
     from minitp import _native as N
     from minitp import kernels as K
@@ -70,7 +80,35 @@ def test_linear_resid_matches_float64(m, n, k):
     got = K.linear(x, w, epilogue=N.EPI_RESID, aux=aux).double()
     ref = prod + aux.double()
     bar = _bound(prod, x, w, torch.bfloat16, k) + 2 * 2.0 ** -9 * ref.abs()
-    assert ((got - ref).abs() <= bar).all()
+    over = ((got - ref).abs() - bar).max().item()
+    assert over <= 0, over
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (2, 4864, 896), (5, 130, 72), (33, 77, 200), (64, 4864, 896),
+                                   (65, 96, 1000), (130, 1001, 520), (300, 4864, 264), (700, 2368, 136)])
+def test_gate_up_swiglu_matches_float64(m, n, k, dtype):
+    """Bar: the products' bars through silu(g) u (|silu'| < 1.1), plus the
+    roundings of g, u, silu(g) and the output."""
+    from minitp import _native as N
+    from minitp import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(m + 3 * n + k)
+    x = torch.randn(m, k, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(2 * n, k, generator=g, device=DEV) * 0.05).to(dtype)
+    y = x.double() @ w.double().t()
+    gate, up = y[:, :n], y[:, n:]
+    b = _bound(y, x, w, dtype, k)
+    ref = torch.nn.functional.silu(gate) * up
+    unit = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -22
+    bar = 1.1 * b[:, :n] * up.abs() + torch.nn.functional.silu(gate).abs() * b[:, n:] + 4 * unit * ref.abs() + 1e-6 * (
+        dtype == torch.bfloat16)
+    outs = [K.gate_up_swiglu(x, w)]
+    if dtype == torch.bfloat16 and m <= 32 and n % 2 == 0:  # the GEMV rows of minitp_linear, any even width
+        outs.append(K.linear(x, w, epilogue=N.EPI_SWIGLU))
+    for got in outs:
+        over = ((got.double() - ref).abs() - 1.01 * bar).max().item()
+        assert over <= 0, over
 
 
 @pytest.mark.parametrize("tokens", [33, 65, 129, 200, 321])
