@@ -900,8 +900,9 @@ __global__ __launch_bounds__(256) void prefill_attn_f32_kernel(const float* q, c
       for (int j = 0; j < E; ++j) orow[64 * hf + E * (4 * lq + e) + j] = o[hf][j][e] / l;
 }
 
-// Prefill on matrix cores (bf16): block = (b * Hq + h, PQ-query tile), wave
-// w = the 16-query strip t0 = PQ y + 16 w (all strips share each staged tile). Per 64-key tile staged in LDS (K
+// Prefill on matrix cores (bf16, head dims that are no multiple of 32: D =
+// 16): block = (b * Hq + h, PQ-query tile), wave w = the 16-query strip
+// t0 = PQ y + 16 w (all strips share each staged tile). Per 64-key tile staged in LDS (K
 // row-major, V transposed so that a V operand is 4 consecutive keys), the
 // products run transposed: S^T = K Q^T by MFMA 16x16x16 leaves lane
 // (q, r) holding keys 4q .. 4q + 3 of query r, which is exactly its B operand
@@ -936,27 +937,15 @@ __global__ __launch_bounds__(PW * 64) void prefill_attn_mfma_kernel(const bf16* 
   const bf16* vbase = vc + ((int64_t)b * s.Hkv + g) * s.S * D;
   const float sl2 = scale * 1.4426950408889634f;
 
-  // head dims that are a multiple of 32 run gfx950's 16x16x32 MFMA (8 bf16 per
-  // lane per operand: k = 8 (lane / 16) + e), 16 keeps 16x16x16 (k = 4 (lane / 16) + e)
-  constexpr bool W32 = D % 32 == 0;
-  typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+  // 16x16x16 MFMA (k = 4 (lane / 16) + e)
   short4_t qa[KS];
-  bf16x8_t qa8[W32 ? D / 32 : 1];
   {
     const int64_t t = t0 + lr;
     const bf16* qrow = q + (((int64_t)b * s.T + (t < s.T ? t : 0)) * s.Hq + h) * D;
-    if constexpr (W32) {
 #pragma unroll
-      for (int kb = 0; kb < D / 32; ++kb) {
-        const uint4 v = t < s.T ? *(const uint4*)(qrow + kb * 32 + 8 * lq) : make_uint4(0, 0, 0, 0);
-        qa8[kb] = __builtin_bit_cast(bf16x8_t, v);
-      }
-    } else {
-#pragma unroll
-      for (int kb = 0; kb < KS; ++kb) {
-        const uint2 v = t < s.T ? *(const uint2*)(qrow + kb * 16 + 4 * lq) : make_uint2(0, 0);
-        qa[kb] = __builtin_bit_cast(short4_t, v);
-      }
+    for (int kb = 0; kb < KS; ++kb) {
+      const uint2 v = t < s.T ? *(const uint2*)(qrow + kb * 16 + 4 * lq) : make_uint2(0, 0);
+      qa[kb] = __builtin_bit_cast(short4_t, v);
     }
   }
   float4_t o[KS];
@@ -1029,18 +1018,10 @@ __global__ __launch_bounds__(PW * 64) void prefill_attn_mfma_kernel(const bf16* 
     for (int kbk = 0; kbk < KB; ++kbk) {
       float4_t acc = {0.f, 0.f, 0.f, 0.f};
       const char* krow = Ks + (kbk * 16 + lr) * KROW;
-      if constexpr (W32) {
 #pragma unroll
-        for (int kb = 0; kb < D / 32; ++kb) {
-          const bf16x8_t kv = __builtin_bit_cast(bf16x8_t, *(const uint4*)(krow + (kb * 32 + 8 * lq) * 2));
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qa8[kb], acc, 0, 0, 0);
-        }
-      } else {
-#pragma unroll
-        for (int kb = 0; kb < KS; ++kb) {
-          const short4_t kv = *(const short4_t*)(krow + (kb * 16 + 4 * lq) * 2);
-          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(kv, qa[kb], acc, 0, 0, 0);
-        }
+      for (int kb = 0; kb < KS; ++kb) {
+        const short4_t kv = *(const short4_t*)(krow + (kb * 16 + 4 * lq) * 2);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(kv, qa[kb], acc, 0, 0, 0);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1072,31 +1053,13 @@ __global__ __launch_bounds__(PW * 64) void prefill_attn_mfma_kernel(const bf16* 
       }
       pk[kk] = make_uint2(pack_bf16x2(pr[0], pr[1]), pack_bf16x2(pr[2], pr[3]));
     }
-    if constexpr (W32) {
-      // one MFMA per 32 keys: k-index 8 lq + e is key 32 j + 4 lq + e (e < 4) or
-      // 32 j + 16 + 4 lq + (e - 4), the same permutation in both operands
 #pragma unroll
-      for (int j = 0; j < KB / 2; ++j) {
-        const bf16x8_t pb = __builtin_bit_cast(bf16x8_t, make_uint4(pk[2 * j].x, pk[2 * j].y, pk[2 * j + 1].x,
-                                                                    pk[2 * j + 1].y));
+    for (int kk = 0; kk < KB; ++kk) {
+      const short4_t pb = __builtin_bit_cast(short4_t, pk[kk]);
 #pragma unroll
-        for (int dn = 0; dn < KS; ++dn) {
-          const char* vrow = Vt + (dn * 16 + lr) * VROW;
-          const uint2 v0 = *(const uint2*)(vrow + (32 * j + 4 * lq) * 2);
-          const uint2 v1 = *(const uint2*)(vrow + (32 * j + 16 + 4 * lq) * 2);
-          const bf16x8_t va = __builtin_bit_cast(bf16x8_t, make_uint4(v0.x, v0.y, v1.x, v1.y));
-          o[dn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb, o[dn], 0, 0, 0);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < KB; ++kk) {
-        const short4_t pb = __builtin_bit_cast(short4_t, pk[kk]);
-#pragma unroll
-        for (int dn = 0; dn < KS; ++dn) {
-          const short4_t va = *(const short4_t*)(Vt + (dn * 16 + lr) * VROW + (kk * 16 + 4 * lq) * 2);
-          o[dn] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, pb, o[dn], 0, 0, 0);
-        }
+      for (int dn = 0; dn < KS; ++dn) {
+        const short4_t va = *(const short4_t*)(Vt + (dn * 16 + lr) * VROW + (kk * 16 + 4 * lq) * 2);
+        o[dn] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, pb, o[dn], 0, 0, 0);
       }
     }
   }
@@ -1131,38 +1094,46 @@ __device__ __forceinline__ float quad_rows_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// Long-prompt prefill on matrix cores (bf16, D % 32 == 0). Block = one
-// 128-query tile of one head; its four waves own 32 queries each, as two
-// 16-query strips that share every K and V operand read from LDS (half the
-// LDS traffic of one strip per wave). Products transposed as in
+// Prefill on matrix cores (bf16, D % 32 == 0). Block = one tile of 64 NS
+// queries of one head; its four waves (per group) own NS strips of 16 queries
+// each; two strips share every K and V operand read from LDS (half the LDS
+// traffic of one strip per wave), one gives twice the blocks. Products transposed as in
 // prefill_attn_mfma_kernel (S^T = K Q^T, O^T = V^T P^T, 16x16x32 MFMA), with
 //  * K / V tiles of 64 keys double-buffered in LDS: one barrier per tile, the
 //    next tile's global loads in flight during the current tile's math;
 //  * the causal mask applied only on tiles that cross a query of the wave,
 //    the 1/sqrt(D) scale folded into the exponent (exp2(s * c - m)), and the
-//    running-sum / output rescale skipped when no lane's maximum moved;
+//    running-sum / output rescale skipped when no lane's maximum moved (by
+//    more than a slack on two strips, where probabilities may pass 1);
 //  * query tiles dispatched last (longest) first, and the heads of one KV
 //    group kept on one XCD when the head count allows (blocks go to the
 //    eight XCDs round-robin by linear id, and each XCD has its own L2).
-template <int D>
-__global__ __launch_bounds__(256, 2) void prefill_attn_fa_kernel(const bf16* q, const bf16* kc, const bf16* vc, bf16* out,
-                                                              AttnShape s, int64_t cache_len, float scale,
-                                                              PrefillKV kv) {
+//
+// NS strips of 16 queries per wave, 64 NS per block; GROUPS groups of four
+// waves each take every GROUPS-th key tile (through LDS buffers of their own)
+// and merge at the end, in group order: too few blocks to fill the CUs then
+// still walk their keys GROUPS tiles at a time.
+template <int D, int NS, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, 2) void prefill_attn_fa_kernel(const bf16* q, const bf16* kc,
+                                                                          const bf16* vc, bf16* out, AttnShape s,
+                                                                          int64_t cache_len, float scale,
+                                                                          PrefillKV kv) {
   kv.resolve(kc, vc, cache_len);
   typedef float float4_t __attribute__((ext_vector_type(4)));
   typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-  constexpr int NS = 2;              // 16-query strips per wave
-  constexpr float RESCALE_SLACK = 8.f;
+  constexpr float RESCALE_SLACK = NS == 2 ? 8.f : 0.f;
   constexpr int PQ = 4 * 16 * NS;    // queries per block
   constexpr int KT = 64, KB = KT / 16, KS = D / 16, D32 = D / 32, PPRW = D / 8;
   constexpr int KROW = D * 2 + 16, VROW = KT * 2 + 8;
   constexpr int KBYTES = KT * KROW, STAGE = KBYTES + D * VROW;
-  __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+  __shared__ __attribute__((aligned(16))) char lds_all[GROUPS * 2 * STAGE];
   const int G = s.Hq / s.Hkv;
   int bh = blockIdx.x;
   if (gridDim.x % 8 == 0) bh = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;  // XCD c: a run of heads
   const int b = bh / s.Hq, h = bh % s.Hq, g = h / G;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;  // within the group
+  char* const lds = lds_all + group * 2 * STAGE;
   const int lr = lane % 16, lq = lane / 16;
   const int64_t qt = (int64_t)gridDim.y - 1 - blockIdx.y;
   const int64_t tw = qt * PQ + wave * 16 * NS;  // first query of this wave
@@ -1241,12 +1212,14 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_fa_kernel(const bf16* q, 
     }
   };
 
-  load_tile(0);
+  // (tiles past the last, which groups may have, read zeros and are skipped)
+  const int64_t nit = cdiv(ntiles, (int64_t)GROUPS);
+  load_tile(group * KT);
   store_tile(lds);
-  if (ntiles > 1) load_tile(KT);
+  if (nit > 1) load_tile((GROUPS + group) * KT);
   __syncthreads();
-  for (int64_t it = 0; it < ntiles; ++it) {
-    const int64_t k0 = it * KT;
+  for (int64_t it = 0; it < nit; ++it) {
+    const int64_t k0 = (it * GROUPS + group) * KT;
     const char* Ks = lds + (it & 1) * STAGE;
     const char* Vt = Ks + KBYTES;
     if (tw < s.T && k0 <= cache_len + tw + 16 * NS - 1) {  // the wave sees part of the tile
@@ -1280,7 +1253,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_fa_kernel(const bf16* q, 
 #pragma unroll
       for (int st = 0; st < NS; ++st) {
         // this lane's query: its 64 keys sit in lanes lr, lr + 16, + 32, + 48. Every
-        // query sees key 0 of tile 0, so the running maximum is finite from there on.
+        // query sees key 0 of tile 0, so the running maximum is finite from there
+        // on in group 0; a query that sees no key of another group's tiles keeps
+        // m = -inf there, and 0 stands in for it in the exponents.
         float mx = acc[st][0][0];
 #pragma unroll
         for (int kbk = 0; kbk < KB; ++kbk)
@@ -1293,7 +1268,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_fa_kernel(const bf16* q, 
         // scale (the result is the same up to rounding, fewer rescales).
         if (__builtin_amdgcn_ballot_w64(mx > m[st] + RESCALE_SLACK)) {
           const float mn = fmaxf(m[st], mx);
-          const float alpha = __builtin_amdgcn_exp2f(m[st] - mn);
+          const float alpha = GROUPS > 1 && mn == -__builtin_inff() ? 1.f : __builtin_amdgcn_exp2f(m[st] - mn);
           m[st] = mn;
           lsum[st] *= alpha;
 #pragma unroll
@@ -1301,12 +1276,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_fa_kernel(const bf16* q, 
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[st][dn][i] *= alpha;
         }
+        const float mref = GROUPS > 1 && m[st] == -__builtin_inff() ? 0.f : m[st];
 #pragma unroll
         for (int kbk = 0; kbk < KB; ++kbk) {
           float pr[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            pr[i] = __builtin_amdgcn_exp2f(fmaf(acc[st][kbk][i], sl2, -m[st]));
+            pr[i] = __builtin_amdgcn_exp2f(fmaf(acc[st][kbk][i], sl2, -mref));
             lsum[st] += pr[i];
           }
           pk[st][kbk] = make_uint2(pack_bf16x2(pr[0], pr[1]), pack_bf16x2(pr[2], pr[3]));
@@ -1333,9 +1309,42 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_fa_kernel(const bf16* q, 
         }
       }
     }
-    if (it + 1 < ntiles) store_tile(lds + ((it + 1) & 1) * STAGE);  // that buffer was last read before the previous barrier
+    if (it + 1 < nit) store_tile(lds + ((it + 1) & 1) * STAGE);  // that buffer was last read before the previous barrier
     __syncthreads();
-    if (it + 2 < ntiles) load_tile((it + 2) * KT);
+    if (it + 2 < nit) load_tile(((it + 2) * GROUPS + group) * KT);
+  }
+  if constexpr (GROUPS > 1) {
+    // (the last barrier freed every buffer) [group - 1][wave][strip][value][lane]
+    constexpr int VALS = KS * 4 + 2;
+    static_assert((GROUPS - 1) * 4 * NS * VALS * 256 <= GROUPS * 2 * STAGE, "the group exchange fits the stages");
+    float* xch = (float*)lds_all;
+    auto at = [&](int g2, int st, int v) { return (((g2 * 4 + wave) * NS + st) * VALS + v) * 64 + lane; };
+    if (group > 0) {
+#pragma unroll
+      for (int st = 0; st < NS; ++st) {
+        xch[at(group - 1, st, 0)] = m[st];
+        xch[at(group - 1, st, 1)] = lsum[st];
+#pragma unroll
+        for (int dn = 0; dn < KS; ++dn)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) xch[at(group - 1, st, 2 + dn * 4 + i)] = o[st][dn][i];
+      }
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g2 = 0; g2 < GROUPS - 1; ++g2)
+#pragma unroll
+      for (int st = 0; st < NS; ++st) {
+        const float mg = xch[at(g2, st, 0)], mn = fmaxf(m[st], mg);
+        const float a0 = __builtin_amdgcn_exp2f(m[st] - mn), a1 = mg == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(mg - mn);
+        m[st] = mn;
+        lsum[st] = lsum[st] * a0 + xch[at(g2, st, 1)] * a1;
+#pragma unroll
+        for (int dn = 0; dn < KS; ++dn)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[st][dn][i] = o[st][dn][i] * a0 + xch[at(g2, st, 2 + dn * 4 + i)] * a1;
+      }
   }
 #pragma unroll
   for (int st = 0; st < NS; ++st) {
@@ -1396,18 +1405,35 @@ int prefill_dispatch(hipStream_t st, const void* q, const void* k, const void* v
                      int64_t cache_len, const PrefillKV& kv) {
   const float scale = 1.0f / sqrtf((float)D);
   if constexpr (sizeof(T) == 2) {
-    // 128-query blocks (eight strips share each staged K / V tile) once they
-    // fill the chip; 64-query blocks for short prompts
-    if (D % 32 == 0 && (int64_t)s.B * s.Hq * cdiv(s.T, 128) >= 512)
-      hipLaunchKernelGGL((prefill_attn_fa_kernel<D % 32 == 0 ? D : 32>), dim3(s.B * s.Hq, (unsigned)cdiv(s.T, 128)),
-                         dim3(256), 0, st, (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, s, cache_len,
-                         scale, kv);
-    else if ((int64_t)s.B * s.Hq * cdiv(s.T, 128) >= 512)
+    const int64_t units = (int64_t)s.B * s.Hq;
+    if constexpr (D % 32 == 0) {
+      // 128-query blocks once they fill the chip twice (two per CU). Fewer:
+      // 64-query blocks (2 x 700 tokens, 28 heads of 128, 336 / 616 blocks: 25.5
+      // against 22.5 us; 2 x 1024, 448 / 896: 36.6 against 39.3), and while
+      // all of those are resident at once (two groups: 139 KiB of LDS at D =
+      // 128, 72 at 64) and the cache may hold long contexts, two groups of
+      // waves per block walk alternate key tiles (512 queries on 1,500
+      // cached keys, 28 heads of 128: 38.5 against 45.7 us; 1,000 queries, 14
+      // heads of 64: 13.1 against 15.1; 128 queries on nothing: 5.2 against
+      // 4.8). The choice depends on nothing but the launch's shape, so a
+      // replayed graph and a direct launch agree bit for bit.
+      auto go = [&](auto kern, int queries, int threads) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)units, (unsigned)cdiv(s.T, queries)), dim3(threads), 0, st,
+                           (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, s, cache_len, scale, kv);
+      };
+      if (units * cdiv(s.T, 128) >= 512)
+        go(prefill_attn_fa_kernel<D, 2, 1>, 128, 256);
+      else if (s.S >= 1024 && units * cdiv(s.T, 64) <= device_cus() * (D <= 64 ? 2 : 1))
+        go(prefill_attn_fa_kernel<D, 1, 2>, 64, 512);
+      else
+        go(prefill_attn_fa_kernel<D, 1, 1>, 64, 256);
+    } else if (units * cdiv(s.T, 128) >= 512) {
       hipLaunchKernelGGL((prefill_attn_mfma_kernel<D, 8>), dim3(s.B * s.Hq, (unsigned)cdiv(s.T, 128)), dim3(512), 0,
                          st, (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, s, cache_len, scale, kv);
-    else
+    } else {
       hipLaunchKernelGGL((prefill_attn_mfma_kernel<D, 4>), dim3(s.B * s.Hq, (unsigned)cdiv(s.T, 64)), dim3(256), 0,
                          st, (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, s, cache_len, scale, kv);
+    }
   } else
     hipLaunchKernelGGL((prefill_attn_f32_kernel<D>), dim3(s.B * s.Hq, (unsigned)cdiv(s.T, QT)), dim3(256), 0, st,
                        (const float*)q, (const float*)k, (const float*)v, (float*)out, s, cache_len, scale, kv);
