@@ -148,7 +148,9 @@ def require_gpu(*tensors: torch.Tensor, what: str = "op") -> None:
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream (the raw handle: building a
+    torch.cuda.Stream for it on every launch costs more than the ctypes call)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
