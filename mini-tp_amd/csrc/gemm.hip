@@ -409,7 +409,10 @@ constexpr float F32_ALONE = 1.2f;
 constexpr TileCost TILE256_COST = {256, 256, 1.33f, 5.f};
 enum { KIND_XL = 0, KIND_L = 1, KIND_N = 2, KIND_S = 3, KIND_XS = 4 };
 constexpr int64_t XS_ROWS = 32, S_NT_ROWS = 64;
-constexpr float FIXED_US = 3.3f, REDUCE_US = 3.f;
+// (REDUCE_US: the reduction launch takes 3 us, and a direct call's host as long
+// again for it and its scratch as an unsplit launch: 33 x 4608 x 3584 then
+// 33 x 3584 x 3584 and three small kernels, 58.6 us a pass split, host-bound)
+constexpr float FIXED_US = 3.3f, REDUCE_US = 12.f;
 constexpr float PARTIALS_PER_US = 1e6f;   // fp32 partials written and read back
 constexpr int64_t SPLIT_MIN_STAGES = 2;   // stages a split runs at least
 
