@@ -406,7 +406,6 @@ constexpr TileCost TILE_COST[] = {
 // a stage of 64 x 64), blocks that share one fill in for each other (0.53)
 constexpr TileCost F32_COST[] = {{64, 64, 0.53f, 1.f}, {32, 64, 0.33f, 0.5f}};
 constexpr float F32_ALONE = 1.2f;
-constexpr TileCost TILE256_COST = {256, 256, 1.33f, 5.f};
 enum { KIND_XL = 0, KIND_L = 1, KIND_N = 2, KIND_S = 3, KIND_XS = 4 };
 constexpr int64_t XS_ROWS = 32, S_NT_ROWS = 64;
 // (REDUCE_US: the reduction launch takes 3 us, and a direct call's host as long
@@ -522,10 +521,12 @@ int gemm_typed(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bia
 bool gemm_prefers_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu, int64_t ws_bytes,
                        float split_us) {
   if (!gemm_tile_supported(M, N, K, ldx, ldy, swiglu)) return false;
-  const int64_t tiles = cdiv(M, 256) * cdiv(swiglu ? 2 * N : N, 256), cus = device_cus(), rem = tiles % cus;
-  // (a last round at most half full is split over K when the caller brings the workspace)
-  const float rounds = (float)(tiles / cus) + (rem == 0 ? 0.f : tiles > cus && 2 * rem <= cus && ws_bytes ? 0.6f : 1.f);
-  const float us = FIXED_US + rounds * ((float)cdiv(K, 64) * TILE256_COST.stage_us + TILE256_COST.round_us);
+  const int64_t tiles = cdiv(M, 256) * cdiv(swiglu ? 2 * N : N, 256), cus = device_cus(), steps = cdiv(K, 64);
+  // (the last round may be split over K when the caller brings the workspace)
+  int split;
+  const float round = (float)steps * TILE_STAGE_US + TILE_ROUND_US;
+  const float last = ws_bytes ? gemm_tile_tail(tiles, steps, cus, &split) : tiles % cus ? round : 0.f;
+  const float us = FIXED_US + (float)(tiles / cus) * round + last;
   return us <= gemm_plan(MINITP_BF16, M, N, K, swiglu, swiglu ? 0 : ws_bytes, split_us).us;
 }
 

@@ -52,6 +52,7 @@ constexpr int ROWB = TK * 2;  // bytes per row per stage
 constexpr int A_BYTES = TM * ROWB, B_BYTES = TN * ROWB;
 constexpr int STAGE_BYTES = A_BYTES + B_BYTES;  // 64 KiB
 constexpr int LDS_TILE_BYTES = 2 * STAGE_BYTES;
+constexpr int TILE_SPLIT_MAX = 4;  // parts of a tile of the split last round
 constexpr int GROUP_M = 8;  // row tiles per group (4 measured the same, 16 and 32 slower)
 // waves along N and M: 4 x 4 (64 x 64 wave tiles, four waves per SIMD; the
 // default), 4 x 2 (128 x 64, two per SIMD) or 2 x 2 (128 x 128, one per SIMD)
@@ -289,32 +290,38 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_tile_kernel(const
     }
     __syncthreads();
     if (!last_blk) return;
+    // every part, this block's own too, is read back two parts x four quads
+    // of loads at a time, not load by load, each a device-scope round trip
+    // (433 x 37888 x 3584, 40 of 296 tiles split: a four-layer prompt of 433
+    // tokens 1429 -> 1414 us)
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FN; ++j) {
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          float v[4] = {0.f, 0.f, 0.f, 0.f};
-          for (int p = 0; p < tail_split; ++p) {
-            float x4[4];
-            if (p == part) {
+        for (int p0 = 0; p0 < TILE_SPLIT_MAX; p0 += 2) {
+          if (p0 >= tail_split) break;
+          u32x4 w4[2][4];
 #pragma unroll
-              for (int e = 0; e < 4; ++e) x4[e] = acc[i][j][4 * r4 + e];
-            } else {
-              const u32x4 w4 = __builtin_bit_cast(
-                  u32x4, __builtin_amdgcn_raw_buffer_load_b128(pr, poff(p, (i * FN + j) * 4 + r4), 0, 16 /* sc1 */));
-              x4[0] = __uint_as_float(w4.x);
-              x4[1] = __uint_as_float(w4.y);
-              x4[2] = __uint_as_float(w4.z);
-              x4[3] = __uint_as_float(w4.w);
-            }
+          for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = p == 0 ? x4[e] : v[e] + x4[e];
+            for (int r4 = 0; r4 < 4; ++r4)
+              w4[u][r4] = __builtin_bit_cast(
+                  u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                             pr, poff(p0 + u < tail_split ? p0 + u : p0, (i * FN + j) * 4 + r4), 0, 16 /* sc1 */));
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            if (p0 + u >= tail_split) break;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float x1 = __uint_as_float(w4[u][r4][e]);
+                acc[i][j][4 * r4 + e] = p0 + u == 0 ? x1 : acc[i][j][4 * r4 + e] + x1;
+              }
           }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][j][4 * r4 + e] = v[e];
         }
+      }
   }
 
   // epilogue: lane holds column (lane % 32) of rows 8 (r / 4) + 4 half + r % 4
@@ -357,23 +364,18 @@ template <int EPI>
 int launch_tile(hipStream_t st, const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy,
                 int64_t M, int64_t N, int64_t K, TileTail tail) {
   constexpr int WM = MINITP_TILE_WAVES_M, WN = MINITP_TILE_WAVES_N;
-  constexpr int64_t PART_BYTES = (int64_t)TM * TN * 4;  // one fp32 tile
   const void* kern = (const void*)gemm_tile_kernel<EPI, WM, WN>;
   if (const int rc = ensure_lds_limit(kern, LDS_TILE_BYTES)) return rc;
   const int tiles_m = (int)cdiv(M, TM);
   const int tiles_n = (int)cdiv(N, EPI == TILE_SWIGLU ? TN / 2 : TN);
   const int tiles = tiles_m * tiles_n;
   // One block per CU at a time (128 KiB of LDS): tiles run in rounds of
-  // `cus`. A last round at most half full is split over K into S parts
-  // (S rem <= cus blocks), so that it takes about 1/S of a round; it needs
-  // the workspace and S <= the K steps.
+  // `cus`. A last round at most half full is split over K into the number of
+  // parts that gemm_tile_tail finds worth their partials (one: none).
   const int cus = device_cus();
-  const int rem = tiles % cus, nk = (int)cdiv(K, TK);
+  const int rem = tiles % cus;
   int split = 1;
-  if (tail.part != nullptr && tail.count != nullptr && tiles >= cus && rem > 0 && 2 * rem <= cus) {
-    split = std::min(std::min(cus / rem, 4), nk);
-    if ((int64_t)rem * split * PART_BYTES > TILE_TAIL_BYTES || rem > SPLIT_MAX_TUPLES) split = 1;
-  }
+  if (tail.part != nullptr && tail.count != nullptr) (void)gemm_tile_tail(tiles, cdiv(K, TK), cus, &split);
   const int full = split > 1 ? tiles - rem : tiles;
   const int per_xcd = (full + 7) / 8;
   const int grid = 8 * per_xcd + (split > 1 ? rem * split : 0);
@@ -385,6 +387,28 @@ int launch_tile(hipStream_t st, const void* x, int64_t ldx, const void* w, const
 }
 
 }  // namespace
+
+// Microseconds of the last round of `tiles` tiles on `cus` CUs and the K
+// parts (at most cus / rest, and what the workspace holds) that make it
+// shortest. A stage of 64 takes 1.33 us and a tile's start and epilogue 5
+// (measured); a split adds its partials' store, arrival and read-back, about
+// 10 us and 4 a part.
+float gemm_tile_tail(int64_t tiles, int64_t steps, int64_t cus, int* split) {
+  const int64_t rem = tiles % cus;
+  *split = 1;
+  if (rem == 0) return 0.f;
+  float best = (float)steps * TILE_STAGE_US + TILE_ROUND_US;
+  if (tiles < cus || 2 * rem > cus || rem > SPLIT_MAX_TUPLES) return best;
+  for (int64_t s = 2; s <= TILE_SPLIT_MAX && s * rem <= cus && s <= steps; ++s) {
+    if (rem * s * (int64_t)TM * TN * 4 > TILE_TAIL_BYTES) break;
+    const float us = (float)cdiv(steps, s) * TILE_STAGE_US + TILE_ROUND_US + 10.f + 4.f * (float)s;
+    if (us < best) {
+      best = us;
+      *split = (int)s;
+    }
+  }
+  return best;
+}
 
 bool gemm_tile_supported(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu) {
   const int64_t w_rows = swiglu ? 2 * N : N;

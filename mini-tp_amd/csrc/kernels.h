@@ -175,6 +175,9 @@ bool gemm_prefers_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy
 // [M, N]. MINITP_ERR_UNSUPPORTED for shapes it does not serve (too few
 // tiles, operands past 4 GiB, unaligned rows).
 bool gemm_tile_supported(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu);
+constexpr float TILE_STAGE_US = 1.33f, TILE_ROUND_US = 5.f;  // per K stage of 64, per tile
+// the time of its last round in microseconds and the K parts that round is split into
+float gemm_tile_tail(int64_t tiles, int64_t steps, int64_t cus, int* split);
 int launch_gemm_tile(hipStream_t st, const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy,
                      int64_t M, int64_t N, int64_t K, bool swiglu, TileTail tail = TileTail{nullptr, nullptr});
 // elementwise.hip
