@@ -131,8 +131,9 @@ __global__ void rope_kv_write_kernel(const T* qkv, int64_t ld, T* q_out, T* k_ca
 
 // The same as rope_kv_write_kernel with W pairs per thread (D / 2 % W == 0):
 // vector loads of the qkv row (the caller checks its alignment) and of the
-// fp32 tables, vector stores wherever the destination allows them. One block
-// per token, so the only divisions are 32-bit ones by the pieces of a head.
+// fp32 tables, vector stores wherever the destination allows them. Blocks
+// (x, y) share token x, so the only divisions are 32-bit ones by the pieces
+// of a head.
 // PART: the projection is the split-K partial product (qp) plus the bias,
 // rounded to the dtype as gemm_reduce_kernel stores it, instead of a qkv row.
 template <typename T, int W, bool PART>
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(256) void rope_kv_writev_kernel(const T* qkv, int64
   const int64_t pos = positions[t];
   const bool pos_ok = pos >= 0 && pos < max_pos;
   const int half = D / 2, groups = half / W, heads = Hq + 2 * Hkv;
-  for (int idx = threadIdx.x; idx < heads * groups; idx += blockDim.x) {
+  for (int idx = blockIdx.y * blockDim.x + threadIdx.x; idx < heads * groups; idx += gridDim.y * blockDim.x) {
     const int head = idx / groups, i = (idx % groups) * W;
     if (halted && head >= Hq) return;
     float xa[W], xb[W], oa[W], ob[W];
@@ -270,13 +271,19 @@ int launch_rope_kv_write_partials(hipStream_t st, int dtype, const Partials& qkv
   // (four pairs a thread: 128 tokens of the 0.5B shape then load their
   // partials from 128 blocks of 192 threads; as 36 blocks of 256 threads of
   // eight pairs with 64-bit index divisions this launch took 6.5 us, now 4.4)
-  const unsigned threads = rope_threads(heads * (D / 8));
+  // Few tokens: a block per wave of pieces, so that the loads of a token's
+  // partials are in flight on several CUs (7B shape, 2 and 20 tokens: 7.0 and 8.6 us as one
+  // block a token, 4.6 and 4.8 so)
+  const int64_t pieces = heads * (D / 8), waves = cdiv(pieces, 64);
+  const bool few = B * T_ * waves <= 4 * device_cus();
+  const unsigned threads = few ? 64 : rope_threads(pieces);
+  const dim3 grid((unsigned)(B * T_), few ? (unsigned)waves : 1);
   if (dtype == MINITP_F32)
-    rope_kv_writev_kernel<float, 4, true><<<(unsigned)(B * T_), threads, 0, st>>>(
+    rope_kv_writev_kernel<float, 4, true><<<grid, threads, 0, st>>>(
         nullptr, 0, qkv, (const float*)bias, (float*)q_out, nullptr, nullptr, cos_tab, sin_tab, nullptr, max_pos, B,
         (int)T_, (int)Hq, (int)Hkv, (int)D, S, 0, nullptr, state, layer);
   else
-    rope_kv_writev_kernel<bf16, 4, true><<<(unsigned)(B * T_), threads, 0, st>>>(
+    rope_kv_writev_kernel<bf16, 4, true><<<grid, threads, 0, st>>>(
         nullptr, 0, qkv, (const bf16*)bias, (bf16*)q_out, nullptr, nullptr, cos_tab, sin_tab, nullptr, max_pos, B,
         (int)T_, (int)Hq, (int)Hkv, (int)D, S, 0, nullptr, state, layer);
   MINITP_LAUNCH_CHECK();
