@@ -467,26 +467,26 @@ __global__ __launch_bounds__(MERGE_T) void decode_merge_kernel(DecodeArgs a, int
 
 // ---------------------------------------------------------------------------
 // Grouped decode attention on MFMA (bf16, D = 64 or 128, G <= GMAX query
-// heads per KV head). The G heads of a KV group are the 16-row side of
-// v_mfma_f32_16x16x32_bf16 (rows G..15 zero): the scores of 16 key positions
-// are D / 32 MFMAs (A: lane l holds q head l % 16, dims 32 s + 8 (l / 16)
-// .. +7; B: key row p + l % 16, the same dims) and P V of 32 positions is
-// D / 16 MFMAs. P V wants each lane's 8 consecutive positions of one V
-// column and of one P row, so both pass through wave-private LDS: the V tile
-// row-major with a row stride of 2 D + 8 bytes (the four lane groups' 16-bit
-// column reads, 8 rows apart, land in different banks), P as [head][position]
-// bf16 rows of 80 bytes (one conflict-free 16-byte read per lane). Softmax
-// per head in fp32 (base 2, the 1/sqrt(D) scale folded into the exponent);
-// P is rounded to bf16 for its MFMA.
+// heads per KV head). The G heads of a KV group are the 16-column side of
+// v_mfma_f32_16x16x32_bf16 (columns G..15 zero), products transposed: S^T =
+// K Q^T for 16 key positions is D / 32 MFMAs, O^T += V^T P^T of 32 positions
+// D / 16. A lane then holds eight positions of ONE head: its maximum needs
+// two lane exchanges, its sum none until the end, and its probabilities are
+// the P^T operand as they are (the k-index of both operands permuted alike).
+// V^T wants four positions of a dim at a time: V is loaded by whole rows and
+// transposed on its way into wave-private LDS. Softmax per head in fp32 (base
+// 2, the 1/sqrt(D) scale folded into the exponent); P is rounded to bf16 for
+// its MFMA.
 // Block = NWM waves over one split's position range, 32-position tiles
 // round robin, each tile's K and V loads issued before the previous tile's
 // math. Waves merge in LDS; splits merge as in decode_attn_kernel (same
 // workspace layout and merge arithmetic), inside a forward by the unit's
 // last split block (arrival words in the step state), else by the merge
-// kernel. Measured at batch 32 (0.5B shape, context about 2,300): 4 splits
-// of 8 waves 13.3 us a layer with the in-kernel merge (10.5 + 4.8 us with
-// the merge kernel); 1, 2, 6 or 8 splits, 16 waves, or three tiles of
-// loads in flight per wave were all slower or no faster.
+// kernel. Batch 32 at 2,300 positions (0.5B shape, 38 MB a layer, HBM-bound
+// past a fixed 5 us and 2 us of split merge): 12.8 us a layer, and the step
+// 1017 -> 993 us against S = Q K^T with heads as rows (16 reductions a tile,
+// V by 16-byte columns and 16-bit LDS reads). 16 waves, 8 splits of 8 and of 4
+// waves, 16 of 4: 13.1, 12.8, 13.8, 17.5 us.
 #ifndef MINITP_DEC_MF_WAVES
 #define MINITP_DEC_MF_WAVES 8
 #endif
@@ -496,18 +496,34 @@ typedef float f32x4_a __attribute__((ext_vector_type(4)));
 
 template <int D>
 struct MfDec {
-  static constexpr int VS = 2 * D + 8;         // V tile row stride in LDS (bytes)
-  static constexpr int PS = 80;                // P row stride in LDS (bytes)
-  static constexpr int VL = D / 16;            // 16-byte V loads per lane per tile (32 rows x D)
-  static constexpr int WAVE_LDS = 32 * VS + 16 * PS;
+  static constexpr int VL = D / 16;       // 16-byte V loads per lane per tile (32 rows x D)
+  static constexpr int WAVE_LDS = D * 64;  // V tile transposed: 32 positions of each dim
+  static_assert(GMAX * D * 4 <= WAVE_LDS, "the wave's outputs fit its V stage");
 };
+
+// Maximum / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 on gfx950's permlane
+// swaps (VALU, no LDS round trip): with both operands equal, a 16-swap leaves
+// lane l's value in one result and lane l ^ 16's in the other, a 32-swap
+// likewise for l ^ 32.
+__device__ __forceinline__ float quad_rows_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float quad_rows_sum(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
 
 template <int D>
 __global__ __launch_bounds__(NWM * 64) void decode_attn_mfma_kernel(DecodeArgs a) {
   using Geo = MfDec<D>;
   constexpr int KS = D / 32;   // 32-dim steps of the scores
-  constexpr int DB = D / 16;   // 16-column blocks of the output
-  constexpr int VL = Geo::VL;
+  constexpr int DB = D / 16;   // 16-row blocks of the output
+  constexpr int VL = Geo::VL, CH = D / 8, PGS = 64 / CH;  // 16-byte columns of a V row, position quads per load
   constexpr uint32_t OOB = 0xffffffffu;
   extern __shared__ __attribute__((aligned(16))) char lds[];  // NWM * Geo::WAVE_LDS
   __shared__ float pm[NWM][GMAX], pl[NWM][GMAX];
@@ -524,7 +540,6 @@ __global__ __launch_bounds__(NWM * 64) void decode_attn_mfma_kernel(DecodeArgs a
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, q4 = lane >> 4;
   char* vs = lds + w * Geo::WAVE_LDS;
-  char* ps = vs + 32 * Geo::VS;
 
   const int64_t tiles = cdiv(ctx, (int64_t)32);
   const int64_t span = cdiv(tiles, (int64_t)nsplit);
@@ -535,7 +550,7 @@ __global__ __launch_bounds__(NWM * 64) void decode_attn_mfma_kernel(DecodeArgs a
   const uint32_t kv_bytes = (uint32_t)(ctx * D * 2);  // rows past the context read zeros
   const __amdgpu_buffer_rsrc_t kr = span_rsrc(kc, kv_bytes), vr = span_rsrc(vc, kv_bytes);
 
-  // q heads of the group as the A operand (rows G..15 zero)
+  // q heads of the group as the B operand (columns G..15 zero)
   bf16x8_a qa[KS];
   {
     const bf16* qp = (const bf16*)a.q + ((int64_t)b * s.Hq + (int64_t)g * G) * D;
@@ -545,12 +560,14 @@ __global__ __launch_bounds__(NWM * 64) void decode_attn_mfma_kernel(DecodeArgs a
       qa[k] = __builtin_bit_cast(bf16x8_a, attn_load16(qr, n16 < G ? (uint32_t)((n16 * D + 32 * k + 8 * q4) * 2) : OOB));
   }
 
-  // loads of one tile: K as B operands (two 16-position halves x KS steps),
-  // V rows for the LDS stage (lane l: row l % 32, dims (l / 32) D / 2 ..)
+  // loads of one tile: K as A operands (two 16-position halves x KS steps);
+  // V by whole rows: lane l takes column l % CH of positions 4 (l / CH) + u
+  // (+ 4 PGS a load quad)
   struct Tile {
     uint4 k[2][KS];
     uint4 v[VL];
   };
+  const int vch = lane % CH, vpg = lane / CH;
   auto issue = [&](Tile& tl, int64_t t) {
     const bool live = t < t_end;
     const int64_t p0 = t * 32;
@@ -561,104 +578,118 @@ __global__ __launch_bounds__(NWM * 64) void decode_attn_mfma_kernel(DecodeArgs a
         tl.k[h][k] = attn_load16(kr, live ? (uint32_t)(((p0 + 16 * h + n16) * D + 32 * k + 8 * q4) * 2) : OOB);
 #pragma unroll
     for (int i = 0; i < VL; ++i)
-      tl.v[i] = attn_load16(vr, live ? (uint32_t)(((p0 + (lane & 31)) * D + (lane >> 5) * (D / 2) + 8 * i) * 2) : OOB);
+      tl.v[i] = attn_load16(
+          vr, live ? (uint32_t)(((p0 + 4 * (vpg + i / 4 * PGS) + i % 4) * D + 8 * vch) * 2) : OOB);
+  };
+  // LDS byte of the four positions 4 pg .. + 3 of dim r: two dims share 128
+  // bytes, their 16 quads permuted so that both the writes (16 lanes: columns
+  // of one or two quads) and the reads (16 dims of one quad) reach every bank
+  auto vt_at = [](int r, int pg) {
+    const int c = r >> 3;
+    return (r >> 1) * 128 + (((pg ^ c ^ (r & 6)) & 7) << 4) + (((r ^ pg ^ (c >> 3)) & 1) << 3);
   };
 
   const float sl2 = a.scale * 1.4426950408889634f;  // scores to base-2 exponent units
-  float m[4], l[4];
-  f32x4_a o[DB];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m[r] = -__builtin_inff();
-    l[r] = 0.f;
-  }
+  float m = -__builtin_inff(), l = 0.f;  // head l % 16: base-2 maximum, this lane's part of the sum
+  f32x4_a o[DB];                         // dims 16 c + 4 (l / 16) + r of the head
 #pragma unroll
   for (int c = 0; c < DB; ++c) o[c] = f32x4_a{0.f, 0.f, 0.f, 0.f};
 
-  Tile cur, nxt;
-  int64_t t = t_begin + w;
-  issue(cur, t);
-  for (; t < t_end; t += NWM) {
-    issue(nxt, t + NWM);
-    // V tile -> LDS, row-major (two 8-byte writes per 16-byte piece)
+  auto math = [&](const Tile& tl, int64_t t) {
+    // V tile -> LDS, transposed (8-byte writes: four positions of one dim)
 #pragma unroll
-    for (int i = 0; i < VL; ++i) {
-      char* dst = vs + (lane & 31) * Geo::VS + ((lane >> 5) * (D / 2) + 8 * i) * 2;
-      *(uint2*)dst = make_uint2(cur.v[i].x, cur.v[i].y);
-      *(uint2*)(dst + 8) = make_uint2(cur.v[i].z, cur.v[i].w);
-    }
-    // scores: lane l holds head 4 (l / 16) + r, position p0 + 16 h + l % 16
+    for (int i = 0; i < VL / 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        auto word = [&](int u) {
+          const uint4& x = tl.v[4 * i + u];
+          return e < 2 ? x.x : e < 4 ? x.y : e < 6 ? x.z : x.w;
+        };
+        constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;  // low / high halves of two words
+        const uint32_t sel = e & 1 ? HI : LO;
+        *(uint2*)(vs + vt_at(8 * vch + e, vpg + i * PGS)) =
+            make_uint2(__builtin_amdgcn_perm(word(1), word(0), sel), __builtin_amdgcn_perm(word(3), word(2), sel));
+      }
+    // scores: lane l holds head l % 16, positions p0 + 16 h + 4 (l / 16) + r
     f32x4_a sc[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       sc[h] = f32x4_a{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < KS; ++k)
-        sc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[k], __builtin_bit_cast(bf16x8_a, cur.k[h][k]), sc[h], 0, 0, 0);
+        sc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_a, tl.k[h][k]), qa[k], sc[h], 0, 0, 0);
     }
-    const int64_t p0 = t * 32;
-    float pv[2][4];
+    const int left = (int)std::min<int64_t>(ctx - t * 32, 32);  // positions of the tile
+    if (left < 32) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float x0 = p0 + n16 < ctx ? sc[0][r] * sl2 : -__builtin_inff();
-      float x1 = p0 + 16 + n16 < ctx ? sc[1][r] * sl2 : -__builtin_inff();
-      float mx = fmaxf(x0, x1);
-      mx = fmaxf(mx, flip_low<1>(mx));
-      mx = fmaxf(mx, flip_low<2>(mx));
-      mx = fmaxf(mx, flip_low<4>(mx));
-      mx = fmaxf(mx, flip_low<8>(mx));
-      const float mn = fmaxf(m[r], mx);  // finite: the tile's first position is valid
-      const float alpha = __builtin_amdgcn_exp2f(m[r] - mn);
-      const float e0 = __builtin_amdgcn_exp2f(x0 - mn), e1 = __builtin_amdgcn_exp2f(x1 - mn);
-      float sum = e0 + e1;
-      sum += flip_low<1>(sum);
-      sum += flip_low<2>(sum);
-      sum += flip_low<4>(sum);
-      sum += flip_low<8>(sum);
-      l[r] = fmaf(l[r], alpha, sum);
-      m[r] = mn;
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int c = 0; c < DB; ++c) o[c][r] *= alpha;
-      pv[0][r] = e0;
-      pv[1][r] = e1;
+        for (int r = 0; r < 4; ++r)
+          if (16 * h + 4 * q4 + r >= left) sc[h][r] = -__builtin_inff();
     }
-    // P -> LDS as [head][position] bf16
+    float mx = sc[0][0];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        *(uint16_t*)(ps + (4 * q4 + r) * Geo::PS + (16 * h + n16) * 2) = f32_to_bf16(pv[h][r]);
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[h][r]);
+    mx = quad_rows_max(mx) * sl2;
+    if (__builtin_amdgcn_ballot_w64(mx > m)) {
+      const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int c = 0; c < DB; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[c][r] *= alpha;
+    }
+    uint2 pk[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float pr[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pr[r] = __builtin_amdgcn_exp2f(fmaf(sc[h][r], sl2, -m));
+        l += pr[r];
+      }
+      pk[h] = make_uint2(pack_bf16x2(pr[0], pr[1]), pack_bf16x2(pr[2], pr[3]));
+    }
     wave_lds_sync();
-    // P V: A = P (head l % 16, positions 8 (l / 16) .. +7), B = V column
-    // block c (positions 8 (l / 16) .. +7 of column 16 c + l % 16)
-    const bf16x8_a pa = __builtin_bit_cast(bf16x8_a, *(const uint4*)(ps + n16 * Geo::PS + 16 * q4));
+    // O^T += V^T P^T (k-index 8 (l / 16) + e: position 4 (l / 16) + e, from
+    // e = 4 on 16 + 4 (l / 16) + e - 4, in both operands)
+    const bf16x8_a pb = __builtin_bit_cast(bf16x8_a, make_uint4(pk[0].x, pk[0].y, pk[1].x, pk[1].y));
 #pragma unroll
     for (int c = 0; c < DB; ++c) {
-      uint32_t vw[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const char* src = vs + (8 * q4 + 2 * e) * Geo::VS + (16 * c + n16) * 2;
-        vw[e] = (uint32_t)*(const uint16_t*)src | ((uint32_t)*(const uint16_t*)(src + Geo::VS) << 16);
-      }
-      o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, __builtin_bit_cast(bf16x8_a, make_uint4(vw[0], vw[1], vw[2], vw[3])),
-                                                    o[c], 0, 0, 0);
+      const uint2 v0 = *(const uint2*)(vs + vt_at(16 * c + n16, q4));
+      const uint2 v1 = *(const uint2*)(vs + vt_at(16 * c + n16, 4 + q4));
+      o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_a, make_uint4(v0.x, v0.y, v1.x, v1.y)),
+                                                     pb, o[c], 0, 0, 0);
     }
     wave_lds_sync();  // this tile's LDS reads done before the next tile's writes
-    cur = nxt;
+  };
+  {
+    Tile ta, tb;
+    int64_t t = t_begin + w;
+    issue(ta, t);
+    while (t < t_end) {
+      issue(tb, t + NWM);
+      math(ta, t);
+      t += NWM;
+      if (t >= t_end) break;
+      issue(ta, t + NWM);
+      math(tb, t);
+      t += NWM;
+    }
   }
 
   // ---- the waves' states -> LDS (the V stage is free now) -------------------
   float* po = (float*)vs;  // [GMAX][D] of this wave
+  l = quad_rows_sum(l);
+  if (n16 < G) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int h = 4 * q4 + r;
-    if (h < G) {
-#pragma unroll
-      for (int c = 0; c < DB; ++c) po[h * D + 16 * c + n16] = o[c][r];
-      if (n16 == 0) {
-        pm[w][h] = m[r];
-        pl[w][h] = l[r];
-      }
+    for (int c = 0; c < DB; ++c) *(float4*)(po + n16 * D + 16 * c + 4 * q4) = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
+    if (q4 == 0) {
+      pm[w][n16] = m;
+      pl[w][n16] = l;
     }
   }
   __syncthreads();
@@ -1077,23 +1108,6 @@ __global__ __launch_bounds__(PW * 64) void prefill_attn_mfma_kernel(const bf16* 
         make_uint2(pack_bf16x2(o[dn][0] / l, o[dn][1] / l), pack_bf16x2(o[dn][2] / l, o[dn][3] / l));
 }
 
-// Maximum / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 on gfx950's permlane
-// swaps (VALU, no LDS round trip): with both operands equal, a 16-swap leaves
-// lane l's value in one result and lane l ^ 16's in the other, a 32-swap
-// likewise for l ^ 32.
-__device__ __forceinline__ float quad_rows_max(float v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float quad_rows_sum(float v) {
-  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // Prefill on matrix cores (bf16, D % 32 == 0). Block = one tile of 64 NS
 // queries of one head; its four waves (per group) own NS strips of 16 queries
 // each; two strips share every K and V operand read from LDS (half the LDS
@@ -1464,8 +1478,11 @@ int prefill_by_d(hipStream_t st, const void* q, const void* k, const void* v, vo
 // two chunks per wave, up to about four blocks per CU: at batch 32 x 2,300
 // positions (64 units, 40 chunks) that is 3 splits instead of 2, 3.8 % more
 // tokens per second; one chunk per wave (5 splits) measured 8 % fewer.
-// Splits of the MFMA form: about 2 blocks per CU, each wave at least two
-// 32-position tiles.
+// Splits of the MFMA form: at most one block per CU, each wave at least two
+// 32-position tiles. A few blocks more than CUs make a second round at D =
+// 128, where a block's registers fill a CU (batch 12 at 3,000 positions, 48
+// units: 6 splits 26.9 us a layer, 5 splits 18.6); a split that gives a wave
+// one tile costs more in the merge (batch 16 at 500: 6.2 us, 2 splits 8.0).
 #ifndef MINITP_DEC_MF_BLOCKS
 #define MINITP_DEC_MF_BLOCKS 256
 #endif
@@ -1475,7 +1492,7 @@ int prefill_by_d(hipStream_t st, const void* q, const void* k, const void* v, vo
 int64_t decode_mfma_nsplit(int64_t units, int64_t ctx) {
   const int64_t tiles = cdiv(std::max<int64_t>(ctx, 1), 32);
   const int64_t by_tiles = std::max<int64_t>(1, tiles / (MINITP_DEC_MF_TILES * NWM));
-  return std::max<int64_t>(1, std::min<int64_t>(cdiv(MINITP_DEC_MF_BLOCKS, std::max<int64_t>(units, 1)), by_tiles));
+  return std::max<int64_t>(1, std::min<int64_t>(MINITP_DEC_MF_BLOCKS / std::max<int64_t>(units, 1), by_tiles));
 }
 
 // The MFMA form serves bf16 groups of 2..GMAX heads at D = 64 / 128 from 16

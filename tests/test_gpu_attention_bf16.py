@@ -36,3 +36,25 @@ def test_prefill_attention_bf16_matches_float64(t, cache_len, rows, d, hq, hkv):
     ref = (s.masked_fill(mask, float("-inf")).softmax(-1) @ vv).transpose(1, 2)
     assert torch.isfinite(out).all()
     assert (out - ref).abs().max().item() <= 3e-2
+
+
+@pytest.mark.parametrize("ctx", [1, 33, 511, 1100, 2600])
+@pytest.mark.parametrize("b,hq,hkv,d", [(12, 28, 4, 128), (100, 14, 2, 64), (129, 4, 2, 128), (17, 16, 2, 64)])
+def test_batched_decode_attention_bf16_split_counts(ctx, b, hq, hkv, d):
+    """The grouped decode form at unit counts that do not divide the CUs (one
+    to five splits, the last one shorter or empty), groups of 2, 7 and 8. The
+    bar adds the output's rounding and P's, each 2^-8 of what it rounds."""
+    from minitp import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(ctx + b)
+    q = torch.randn(b, 1, hq, d, generator=g, device=DEV).bfloat16()
+    kc = torch.full((b, hkv, ctx + 3, d), float("nan"), device=DEV, dtype=torch.bfloat16)
+    vc = torch.full_like(kc, float("nan"))
+    kc[:, :, :ctx] = torch.randn(b, hkv, ctx, d, generator=g, device=DEV).bfloat16()
+    vc[:, :, :ctx] = torch.randn(b, hkv, ctx, d, generator=g, device=DEV).bfloat16()
+    out = K.attention(q, kc, vc, ctx - 1).view(b, 1, hq, d).double().transpose(1, 2)
+    kk, vv = (x[:, :, :ctx].double().repeat_interleave(hq // hkv, 1) for x in (kc, vc))
+    p = ((q.double().transpose(1, 2) @ kk.transpose(-1, -2).contiguous()) / d ** 0.5).softmax(-1)
+    ref, ref_abs = p @ vv, p @ vv.abs()
+    assert torch.isfinite(out).all()
+    assert ((out - ref).abs() <= (ref.abs() + ref_abs) * 2 ** -8 + 1e-6).all()
