@@ -337,6 +337,163 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
   }
 }
 
+// The same products as gemm_kernel without a K split or wave groups, for many
+// tiles of few stages: a block walks its share of tiles and the ring of stages
+// runs on across them, so that a tile's epilogue and the next one's first
+// loads overlap (gemm_kernel drains its ring and refills it for every tile:
+// 0.5B LM head of 194 rows 107 us, 5 tiles of 14 stages a block; 97 so, bound
+// by the stages' MFMAs and LDS reads at two waves a SIMD and a last round two
+// thirds full). Loads past the one being waited for include the epilogue's
+// stores: the counted wait is then longer than needed, never shorter, since
+// vector memory operations retire in issue order. Non-temporal weight loads:
+// 4 % slower.
+template <typename T, typename C>
+__global__ __launch_bounds__(C::THREADS) void gemm_stream_kernel(const T* __restrict__ x, int64_t ldx,
+                                                                 const T* __restrict__ w, const T* __restrict__ bias,
+                                                                 T* y, int64_t ldy, int M, int N, int K, int tiles_m,
+                                                                 int tiles_n, int items, const StepState* state) {
+  constexpr int BM = C::BM, BN = C::BN, STAGES = C::STAGES, PPW = C::PPW;
+  constexpr int FM = C::FM, WN = C::WN, ROWB = C::ROWB, ES = (int)sizeof(T), V = 16 / ES, TK = KCH * V;
+  static_assert(C::WK == 1, "a wave tile is one wave's");
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  if (state != nullptr) y = (T*)state->args.logits;
+  // XCD b % 8 takes a contiguous range of tiles, its blocks every stride-th of it
+  const int per_xcd = (items + 7) >> 3, stride = gridDim.x >> 3;
+  const int first = (blockIdx.x & 7) * per_xcd, mine = min(per_xcd, items - first);
+  int li = blockIdx.x >> 3;
+  if (li >= mine) return;
+
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN % C::WM, wn = wave % WN;
+  auto place = [&](int t, int& m0, int& n0) {
+    const int group = t / (8 * tiles_n), first_m = group * 8, gsz = min(tiles_m - first_m, 8);
+    const int in_group = t - group * 8 * tiles_n;
+    m0 = (first_m + in_group % gsz) * BM;
+    n0 = in_group / gsz * BN;
+  };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  constexpr int A_BYTES = BM * ROWB;
+  auto swz = [](int r) { return (r >> 1) & 7; };
+
+  // ---- the load side: the tile whose stages are being issued -----------------
+  u32x4 xq, wq;
+  uint32_t voff[PPW];
+  int kc[PPW];
+  auto setup = [&](int t) {
+    int m0, n0;
+    place(t, m0, n0);
+    const int x_rows = min(M - m0, BM);
+    const int64_t w_rows = min(N - n0, BN);
+    const uint32_t x_bytes = (uint32_t)(((int64_t)(x_rows - 1) * ldx + K) * ES);
+    const uint32_t w_bytes = (uint32_t)(w_rows * K * ES);
+    xq = rsrc_span(x + (int64_t)m0 * ldx, x_bytes);
+    wq = rsrc_span(w + (int64_t)n0 * K, w_bytes);
+    const uint32_t x_pad = x_bytes <= ROW_OOB ? ROW_OOB : (uint32_t)((int64_t)(x_rows - 1) * ldx * ES);
+    const uint32_t w_pad = w_bytes <= ROW_OOB ? ROW_OOB : 0u;
+#pragma unroll
+    for (int j = 0; j < PPW; ++j) {
+      const int p = wave * PPW + j;
+      const bool is_w = p >= BM / C::PIECE_ROWS;
+      const int r = C::PIECE_ROWS * (is_w ? p - BM / C::PIECE_ROWS : p) + lane / KCH;
+      const int c = (lane % KCH) ^ swz(r);
+      kc[j] = c * V;
+      if (!is_w) {
+        voff[j] = r < x_rows ? (uint32_t)(((int64_t)r * ldx + c * V) * ES) : x_pad;
+      } else {
+        voff[j] = n0 + r < N ? (uint32_t)(((int64_t)r * K + c * V) * ES) : w_pad;
+      }
+    }
+  };
+  const int nk = (K + TK - 1) / TK;
+  int ls = 0, lt = li;  // next stage to issue and its tile
+  // (past the last tile the loads read zeros: every step issues the same
+  // number, so that the waits can count them)
+  auto issue = [&](int stage) {
+    if (ls == nk && lt < mine) {
+      lt += stride;
+      ls = 0;
+      if (lt < mine) setup(first + lt);
+    }
+    const int k0 = lt < mine ? ls * TK : K;
+    const uint32_t base = lds0 + stage * C::STAGE_BYTES + wave * PPW * 1024;
+#pragma unroll
+    for (int j = 0; j < PPW; ++j)
+      load16_lds<C::NT>(wave * PPW + j >= BM / C::PIECE_ROWS ? wq : xq, k0 + kc[j] < K ? voff[j] + (uint32_t)(k0 * ES) : K_OOB,
+                 (uint32_t)__builtin_amdgcn_readfirstlane(base + j * 1024));
+    ++ls;
+  };
+
+  const int ar = wm * (32 * FM) + (lane & 31), br = wn * 64 + (lane & 31);
+  const int a_off = ar * ROWB, b_off = A_BYTES + br * ROWB, a_swz = swz(ar), b_swz = swz(br);
+  constexpr int KS = KCH / 2;
+  setup(first + lt);
+#pragma unroll 1
+  for (int s = 0; s < STAGES - 1; ++s) issue(s);
+  int rd = 0, wr_stage = STAGES - 1;
+  for (; li < mine; li += stride) {
+    f32x16 acc[FM][2];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int kt = 0; kt < nk; ++kt) {
+      stage_barrier<(STAGES - 2) * PPW>();
+      issue(wr_stage);
+      const char* st = lds + rd * C::STAGE_BYTES;
+      u32x4 av[2][FM], bv[2][2];
+      auto fetch = [&](int s, u32x4(&a)[FM], u32x4(&b)[2]) {
+        const int c = s * 2 + half;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) a[i] = *(const u32x4*)(st + a_off + i * 32 * ROWB + ((c ^ a_swz) << 4));
+#pragma unroll
+        for (int j = 0; j < 2; ++j) b[j] = *(const u32x4*)(st + b_off + j * 32 * ROWB + ((c ^ b_swz) << 4));
+      };
+      fetch(0, av[0], bv[0]);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (s + 1 < KS) fetch(s + 1, av[(s + 1) & 1], bv[(s + 1) & 1]);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma_step<T>(bv[s & 1][j], av[s & 1][i], acc[i][j]);
+      }
+      rd = rd + 1 == STAGES ? 0 : rd + 1;
+      wr_stage = wr_stage + 1 == STAGES ? 0 : wr_stage + 1;
+    }
+    int m0, n0;
+    place(first + li, m0, n0);
+    const bool quads = N % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & (4 * sizeof(T) - 1)) == 0;
+    const int col0 = n0 + wn * 64 + 4 * half;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int64_t row = m0 + wm * (32 * FM) + i * 32 + (lane & 31);
+      if (row >= M) continue;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int col = col0 + j * 32 + 8 * q;
+          if (col >= N) continue;
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[e] = acc[i][j][4 * q + e] + (bias != nullptr && col + e < N ? load_f32<T>(bias, col + e) : 0.f);
+          T* o = y + row * ldy + col;
+          if (quads) {
+            store_vec<T, 4>(o, v);
+          } else {
+#pragma unroll 1
+            for (int e = 0; e < 4 && col + e < N; ++e) store_f32<T>(o, e, e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3]);
+          }
+        }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the last zero stages land before the LDS is given back)
+}
+
 // y = epilogue(sum over the S splits of part[s][M][N]), splits added in order;
 // PER (4 when N is a multiple of 4) consecutive elements of a row per thread.
 template <typename T, int EPI, int PER>
@@ -389,6 +546,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restric
 // 204; 30 x 151936 x 896: 114 us against 158 on 64 x 64).
 using TileXL = Tile<256, 128, 2, 3>;
 using TileL = Tile<128, 128, 2, 4>;
+using TileStream = Tile<256, 128, 1, 3>;
 using TileN = Tile<64, 128, 4, 4>;
 using TileS = Tile<64, 64, 4, 4>;
 using TileSnt = Tile<64, 64, 4, 4, true>;
@@ -464,6 +622,28 @@ int launch_cfg(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bia
   return MINITP_OK;
 }
 
+// Two rounds of 256 x 128 tiles and more, of at most 32 stages: the running
+// ring saves about 4.5 us a tile and its eight waves lose 0.12 a stage against
+// gemm_kernel's sixteen (N = 151,936, K = 896, 14 stages: 150 rows 99.5 -> 86.5
+// us, 194 rows 107 -> 97, 250 rows 119.6 -> 105; N = 152,064, K = 3,584, 56
+// stages, 200 rows: 307 against 318).
+inline bool stream_pays(int64_t M, int64_t N, int64_t K) {
+  return cdiv(M, 256) * cdiv(N, 128) >= 2 * (int64_t)device_cus() && K <= 2048;
+}
+
+template <typename T, typename C>
+int launch_stream(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
+                  int64_t N, int64_t K, const StepState* state) {
+  if (const int rc = ensure_lds_limit((const void*)gemm_stream_kernel<T, C>, C::RING_BYTES)) return rc;
+  const int tiles_m = (int)cdiv(M, C::BM), tiles_n = (int)cdiv(N, C::BN);
+  const int64_t items = (int64_t)tiles_m * tiles_n;
+  const dim3 grid((unsigned)(8 * cdiv(std::min<int64_t>(items, device_cus()), 8)));
+  hipLaunchKernelGGL((gemm_stream_kernel<T, C>), grid, dim3(C::THREADS), C::RING_BYTES, st, x, ldx, w, bias, y, ldy,
+                     (int)M, (int)N, (int)K, tiles_m, tiles_n, (int)items, state);
+  MINITP_LAUNCH_CHECK();
+  return MINITP_OK;
+}
+
 template <typename T, int OUT>
 int launch_plan(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
                 int64_t N, int64_t K, const T* aux, const StepState* state, float* part, const GemmPlan& p) {
@@ -471,6 +651,9 @@ int launch_plan(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bi
     return launch_cfg<T, decltype(cfg), OUT>(st, x, ldx, w, bias, y, ldy, M, N, K, aux, state, part, p);
   };
   if constexpr (sizeof(T) == 2) {
+    if constexpr (OUT == MINITP_EPI_NONE)
+      if (p.kind == KIND_XL && p.S == 1 && stream_pays(M, N, K))
+        return launch_stream<T, TileStream>(st, x, ldx, w, bias, y, ldy, M, N, K, state);
     if (p.kind == KIND_XL) return go(TileXL{});
     if (p.kind == KIND_L) return go(TileL{});
     if (p.kind == KIND_N) return go(TileN{});

@@ -132,3 +132,11 @@ def test_swiglu_forms_agree_with_the_module(tokens):
     model.use_rotary_cache = True
     for a, b in zip(*out):
         torch.testing.assert_close(a, b, atol=0.05, rtol=0.02)
+
+
+@pytest.mark.parametrize("m,n,k", [(250, 65700, 200), (194, 65665, 264), (255, 98432, 896), (300, 65664, 72)])
+def test_linear_of_many_tiles_matches_float64(m, n, k):
+    """Products whose blocks walk several tiles on one running ring of stages:
+    last row and column tiles not full, columns not in fours, a last round
+    that some blocks sit out; the bar of the plain products."""
+    test_linear_matches_float64(m, n, k, torch.bfloat16)
