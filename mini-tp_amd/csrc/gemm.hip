@@ -68,13 +68,15 @@ constexpr uint32_t ROW_OOB = 0xF0000000u, K_OOB = 0xFFFFFFF0u;
 // 16 bytes per lane from the resource at voff straight into LDS: lane l's
 // bytes land at lds_addr + 16 l (wave-uniform, in m0). NT: non-temporal. asm, so that the
 // compiler does not wait for these loads at every LDS read: the kernel waits
-// for them itself, by count.
+// for them itself, by count. The s_nop is the wait state that gfx9 hardware
+// asks for between the scalar write of m0 and a load to LDS (the compiler
+// inserts it for its own loads, but does not look into asm).
 template <bool NT>
 __device__ __forceinline__ void load16_lds(u32x4 r, uint32_t voff, uint32_t lds_addr) {
   if constexpr (NT)
-    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen nt lds" ::"v"(voff), "s"(r), "{m0}"(lds_addr) : "memory");
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen nt lds" ::"v"(voff), "s"(r), "{m0}"(lds_addr) : "memory");
   else
-    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(lds_addr) : "memory");
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(lds_addr) : "memory");
 }
 
 __device__ __forceinline__ u32x4 rsrc_span(const void* base, uint32_t bytes) {

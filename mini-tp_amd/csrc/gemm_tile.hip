@@ -84,9 +84,12 @@ __device__ __forceinline__ u32x4 rsrc_words(const void* base, uint32_t bytes) {
 // m0); an offset past the range writes zeros. Issued as asm so that the
 // compiler does not make every later LDS read wait for these loads: the
 // kernel waits for them itself (vmcnt(0) before the barrier that publishes
-// the stage).
+// the stage). A load to LDS may not follow the scalar write of m0 directly
+// (one wait state on gfx9 hardware); the compiler, which inserts that state for its own
+// loads, does not look into asm, so it is part of the asm.
 __device__ __forceinline__ void dma16(u32x4 r, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
-  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(lds_addr) : "memory");
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(lds_addr)
+               : "memory");
 }
 
 // byte offset of chunk c of row r inside an operand's stage buffer. The LDS
