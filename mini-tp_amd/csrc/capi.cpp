@@ -174,10 +174,6 @@ GemvArgs gemv_args(const void* x, int64_t ldx, const void* w, const void* bias, 
   return g;
 }
 
-// The GEMV forms finish whole SwiGLU tuples: pairs of outputs, eight on the
-// MFMA form (a narrower remainder would be left unwritten).
-bool gemv_swiglu_width(int dtype, int64_t M, int64_t N) { return N % (gemv_mfma_rows(dtype, M) ? 8 : 2) == 0; }
-
 int gemv_epilogue(int epilogue) {
   return epilogue == MINITP_EPI_RESID ? EPI_RESID : epilogue == MINITP_EPI_SWIGLU ? EPI_SWIGLU : EPI_STORE;
 }
@@ -204,8 +200,6 @@ int minitp_linear_ws(void* stream, int dtype, const void* x, int64_t ldx, const 
   MINITP_CHECK_ARG(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0) && aligned16(workspace),
                    "linear: workspace %p of %lld bytes", workspace, (long long)workspace_bytes);
   hipStream_t st = S(stream);
-  if (epilogue == MINITP_EPI_SWIGLU && gemv_entry_rows(dtype, M, K) && !gemv_swiglu_width(dtype, M, N))
-    return launch_gemm_swiglu(st, dtype, x, ldx, w, y, ldy, M, N, K);
   if (epilogue == MINITP_EPI_SWIGLU ? gemv_entry_rows(dtype, M, K) : gemv_supported(dtype, M, K))
     return launch_gemv(st, dtype, PRO_NONE, gemv_epilogue(epilogue), gemv_args(x, ldx, w, bias, y, ldy, M, N, K, aux));
   if (epilogue == MINITP_EPI_SWIGLU) {
@@ -224,7 +218,7 @@ int minitp_gate_up_swiglu(void* stream, int dtype, const void* x, int64_t ldx, c
   int rc = linear_checks(dtype, x, ldx, w, nullptr, y, ldy, M, N, K, MINITP_EPI_NONE, nullptr);
   if (rc || M == 0 || N == 0) return rc;
   hipStream_t st = S(stream);
-  if (gemv_supported(dtype, M, K) && gemv_swiglu_width(dtype, M, N))
+  if (gemv_supported(dtype, M, K))
     return launch_gemv(st, dtype, PRO_NONE, EPI_SWIGLU, gemv_args(x, ldx, w, nullptr, y, ldy, M, N, K, nullptr));
   return launch_gemm_swiglu(st, dtype, x, ldx, w, y, ldy, M, N, K);
 }

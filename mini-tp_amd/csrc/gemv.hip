@@ -99,12 +99,15 @@ __device__ __forceinline__ void tuple_rows(int64_t t, const GemvArgs& a, int64_t
 
 template <int EPI, int PP = P>
 __host__ __device__ __forceinline__ int64_t num_tuples(const GemvArgs& a) {
-  if constexpr (EPI == EPI_SWIGLU) return a.N / PP;
+  if constexpr (EPI == EPI_SWIGLU) return cdiv(a.N, PP);
   if constexpr (is_qkv<EPI>()) return (int64_t)(a.a.Hq + 2 * a.a.Hkv) * (a.a.D / 2) / PP;
   return cdiv(a.N, 2 * PP);
 }
 
 // Rows that exist in the weight matrix (contiguous tuples can overhang N).
+// SwiGLU tuples overhang in the MFMA and LDS forms alone (the register form
+// takes one pair a tuple when N is odd): there a gate row past N is an up row,
+// read and not used, and an up row past 2 N reads zeros.
 template <int EPI>
 __device__ __forceinline__ bool row_valid(int64_t r, const GemvArgs& a) {
   if constexpr (EPI == EPI_STORE || EPI == EPI_RESID || EPI == EPI_ARGMAX) return r < a.N;
@@ -675,7 +678,8 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(GemvArgs a) {
       rows[P + p] = rb + p;
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) rok[r] = tup_ok && row_valid<EPI>(rows[r], a);
+    for (int r = 0; r < R; ++r)
+      rok[r] = tup_ok && row_valid<EPI>(rows[r], a) && (EPI != EPI_SWIGLU || r < P || rows[r] < 2 * a.N);
 
     float acc[MM][R];
 #pragma unroll
@@ -791,7 +795,7 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(GemvArgs a) {
                   store_f32<T>(y, m * a.ldy + row_b, add_rn(load_f32<T>(aux, m * a.ldy + row_b), round_to<T>(vb)));
               } else if constexpr (EPI == EPI_SWIGLU) {
                 T* y = (T*)a.y;
-                store_f32<T>(y, m * a.ldy + row_a, swiglu<T>(round_to<T>(va), round_to<T>(vb)));
+                if (rok[P + p]) store_f32<T>(y, m * a.ldy + row_a, swiglu<T>(round_to<T>(va), round_to<T>(vb)));
               } else if constexpr (EPI == EPI_QKV_ROPE) {
                 const T* bias = (const T*)a.bias;
                 // F.linear output with bias, rounded to the dtype (fused.py:58)
@@ -1002,7 +1006,7 @@ __device__ __forceinline__ void tuple16_rows(int64_t t, const GemvArgs& a, int64
 
 template <int EPI>
 __host__ __device__ __forceinline__ int64_t num_tuples16(const GemvArgs& a) {
-  if constexpr (EPI == EPI_SWIGLU) return a.N / P16;
+  if constexpr (EPI == EPI_SWIGLU) return cdiv(a.N, P16);
   if constexpr (is_qkv<EPI>()) return (int64_t)(a.a.Hq + 2 * a.a.Hkv) * (a.a.D / 2) / P16;
   return cdiv(a.N, 2 * P16);
 }
@@ -1296,7 +1300,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(GemvArgs a) {
       pa0[r] = __shfl_xor(acc[j][0][r], 8);
       pa1[r] = HV ? 0.f : __shfl_xor(acc[j][1][r], 8);
     }
-    if (t0 + j >= ntup || nidx >= P16) continue;
+    if (t0 + j >= ntup || nidx >= P16 || (EPI == EPI_SWIGLU && ra[j] + nidx >= a.N)) continue;
     const int p = nidx;
     const int64_t row_a = ra[j] + p, row_b = rb[j] + p;
     const bool oka = row_valid<EPI>(row_a, a), okb = row_valid<EPI>(row_b, a);
@@ -1517,7 +1521,9 @@ __global__ __launch_bounds__(256) void gemv_mfma_loop_kernel(GemvArgs a) {
     // (lane nidx + 8); plain store: every lane finishes its own column
     const int p = nidx & (P16 - 1);
     const int64_t row_a = EPI == EPI_STORE ? (nidx < P16 ? ra + p : rb + p) : ra + p;
-    const bool oka = (EPI == EPI_STORE || nidx < P16) && row_valid<EPI>(row_a, a);
+    // (pairs of the tuple: the last one's may be fewer)
+    const int pairs = EPI == EPI_SWIGLU ? (int)std::min<int64_t>(P16, a.N - ra) : P16;
+    const bool oka = (EPI == EPI_STORE || nidx < pairs) && row_valid<EPI>(row_a, a);
     float bias_a = 0.f;
     if constexpr (EPI == EPI_STORE)  // a zero-length resource reads zeros
       bias_a = bf16_to_f32((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, oka ? (uint32_t)(row_a * 2) : OOBW, 0, 0));
@@ -1803,7 +1809,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_split_kernel(GemvArgs a, int ns
         pa0[r] = __shfl_xor(acc[j][0][r], 8);
         pa1[r] = __shfl_xor(acc[j][1][r], 8);
       }
-      if (t0 + j >= ntup || nidx >= P16) continue;
+      if (t0 + j >= ntup || nidx >= P16 || (EPI == EPI_SWIGLU && ra[j] + nidx >= a.N)) continue;
       const int p = nidx;
       const int64_t row_a = ra[j] + p, row_b = rb[j] + p;
       const bool oka = row_valid<EPI>(row_a, a), okb = row_valid<EPI>(row_b, a);
@@ -2019,6 +2025,9 @@ int launch_reg_pp(hipStream_t st, const GemvArgs& a) {
 // same bit for bit.
 template <typename T, int MM, int KSPLIT, int JMAX, int PRO, int EPI>
 int launch_reg(hipStream_t st, const GemvArgs& a) {
+  if constexpr (EPI == EPI_SWIGLU) {  // (an odd number of pairs)
+    if (a.N % P != 0) return launch_reg_pp<T, MM, KSPLIT, JMAX, PRO, EPI, 1>(st, a);
+  }
   if constexpr (EPI != EPI_ARGMAX && PRO != PRO_PART_NORM) {
     if (cdiv(num_tuples<EPI>(a), (int64_t)(4 / KSPLIT)) < device_cus())
       return launch_reg_pp<T, MM, KSPLIT, JMAX, PRO, EPI, 1>(st, a);
@@ -2083,7 +2092,7 @@ bool use_split(const GemvArgs& a) {
   } else {
     const int64_t nchunk = a.K / Vec<T>::N;
     return a.split_part != nullptr && a.split_count != nullptr && nchunk > SPLIT_MIN_CHUNKS &&
-           a.split_part_bytes >= gemv_split_part_bytes(1) &&
+           a.split_part_bytes >= gemv_split_part_bytes(1) && (EPI != EPI_SWIGLU || a.N % P == 0) &&
            num_tuples<EPI>(a) <= SPLIT_MAX_TUPLES && cdiv(nchunk, 256 * SPLIT_JMAX) <= SPLIT_MAX_SEG &&
            a.K * (int64_t)sizeof(T) < (1LL << 31);
   }

@@ -272,6 +272,56 @@ def test_add_rmsnorm_linear_parts(k, nparts, dtype):
     assert torch.equal(y.cpu(), y_ref.reshape(-1).cpu())
 
 
+@pytest.mark.parametrize("dtype,m,k", [(torch.bfloat16, 1, 896), (torch.bfloat16, 2, 3584), (torch.bfloat16, 3, 896),
+                                       (torch.bfloat16, 5, 264), (torch.bfloat16, 17, 896), (torch.bfloat16, 32, 1024),
+                                       (torch.float32, 1, 896), (torch.float32, 2, 1000), (torch.float32, 4, 512),
+                                       (torch.float32, 1, 20000)])
+@pytest.mark.parametrize("n", [2, 6, 130, 4098])
+def test_swiglu_rows_finish_every_width(n, dtype, m, k):
+    """SwiGLU widths that are no multiple of a GEMV tuple (2, 4 or 8 pairs),
+    the last tuple overhanging the weight: the same bits as the first n
+    outputs of a weight padded to whole tuples, nothing left unwritten."""
+    from minitp import _native as N
+
+    if n * k > 4e7:
+        pytest.skip("wide and long: nothing new")
+    g = torch.Generator(device=DEV).manual_seed(n + m * 7 + k)
+    pad = -n % 8
+    x = torch.randn(m, k, generator=g, device=DEV).to(dtype)
+    nw = (1 + 0.1 * torch.randn(k, generator=g, device=DEV)).to(dtype)
+    gate, up = (torch.randn(n + pad, k, generator=g, device=DEV).mul_(0.05).to(dtype) for _ in range(2))
+    wide, w = torch.cat([gate, up]), torch.cat([gate[:n], up[:n]])
+    calls = [lambda w, out: _k().linear(x, w, epilogue=N.EPI_SWIGLU, out=out)]
+    if k <= 1024 or (m <= 2 and k <= 4096):
+        calls.append(lambda w, out: _k().rmsnorm_linear(x, nw, 1e-6, w, epilogue=N.EPI_SWIGLU, out=out))
+    for call in calls:
+        got, ref = (torch.full((m, c), float("nan"), dtype=dtype, device=DEV) for c in (n, n + pad))
+        call(w, got)
+        call(wide, ref)
+        assert torch.equal(got, ref[:, :n])
+
+
+@pytest.mark.parametrize("dtype,k", [(torch.bfloat16, 896), (torch.float32, 896), (torch.float32, 64)])
+@pytest.mark.parametrize("n", [1, 3, 131, 1025])
+def test_add_rmsnorm_linear_parts_finishes_odd_widths(n, dtype, k):
+    from minitp import _native as N
+
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    x = torch.randn(k, generator=g, device=DEV).to(dtype)
+    parts = torch.randn(3, k, generator=g, device=DEV)
+    nw = (1 + 0.1 * torch.randn(k, generator=g, device=DEV)).to(dtype)
+    gate, up = (torch.randn(n + 1, k, generator=g, device=DEV).mul_(0.05).to(dtype) for _ in range(2))
+    ys = []
+    for w in (torch.cat([gate[:n], up[:n]]), torch.cat([gate, up])):
+        width = w.shape[0] // 2
+        y, x_out = torch.full((width,), float("nan"), dtype=dtype, device=DEV), torch.empty_like(x)
+        N.check(N.lib().minitp_add_rmsnorm_linear_parts(
+            N.stream(), N.dtype_code(dtype), x.data_ptr(), parts.data_ptr(), 3, x_out.data_ptr(), nw.data_ptr(), 1e-6,
+            w.data_ptr(), y.data_ptr(), width, k, N.EPI_SWIGLU), "add_rmsnorm_linear_parts")
+        ys.append(y)
+    assert torch.equal(ys[0], ys[1][:n])
+
+
 def test_rmsnorm_linear_refuses_prefill_shapes():
     x = torch.randn(8, 896, device=DEV)
     nw = torch.ones(896, device=DEV)
