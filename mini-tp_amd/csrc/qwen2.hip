@@ -318,7 +318,9 @@ struct Qwen2Program {
         if (rc) return rc;
         // x += down(act), h = the next layer's input_layernorm(x) (the final norm after the last)
         const void* next_norm = l + 1 < c.num_layers ? L(l + 1, MINITP_W_LN1) : final_norm;
-        rc = partials(w.act, I, L(l, MINITP_W_DOWN), H, I, &pp);
+        // (the final norm's weight may have any alignment, the layers' are checked
+        // at creation: the kernel that adds partials wants 16 bytes)
+        rc = aligned16(next_norm) ? partials(w.act, I, L(l, MINITP_W_DOWN), H, I, &pp) : MINITP_ERR_UNSUPPORTED;
         if (rc == MINITP_OK) {
           rc = launch_add_rmsnorm_partials(st, c.dtype, w.x, pp, next_norm, w.h, H, c.eps);
         } else if (rc == MINITP_ERR_UNSUPPORTED) {

@@ -2,7 +2,7 @@
 csrc/rope.hip): RMSNorm on vector pieces against float64 at the edges of what
 stays in registers, SwiGLU on ragged strides, and forwards whose products are
 split over K (their partials added by the consuming kernel) against the
-module path, which never splits, at every row count where the tile or the
+module path, whose products choose their own splits, at every row count where the tile or the
 split changes.
 """
 
@@ -75,3 +75,28 @@ def test_forward_matches_the_module_path(shape, batch, tokens, dtype, atol):
         out.append((logits.float(), kv.k[1].float(), kv.v[1].float()))
     for a, b in zip(*out):
         torch.testing.assert_close(a, b, atol=atol, rtol=0.02 if dtype == torch.bfloat16 else 2e-5)
+
+
+@pytest.mark.parametrize("dtype,atol", [(torch.float32, 2e-5), (torch.bfloat16, 0.05)])
+@pytest.mark.parametrize("batch,tokens", [(40, 1), (1, 33), (1, 300)])
+def test_forward_takes_a_final_norm_of_any_alignment(batch, tokens, dtype, atol):
+    """A final RMSNorm weight that starts one element past a 16-byte boundary
+    (the last down projection's partials cannot be added by the vector
+    kernel then): the module path's logits."""
+    from minitp import synthetic
+    from minitp.generation import make_kv_cache
+
+    cfg = dataclasses.replace(synthetic.QWEN05B, num_hidden_layers=2, vocab_size=2048, max_position_embeddings=512)
+    model = synthetic.build_synthetic_model(cfg, dtype=dtype, device=DEV, seed=0)
+    weight = model.model.norm.weight
+    store = torch.empty(weight.numel() + 1, dtype=dtype, device=DEV)
+    store[1:] = 1 + 0.1 * torch.randn(weight.numel(), generator=torch.Generator(device=DEV).manual_seed(2), device=DEV)
+    model.model.norm.weight = torch.nn.Parameter(store[1:], requires_grad=False)
+    ids = synthetic.synthetic_prompt(cfg.vocab_size, batch, PAST + tokens, seed=1, device=DEV)
+    out = []
+    for rotary in (True, False):  # False: the module path
+        model.use_rotary_cache = rotary
+        kv = make_kv_cache(model, batch, PAST + tokens, init="zeros")
+        model(ids[:, :PAST], kv_cache=kv)
+        out.append(model(ids[:, PAST:], positions=torch.arange(PAST, PAST + tokens, device=DEV), kv_cache=kv).float())
+    torch.testing.assert_close(*out, atol=atol, rtol=0.02 if dtype == torch.bfloat16 else 2e-5)
