@@ -772,6 +772,23 @@ struct PrefillKV {
   }
 };
 
+// A head's cache rows [0, rows) in tiles of KT rows, each read through a
+// resource of its own, so that they may span more than the 4 GiB that one
+// resource reaches; loads of rows past the last read zeros. (Tile numbers in
+// 32 bits: the scalar unit has no 64-bit comparison.)
+template <int KT, int ROW_BYTES>
+struct KvTiles {
+  static constexpr int BYTES = KT * ROW_BYTES;
+  const char* base;
+  int full, rest;  // whole tiles, bytes of the one after them
+  __device__ __forceinline__ KvTiles(const void* p, int64_t rows)
+      : base((const char*)p), full((int)(rows / KT)), rest((int)(rows % KT) * ROW_BYTES) {}
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t at(int tile) const {
+    const int n = tile < full ? BYTES : tile == full ? rest : 0;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (int64_t)tile * BYTES), (short)0, n, 0x00020000);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Prefill, fp32, on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 products
 // and sums). Block = (b * Hq + h, 64-query tile), wave w = the 16-query strip
@@ -834,20 +851,19 @@ __global__ __launch_bounds__(256) void prefill_attn_f32_kernel(const float* q, c
   const int64_t tb_last = std::min<int64_t>(tile0 + QT, s.T) - 1;
   const int64_t key_end = cache_len + tb_last + 1;  // keys the block's queries may see
 
-  const uint32_t kv_bytes = (uint32_t)(key_end * D * 4);
-  const __amdgpu_buffer_rsrc_t krs = span_rsrc(kbase, kv_bytes), vrs = span_rsrc(vbase, kv_bytes);
   uint4 kr[PER], vr[PER];
-  auto load_tile = [&](int64_t k0) {  // rows past key_end read zeros
+  const KvTiles<KT, D * 4> ktiles(kbase, key_end), vtiles(vbase, key_end);
+  auto load_tile = [&](int tile) {
+    const __amdgpu_buffer_rsrc_t krs = ktiles.at(tile), vrs = vtiles.at(tile);
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int i = tid + 256 * u;
-      const int64_t key = k0 + i / (D / 4);
-      const uint32_t off = i < PIECES && key < key_end ? (uint32_t)((key * D + i % (D / 4) * 4) * 4) : kv_bytes;
+      const uint32_t off = (uint32_t)(tid + 256 * u) * 16;  // (past the tile: not stored)
       kr[u] = attn_load16(krs, off);
       vr[u] = attn_load16(vrs, off);
     }
   };
   load_tile(0);
+  int tile = 0;
   for (int64_t k0 = 0; k0 < key_end; k0 += KT) {
     __syncthreads();  // the previous tile is consumed
 #pragma unroll
@@ -860,7 +876,7 @@ __global__ __launch_bounds__(256) void prefill_attn_f32_kernel(const float* q, c
       }
     }
     __syncthreads();
-    if (k0 + KT < key_end) load_tile(k0 + KT);
+    if (k0 + KT < key_end) load_tile(++tile);
     if (t0 >= s.T || k0 > cache_len + t0 + 15) continue;  // this strip sees none of the tile
     const int64_t limit = cache_len + t - k0;             // last key of the tile this query may see
     float sc[KB][4];
@@ -998,15 +1014,14 @@ __global__ __launch_bounds__(PW * 64) void prefill_attn_mfma_kernel(const bf16* 
   // fill one contiguous run of a Vt row (no bank conflicts)
   const int kqv = tid % (KT / KQ), pcv = tid / (KT / KQ);
   const bool stager = tid < NPC / KQ;
-  const uint32_t kv_bytes = (uint32_t)(key_end * D * 2);
-  const __amdgpu_buffer_rsrc_t krs = span_rsrc(kbase, kv_bytes), vrs = span_rsrc(vbase, kv_bytes);
   uint4 kr[KQ], vr[KQ];
-  auto load_tile = [&](int64_t k0) {
+  const KvTiles<KT, D * 2> ktiles(kbase, key_end), vtiles(vbase, key_end);
+  auto load_tile = [&](int tile) {
+    const __amdgpu_buffer_rsrc_t krs = ktiles.at(tile), vrs = vtiles.at(tile);
 #pragma unroll
     for (int u = 0; u < KQ; ++u) {
-      const int64_t key = k0 + kq * KQ + u, keyv = k0 + kqv * KQ + u;
-      kr[u] = attn_load16(krs, stager && key < key_end ? (uint32_t)((key * D + pc * 8) * 2) : kv_bytes);
-      vr[u] = attn_load16(vrs, stager && keyv < key_end ? (uint32_t)((keyv * D + pcv * 8) * 2) : kv_bytes);
+      kr[u] = attn_load16(krs, stager ? (uint32_t)(((kq * KQ + u) * D + pc * 8) * 2) : KT * D * 2);
+      vr[u] = attn_load16(vrs, stager ? (uint32_t)(((kqv * KQ + u) * D + pcv * 8) * 2) : KT * D * 2);
     }
   };
   auto store_tile = [&]() {
@@ -1034,11 +1049,12 @@ __global__ __launch_bounds__(PW * 64) void prefill_attn_mfma_kernel(const bf16* 
   };
 
   load_tile(0);
+  int tile = 0;
   for (int64_t k0 = 0; k0 < key_end; k0 += KT) {
     __syncthreads();  // the previous tile is consumed
     store_tile();
     __syncthreads();
-    if (k0 + KT < key_end) load_tile(k0 + KT);  // in flight during this tile's math
+    if (k0 + KT < key_end) load_tile(++tile);  // in flight during this tile's math
     if (t0 >= s.T || k0 > cache_len + t0 + 15) continue;  // this strip sees none of the tile
     // ---- scores, transposed: S^T[key k0 + 16 kbk + 4 lq + i][query t0 + lr]
     // (A = the K rows, B = Q^T: the query operand registers as they are)
@@ -1189,17 +1205,16 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void prefill_attn_fa_kernel(const 
   const int kq = tid / PPRW, pc = tid % PPRW;
   const int kqv = tid % (KT / KQ), pcv = tid / (KT / KQ);
   static_assert(NPC / KQ == 256, "every thread stages");
-  // pieces of keys past key_end lie past the buffer's size and read as zeros
-  const uint32_t kv_bytes = (uint32_t)(key_end * D * 2);
-  const __amdgpu_buffer_rsrc_t krs = span_rsrc(kbase, kv_bytes), vrs = span_rsrc(vbase, kv_bytes);
+  // pieces of keys past key_end lie past the tile's size and read as zeros
   const uint32_t koff = (uint32_t)((kq * KQ * D + pc * 8) * 2), voff = (uint32_t)((kqv * KQ * D + pcv * 8) * 2);
   uint4 kr[KQ], vr[KQ];
-  auto load_tile = [&](int64_t k0) {
-    const uint32_t base = (uint32_t)(k0 * D * 2);
+  const KvTiles<KT, D * 2> ktiles(kbase, key_end), vtiles(vbase, key_end);
+  auto load_tile = [&](int tile) {
+    const __amdgpu_buffer_rsrc_t krs = ktiles.at(tile), vrs = vtiles.at(tile);
 #pragma unroll
     for (int u = 0; u < KQ; ++u) {
-      kr[u] = attn_load16(krs, base + koff + u * D * 2);
-      vr[u] = attn_load16(vrs, base + voff + u * D * 2);
+      kr[u] = attn_load16(krs, koff + u * D * 2);
+      vr[u] = attn_load16(vrs, voff + u * D * 2);
     }
   };
   auto store_tile = [&](char* Ks) {
@@ -1228,9 +1243,9 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void prefill_attn_fa_kernel(const 
 
   // (tiles past the last, which groups may have, read zeros and are skipped)
   const int64_t nit = cdiv(ntiles, (int64_t)GROUPS);
-  load_tile(group * KT);
+  load_tile(group);
   store_tile(lds);
-  if (nit > 1) load_tile((GROUPS + group) * KT);
+  if (nit > 1) load_tile(GROUPS + group);
   __syncthreads();
   for (int64_t it = 0; it < nit; ++it) {
     const int64_t k0 = (it * GROUPS + group) * KT;
@@ -1325,7 +1340,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void prefill_attn_fa_kernel(const 
     }
     if (it + 1 < nit) store_tile(lds + ((it + 1) & 1) * STAGE);  // that buffer was last read before the previous barrier
     __syncthreads();
-    if (it + 2 < nit) load_tile(((it + 2) * GROUPS + group) * KT);
+    if (it + 2 < nit) load_tile((int)(it + 2) * GROUPS + group);
   }
   if constexpr (GROUPS > 1) {
     // (the last barrier freed every buffer) [group - 1][wave][strip][value][lane]

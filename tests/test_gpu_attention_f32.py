@@ -55,3 +55,22 @@ def test_prefill_attention_f32_large_scores():
     # scores of order 13,000 carry an absolute error of up to 13,000 x 2^-24 x 8
     assert torch.isfinite(out).all()
     assert (out.double() - ref).abs().max().item() <= 0.05
+
+
+@pytest.mark.parametrize("dtype,d,t", [(torch.float32, 128, 2), (torch.bfloat16, 128, 3), (torch.bfloat16, 128, 70)])
+def test_prefill_attention_past_4_gib_of_keys(dtype, d, t):
+    """A head whose rows span more than 4 GiB: zeros but for one key past that
+    line (and its image modulo 2^32 bytes), which every query picks."""
+    from minitp import kernels as K
+
+    rows = (1 << 32) // (d * dtype.itemsize)
+    n = rows + 200 + t
+    kc = torch.zeros(1, 1, n, d, dtype=dtype, device=DEV)
+    vc = torch.zeros_like(kc)
+    q = torch.ones(1, t, 1, d, dtype=dtype, device=DEV)
+    at = rows + 100
+    kc[0, 0, at] = 64.0  # score 64 sqrt(128): e^-724 is left for the zero keys
+    vc[0, 0, at] = torch.arange(d, device=DEV).to(dtype)
+    vc[0, 0, at % rows] = -5.0
+    out = K.attention(q, kc, vc, n - t).view(t, d)
+    assert torch.equal(out, vc[0, 0, at].expand(t, d))
