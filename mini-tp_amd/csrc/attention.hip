@@ -1440,19 +1440,20 @@ int prefill_dispatch(hipStream_t st, const void* q, const void* k, const void* v
       // 64-query blocks (2 x 700 tokens, 28 heads of 128, 336 / 616 blocks: 25.5
       // against 22.5 us; 2 x 1024, 448 / 896: 36.6 against 39.3), and while
       // all of those are resident at once (two groups: 139 KiB of LDS at D =
-      // 128, 72 at 64) and the cache may hold long contexts, two groups of
-      // waves per block walk alternate key tiles (512 queries on 1,500
-      // cached keys, 28 heads of 128: 38.5 against 45.7 us; 1,000 queries, 14
-      // heads of 64: 13.1 against 15.1; 128 queries on nothing: 5.2 against
-      // 4.8). The choice depends on nothing but the launch's shape, so a
-      // replayed graph and a direct launch agree bit for bit.
+      // 128, 72 at 64) and the queries see long contexts, two groups of
+      // waves per block walk alternate key tiles. One group against two, 14
+      // heads of 64: 128 queries on nothing 4.9 and 5.2 us, 300 6.9 and 6.9,
+      // 500 9.3 and 8.4, 64 on 500 cached keys 10.2 and 9.2; 28 heads of 128:
+      // 64 on nothing 5.5 and 6.8, 300 10.0 and 10.5, 433 12.8 and 12.7, 64 on
+      // 500 15.6 and 14.6, 512 on 1,500 45.7 and 36. Graph replays are keyed
+      // by the same line, so a replay and a direct launch agree bit for bit.
       auto go = [&](auto kern, int queries, int threads) {
         hipLaunchKernelGGL(kern, dim3((unsigned)units, (unsigned)cdiv(s.T, queries)), dim3(threads), 0, st,
                            (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)out, s, cache_len, scale, kv);
       };
       if (units * cdiv(s.T, 128) >= 512)
         go(prefill_attn_fa_kernel<D, 2, 1>, 128, 256);
-      else if (s.S >= 1024 && units * cdiv(s.T, 64) <= device_cus() * (D <= 64 ? 2 : 1))
+      else if (prefill_attn_far(cache_len + s.T) && units * cdiv(s.T, 64) <= device_cus() * (D <= 64 ? 2 : 1))
         go(prefill_attn_fa_kernel<D, 1, 2>, 64, 512);
       else
         go(prefill_attn_fa_kernel<D, 1, 1>, 64, 256);

@@ -248,6 +248,9 @@ int launch_decode_attention_oproj(hipStream_t st, int dtype, const void* q, cons
                                   const StepState* state, int layer, const OprojArgs& o);
 // Inside a forward (state != null) the caches of layer `layer` and cache_len
 // come from the step state (k_cache, v_cache and cache_len unused).
+// Whether prompt attention over this many keys (cached and new) takes its
+// form for long contexts: part of what a recorded launch depends on.
+inline bool prefill_attn_far(int64_t keys) { return keys >= 448; }
 int launch_prefill_attention(hipStream_t st, int dtype, const void* q, const void* k_cache, const void* v_cache,
                              void* out, const AttnShape& a, int64_t cache_len, const StepState* state = nullptr,
                              int layer = 0);

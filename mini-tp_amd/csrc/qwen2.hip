@@ -108,17 +108,18 @@ struct Ws {
 struct GraphKey {
   int64_t batch, tokens, max_seq;
   void* workspace;
-  bool eos, pick, all;
+  bool eos, pick, all, far;
   bool operator==(const GraphKey& o) const {
     return batch == o.batch && tokens == o.tokens && max_seq == o.max_seq && workspace == o.workspace &&
-           eos == o.eos && pick == o.pick && all == o.all;
+           eos == o.eos && pick == o.pick && all == o.all && far == o.far;
   }
 };
 
 struct GraphEntry {
   GraphKey key;  // eos: the end-of-sequence update after the token selection;
                  // pick: the token selection (next_tok set; batch > 4 has no pick
-                 // node otherwise); all: every position's logits, not the last's
+                 // node otherwise); all: every position's logits, not the last's;
+                 // far: a prompt's attention in its form for long contexts
   hipGraph_t graph;
   hipGraphExec_t exec;
   hipGraphNode_t first;
@@ -556,7 +557,8 @@ static int patch_and_launch(Qwen2Program* p, GraphEntry& g, hipStream_t st, cons
 
 // One forward through a captured graph of its launch sequence: replayed when
 // a graph of this shape (batch, tokens, max_seq, workspace, early stop, token
-// pick, all-position logits: everything the launch sequence depends on)
+// pick, all-position logits, the attention's form: everything the launch
+// sequence depends on)
 // exists, else run eagerly once and recorded. Every kernel after the
 // first reads the per-call values (ids, positions, cache_len, caches, logits,
 // token outputs) from the step state the first kernel writes, so only that
@@ -567,7 +569,7 @@ static int run_graphed(Qwen2Program* p, hipStream_t st, const minitp_qwen2_step&
   if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) return p->run(st, s, w);
   std::lock_guard<std::mutex> lock(p->mu);
   const GraphKey key{s.batch, s.tokens, s.max_seq, s.workspace, s.eos_state != nullptr, s.next_tok != nullptr,
-                     s.logits_all != 0};
+                     s.logits_all != 0, s.tokens > 1 && prefill_attn_far(s.cache_len + s.tokens)};
   const uint64_t now = ++p->clock;
   // calls of this shape
   ShapeCalls* sc = nullptr;

@@ -15,9 +15,9 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("d,hq,hkv", [(32, 4, 2), (64, 14, 2), (128, 28, 4), (16, 4, 2)])
-@pytest.mark.parametrize("rows", [0, 1100])  # cache capacity: below / past the two-group line
+@pytest.mark.parametrize("rows", [0, 1100])  # cache capacity: the keys and a few rows, or more
 @pytest.mark.parametrize("t,cache_len", [(2, 0), (17, 47), (64, 0), (65, 63), (128, 1), (130, 64), (200, 700),
-                                         (1000, 0), (500, 129)])
+                                         (1000, 0), (500, 129), (447, 0), (448, 0), (2, 446), (70, 378)])
 def test_prefill_attention_bf16_matches_float64(t, cache_len, rows, d, hq, hkv):
     from minitp import kernels as K
 

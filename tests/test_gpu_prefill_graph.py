@@ -87,6 +87,34 @@ def test_prefill_graph_replays_match_direct_runs_bitwise(batch, monkeypatch):
     assert torch.isfinite(outs[0][1]).all()
 
 
+@torch.inference_mode()
+@pytest.mark.parametrize("shape", ["qwen2.5-0.5b", "qwen2.5-7b"])
+def test_prefill_graphs_of_one_shape_keep_the_attention_form_apart(shape, monkeypatch):
+    """Chunks of one length on contexts on both sides of the line between the
+    attention's forms (448 keys), each form recorded and replayed in turn:
+    bitwise against direct runs on the same cache."""
+    cfg, (graphed, _), (direct, _) = _models(monkeypatch, shape)
+    from minitp.generation import GenerationState, make_kv_cache
+
+    g = torch.Generator().manual_seed(21)
+    chunk = torch.randint(0, cfg.vocab_size, (1, 60), generator=g).to(DEV)
+    outs = []
+    for model in (graphed, direct):
+        kv = make_kv_cache(model, 1, 1600, init="zeros")
+        gen = torch.Generator(device=DEV).manual_seed(5)
+        for layer in range(2):
+            kv.k[layer].normal_(0, 0.6, generator=gen)
+            kv.v[layer].normal_(0, 0.6, generator=gen)
+        got = []
+        for start in (0, 387, 388, 1500, 10, 700, 0, 388, 387):
+            kv.seq_len = start
+            got.append(GenerationState(model, chunk, 1, prefill_logits="last", kv=kv).prefill().float().clone())
+        outs.append(got)
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("shape,batch,tokens", [("qwen2.5-0.5b", 1, 8), ("qwen2.5-0.5b", 40, 8),
                                                 ("qwen2.5-0.5b", 3, 256), ("qwen2.5-7b", 1, 512)])
 def test_prefill_graph_replays_other_launch_paths_bitwise(shape, batch, tokens, monkeypatch):
