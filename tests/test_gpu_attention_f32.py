@@ -39,6 +39,30 @@ def test_prefill_attention_f32_matches_float64(t, cache_len, d):
     assert (out - ref).abs().max().item() <= 1e-5
 
 
+@pytest.mark.parametrize("t,hq,d", [(64, 28, 128), (40, 14, 64)])
+def test_prefill_attention_f32_scores_in_short_chains(t, hq, d):
+    """The relative 2-norm of the error. A chain of m sums of products of
+    N(0, 1) factors has partial sums of sqrt(k), each rounded by u sqrt(k / 3) (u =
+    2^-24): a variance of u^2 m^2 / 6. Four chains of D / 4 and the two levels
+    of their sum: u^2 (D^2 / 24 + 2 D / 3), and over the D of the scale that is the
+    relative error of a weight, so of an output (the sums over a few dozen keys add
+    little): u sqrt(D / 24 + 2 / 3). One chain of D: u sqrt(D / 6), past the bar."""
+    from minitp import kernels as K
+
+    errs = []
+    for seed in range(4):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        q = torch.randn(2, t, hq, d, generator=g, device=DEV)
+        kc, vc = (torch.randn(2, 2, t, d, generator=g, device=DEV) for _ in range(2))
+        out = K.attention(q, kc, vc, 0).view(2, t, hq, d).double()
+        kk, vv = (x.double().repeat_interleave(hq // 2, 1) for x in (kc, vc))
+        s = (q.double().transpose(1, 2) @ kk.transpose(-1, -2).contiguous()) / d ** 0.5
+        mask = torch.triu(torch.ones(t, t, device=DEV, dtype=torch.bool), 1)
+        ref = (s.masked_fill(mask, float("-inf")).softmax(-1) @ vv).transpose(1, 2)
+        errs.append(((out - ref).norm() / ref.norm()).item())
+    assert sum(errs) / len(errs) <= 1.15 * 2.0 ** -24 * (d / 24 + 2 / 3) ** 0.5, errs
+
+
 def test_prefill_attention_f32_large_scores():
     """Scores far past the exponential's range, one key per query dominating."""
     from minitp import kernels as K
