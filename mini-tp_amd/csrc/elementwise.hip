@@ -223,8 +223,21 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_rows_kernel(const T* xin, T
   ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
-  float tot = red[0];
-  for (int i = 1; i < nt / 64; ++i) tot += red[i];
+  float tot;
+  if constexpr (sizeof(T) == 4) {
+    // fp32 rows: the waves' sums added in 64 bits. What rounds in the last levels
+    // of a sum depends on where its halves lie: as a chain of eight in 32 bits
+    // (the bf16 rows', whose outputs round at 2^-9), rows of 3,584 were 5 % further
+    // from 64-bit results than with four waves' sums in pairs.
+    static_assert(NORM_THREADS == 512, "eight waves");
+    double part[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[i] = i < nt / 64 ? (double)red[i] : 0.0;
+    tot = (float)(((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7])));
+  } else {
+    tot = red[0];
+    for (int i = 1; i < nt / 64; ++i) tot += red[i];
+  }
   const float r = __fdiv_rn(1.0f, __fsqrt_rn(add_rn(__fdiv_rn(tot, (float)hidden), eps)));
   if (keep) {
 #pragma unroll

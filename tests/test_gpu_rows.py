@@ -37,6 +37,27 @@ def test_rmsnorm_matches_float64(rows, hidden, dtype):
     assert ((got - ref).abs() <= 2 * eps * ref.abs() + 1e-30).all()
 
 
+@pytest.mark.parametrize("hidden", [896, 2048, 3584, 8192])
+def test_rmsnorm_f32_sums_add_little_error(hidden):
+    """The relative 2-norm of the error against what the same fp32 steps give
+    with an exact sum of squares (its rounding alone): a fp32 sum's last
+    levels may add 6 % to it (four sums in pairs: 4 %; a chain of eight: 9 %)."""
+    from minitp import kernels as K
+
+    got_err = ref_err = 0.0
+    for seed in range(6):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        x = torch.randn(2000, hidden, generator=g, device=DEV)
+        w = torch.randn(hidden, generator=g, device=DEV)
+        xd = x.double()
+        want = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-6) * w.double()
+        total = (x * x).double().sum(-1, keepdim=True).float()
+        steps = (x * (1.0 / torch.sqrt(total / hidden + 1e-6))) * w
+        got_err += (K.rmsnorm(x, w, 1e-6).double() - want).pow(2).sum().item()
+        ref_err += (steps.double() - want).pow(2).sum().item()
+    assert got_err <= 1.06 ** 2 * ref_err, (got_err / ref_err) ** 0.5
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows,n,pad", [(1, 8, 0), (3, 24, 8), (5, 130, 2), (257, 4864, 0), (2, 12, 4)])
 def test_silu_mul_matches_float64(rows, n, pad, dtype):
