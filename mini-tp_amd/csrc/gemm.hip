@@ -98,18 +98,19 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Tile shape of a launch: BM x BN outputs, WK waves per wave tile (64 columns,
-// 64 rows or all BM = 32), a ring of STAGES, non-temporal loads (NT).
+// Tile shape of a launch: BM x BN outputs in wave tiles of FM x FN fragments
+// (32 x 32), WK waves per wave tile, a ring of STAGES, non-temporal loads (NT).
+// WHOLE: a product of at most STAGES stages, all loaded at once (no ring).
 constexpr int KCH = 8;  // 16-byte chunks of K per row and stage
-template <int BM_, int BN_, int WK_, int STAGES_, bool NT_ = false>
+template <int BM_, int BN_, int WK_, int STAGES_, bool NT_ = false, int FM_ = (BM_ >= 64 ? 2 : 1), int FN_ = 2,
+          bool WHOLE_ = false>
 struct Tile {
-  static constexpr bool NT = NT_;
-  static constexpr int BM = BM_, BN = BN_, WK = WK_, STAGES = STAGES_;
-  static constexpr int FM = BM >= 64 ? 2 : 1;  // 32-row fragments per wave tile
-  static constexpr int WM = BM / (32 * FM), WN = BN / 64, NW = WM * WN * WK, THREADS = 64 * NW;
+  static constexpr bool NT = NT_, WHOLE = WHOLE_;
+  static constexpr int BM = BM_, BN = BN_, WK = WK_, STAGES = STAGES_, FM = FM_, FN = FN_;
+  static constexpr int WM = BM / (32 * FM), WN = BN / (32 * FN), NW = WM * WN * WK, THREADS = 64 * NW;
   static constexpr int ROWB = KCH * 16;
   static constexpr int STAGE_BYTES = (BM + BN) * ROWB;
-  static constexpr int RING_BYTES = STAGES * STAGE_BYTES, XCH_BYTES = WM * WN * (WK - 1) * FM * 8192;
+  static constexpr int RING_BYTES = STAGES * STAGE_BYTES, XCH_BYTES = WM * WN * (WK - 1) * FM * FN * 4096;
   static constexpr int LDS_BYTES = RING_BYTES > XCH_BYTES ? RING_BYTES : XCH_BYTES;
   static constexpr int PIECE_ROWS = 64 / KCH;                   // rows of one 1 KiB load
   static constexpr int PPW = (BM + BN) / PIECE_ROWS / NW;       // loads per wave and stage
@@ -129,17 +130,25 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
                                                           int kper, int tiles_m, int tiles_n, int items,
                                                           const StepState* state) {
   constexpr int BM = C::BM, BN = C::BN, WK = C::WK, STAGES = C::STAGES, PPW = C::PPW;
-  constexpr int FM = C::FM, WN = C::WN, ROWB = C::ROWB, ES = (int)sizeof(T), V = 16 / ES, TK = KCH * V;
+  constexpr int FM = C::FM, FN = C::FN, WN = C::WN, ROWB = C::ROWB, ES = (int)sizeof(T), V = 16 / ES, TK = KCH * V;
+  static_assert(OUT != OUT_SWIGLU || FN == 2, "a wave tile holds whole gate and up fragment pairs");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   if (state != nullptr) y = (T*)state->args.logits;
   const int per_xcd = (items + 7) >> 3;
   const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per_xcd || item >= items) return;
   const int tiles = tiles_m * tiles_n;
-  const int z = item / tiles, t = item - z * tiles;
-  const int group = t / (8 * tiles_n), first_m = group * 8, gsz = min(tiles_m - first_m, 8);
+  // (no division where the quotient is known: the three take 50 to 100 ns ahead
+  // of the first load)
+  int z = 0, group = 0;
+  if (items != tiles) z = item / tiles;
+  const int t = item - z * tiles;
+  if (tiles_m > 8) group = t / (8 * tiles_n);
+  const int first_m = group * 8, gsz = min(tiles_m - first_m, 8);
   const int in_group = t - group * 8 * tiles_n;
-  const int m0 = (first_m + in_group % gsz) * BM, tn = in_group / gsz;
+  int tn = in_group;
+  if (gsz > 1) tn = in_group / gsz;
+  const int m0 = (first_m + in_group - tn * gsz) * BM;
   const int kb = z * kper, ke = min(kb + kper, K);
 
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
@@ -198,32 +207,35 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
                  (uint32_t)__builtin_amdgcn_readfirstlane(base + j * 1024));
   };
 
-  f32x16 acc[FM][2];  // [x fragment][W fragment]
+  f32x16 acc[FM][FN];  // [x fragment][W fragment]
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  const int ar = wm * (32 * FM) + (lane & 31), br = wn * 64 + (lane & 31);
+  const int ar = wm * (32 * FM) + (lane & 31), br = wn * (32 * FN) + (lane & 31);
   // (rows 32 apart share the swizzle)
   const int a_off = ar * ROWB, b_off = A_BYTES + br * ROWB, a_swz = swz(ar), b_swz = swz(br);
   constexpr int KS = KCH / 2 / WK;  // substeps of a stage per wave group
 #pragma unroll 1
-  for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
+  for (int s = 0; s < (C::WHOLE ? nk : STAGES - 1); ++s) issue(s, s);
+  if constexpr (C::WHOLE) stage_barrier<0>();
   int rd = 0, wr_stage = STAGES - 1;
   for (int kt = 0; kt < nk; ++kt) {
-    stage_barrier<(STAGES - 2) * PPW>();
-    issue(kt + STAGES - 1, wr_stage);
+    if constexpr (!C::WHOLE) {
+      stage_barrier<(STAGES - 2) * PPW>();
+      issue(kt + STAGES - 1, wr_stage);
+    }
     const char* st = lds + rd * C::STAGE_BYTES;
-    u32x4 av[2][FM], bv[2][2];
-    auto fetch = [&](int s, u32x4(&a)[FM], u32x4(&b)[2]) {
+    u32x4 av[2][FM], bv[2][FN];
+    auto fetch = [&](int s, u32x4(&a)[FM], u32x4(&b)[FN]) {
       const int c = (s * WK + wk) * 2 + half;
 #pragma unroll
       for (int i = 0; i < FM; ++i) a[i] = *(const u32x4*)(st + a_off + i * 32 * ROWB + ((c ^ a_swz) << 4));
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = *(const u32x4*)(st + b_off + j * 32 * ROWB + ((c ^ b_swz) << 4));
+      for (int j = 0; j < FN; ++j) b[j] = *(const u32x4*)(st + b_off + j * 32 * ROWB + ((c ^ b_swz) << 4));
     };
     fetch(0, av[0], bv[0]);
 #pragma unroll
@@ -232,7 +244,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_step<T>(bv[s & 1][j], av[s & 1][i], acc[i][j]);
+        for (int j = 0; j < FN; ++j) acc[i][j] = mfma_step<T>(bv[s & 1][j], av[s & 1][i], acc[i][j]);
     }
     rd = rd + 1 == STAGES ? 0 : rd + 1;
     wr_stage = wr_stage + 1 == STAGES ? 0 : wr_stage + 1;
@@ -248,15 +260,15 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
     __syncthreads();  // (the ring is free: every wave's last reads and loads are done)
     u32x4* xch = (u32x4*)lds;
     const int wt = wave % (C::WM * WN);
-    auto slot = [&](int f, int g, int q) { return (((wt * 2 * FM + f) * (WK - 1) + g) * 4 + q) * 64 + lane; };
+    auto slot = [&](int f, int g, int q) { return (((wt * FM * FN + f) * (WK - 1) + g) * 4 + q) * 64 + lane; };
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int owner = q * WK / 4;
       if (owner == wk) continue;
       const int g = wk < owner ? wk : wk - 1;
 #pragma unroll
-      for (int f = 0; f < 2 * FM; ++f) {
-        const f32x16& a = acc[f >> 1][f & 1];
+      for (int f = 0; f < FM * FN; ++f) {
+        const f32x16& a = acc[f / FN][f % FN];
         xch[slot(f, g, q)] = u32x4{__float_as_uint(a[4 * q]), __float_as_uint(a[4 * q + 1]),
                                    __float_as_uint(a[4 * q + 2]), __float_as_uint(a[4 * q + 3])};
       }
@@ -266,14 +278,14 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
     for (int q = 0; q < 4; ++q) {
       if (q * WK / 4 != wk) continue;
 #pragma unroll
-      for (int f = 0; f < 2 * FM; ++f) {
+      for (int f = 0; f < FM * FN; ++f) {
         float v[4];
 #pragma unroll
         for (int g = 0; g < WK; ++g) {
           float p[4];
           if (g == wk) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) p[e] = acc[f >> 1][f & 1][4 * q + e];
+            for (int e = 0; e < 4; ++e) p[e] = acc[f / FN][f % FN][4 * q + e];
           } else {
             const u32x4 u = xch[slot(f, g < wk ? g : g - 1, q)];
 #pragma unroll
@@ -283,7 +295,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
           for (int e = 0; e < 4; ++e) v[e] = g == 0 ? p[e] : v[e] + p[e];
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[f >> 1][f & 1][4 * q + e] = v[e];
+        for (int e = 0; e < 4; ++e) acc[f / FN][f % FN][4 * q + e] = v[e];
       }
     }
   }
@@ -300,7 +312,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
     for (int e = 0; e < 4; ++e) {
       const float a = acc[i][j][4 * q + e];
       if constexpr (OUT == OUT_SWIGLU)
-        v[e] = swiglu<T>(round_to<T>(a + 0.f), round_to<T>(acc[i][1][4 * q + e] + 0.f));
+        v[e] = swiglu<T>(round_to<T>(a + 0.f), round_to<T>(acc[i][FN - 1][4 * q + e] + 0.f));
       else if constexpr (OUT == MINITP_EPI_RESID)
         v[e] = col + e < N ? add_rn(load_f32<T>(aux, row * ldy + col + e), round_to<T>(a)) : 0.f;
       else if constexpr (OUT == MINITP_EPI_NONE)
@@ -309,7 +321,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
         v[e] = a;
     }
   };
-  constexpr int FJ = OUT == OUT_SWIGLU ? 1 : 2;
+  constexpr int FJ = OUT == OUT_SWIGLU ? 1 : FN;
   const int col0 = n0 + wn * (32 * FJ) + 4 * half;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -553,6 +565,23 @@ using TileN = Tile<64, 128, 4, 4>;
 using TileS = Tile<64, 64, 4, 4>;
 using TileSnt = Tile<64, 64, 4, 4, true>;
 using TileXS = Tile<32, 64, 4, 6, true>;
+// Unsplit bf16 products of at most SHORT_STAGES stages: waves with a smaller
+// wave tile each instead of wave groups that share K. The groups' exchange and
+// the deeper ring cost more than they give there: 64 x 1000 x 520 8.1 us on
+// 64 x 64 tiles of groups, 5.7 so; 33 x 64 x 64 4.1, 2.8; 128 x 9728 x 896 (64 x
+// 128 tiles) 11.6, 10.7; 256 x 9728 x 896 (128 x 128) 14.4, 13.6; from 24 stages on
+// the groups win (600 x 512 x 2048 10.5 against 11.4: a 32 x 32 wave tile reads
+// twice the LDS bytes). Many blocks want a short ring, so that more of them share
+// a CU: 33 x 151936 x 896 on 64 x 128 53.7 us with 3 stages, 59.0 with 4 (64 on
+// groups); 33 x 37888 x 3584, 592 blocks of 64 x 64, 55.7 with 2 stages, 58.1 with 4
+// (57.7 on groups and non-temporal loads), so one row tile of many blocks takes them too.
+constexpr int64_t SHORT_STAGES = 16;
+using TileS2w = Tile<64, 64, 1, 2, false, 1, 1, true>;
+using TileS2 = Tile<64, 64, 1, 2, false, 1, 1>;
+using TileS4 = Tile<64, 64, 1, 4, false, 1, 1>;
+using TileN3 = Tile<64, 128, 1, 3, false, 1, 1>;
+using TileN4 = Tile<64, 128, 1, 4, false, 1, 1>;
+using TileL3 = Tile<128, 128, 1, 3, false, 2, 1>;
 using TileS32 = Tile<64, 64, 4, 3>;
 using TileXS32 = Tile<32, 64, 4, 3, true>;
 
@@ -656,6 +685,16 @@ int launch_plan(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bi
     if constexpr (OUT == MINITP_EPI_NONE)
       if (p.kind == KIND_XL && p.S == 1 && stream_pays(M, N, K))
         return launch_stream<T, TileStream>(st, x, ldx, w, bias, y, ldy, M, N, K, state);
+    if constexpr (OUT == MINITP_EPI_NONE || OUT == MINITP_EPI_RESID) {
+      const int64_t stages = cdiv(K, 64), cus = device_cus();
+      const int64_t blocks = cdiv(M, TILE_COST[p.kind].bm) * cdiv(N, TILE_COST[p.kind].bn);
+      const bool shallow = stages <= SHORT_STAGES;
+      if (p.kind == KIND_S && stages <= 2) return go(TileS2w{});
+      if (p.kind == KIND_S && blocks > 2 * cus && (shallow || M <= S_NT_ROWS)) return go(TileS2{});
+      if (p.kind == KIND_S && shallow) return go(TileS4{});
+      if (p.kind == KIND_N && shallow) return blocks > cus ? go(TileN3{}) : go(TileN4{});
+      if (p.kind == KIND_L && shallow) return go(TileL3{});
+    }
     if (p.kind == KIND_XL) return go(TileXL{});
     if (p.kind == KIND_L) return go(TileL{});
     if (p.kind == KIND_N) return go(TileN{});

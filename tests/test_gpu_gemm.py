@@ -140,3 +140,17 @@ def test_linear_of_many_tiles_matches_float64(m, n, k):
     last row and column tiles not full, columns not in fours, a last round
     that some blocks sit out; the bar of the plain products."""
     test_linear_matches_float64(m, n, k, torch.bfloat16)
+
+
+@pytest.mark.parametrize("m,n,k", [(433, 64, 64), (33, 40000, 72), (1500, 2001, 128), (64, 2000, 136), (300, 901, 1024),
+                                   (64, 37893, 1096), (130, 9731, 896), (64, 50001, 1000), (250, 9730, 1000)])
+def test_linear_of_few_stages_matches_float64(m, n, k):
+    """Products of at most 16 stages on every tile shape (whole in the ring,
+    two to four stages, 64 x 64 to 128 x 128), and one row tile of many
+    blocks past that: ragged rows, columns and stages."""
+    test_linear_matches_float64(m, n, k, torch.bfloat16)
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 1001, 104), (129, 9731, 136), (300, 901, 896), (200, 9730, 1000)])
+def test_linear_resid_of_few_stages_matches_float64(m, n, k):
+    test_linear_resid_matches_float64(m, n, k)
