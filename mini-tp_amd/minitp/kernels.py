@@ -148,13 +148,20 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *
         ldy = out.stride(-2) if out.dim() > 1 else n_out
     dt = N.dtype_code(x.dtype)
     bias = bias.contiguous() if bias is not None else None
-    # (up to 32 bf16 rows and 1 fp32 row run as GEMVs, which need none)
-    need = _split_bytes(x.device, dt, m, n_out, w.shape[1], epilogue) if m > (1 if dt == N.F32 else 32) else 0
-    # (scratch of the call: from the caching allocator, on the current stream)
-    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need > 0 else None
+    need, ws = _split_scratch(x, dt, m, n_out, w.shape[1], epilogue)
     N.check(_lib().minitp_linear_ws(N.stream(), dt, xr.data_ptr(), ldx, w.data_ptr(), N.ptr(bias), out.data_ptr(), ldy,
-                                    m, n_out, w.shape[1], epilogue, N.ptr(aux), N.ptr(ws), max(need, 0)), "linear")
+                                    m, n_out, w.shape[1], epilogue, N.ptr(aux), N.ptr(ws), need), "linear")
     return out
+
+
+def _split_scratch(x: torch.Tensor, dtype: int, m: int, n: int, k: int, epilogue: int) -> tuple[int, torch.Tensor | None]:
+    """Scratch of a product that splits over K: from the caching allocator, on
+    the current stream. (Up to 8,192 elements a row, up to 32 bf16 rows and 1
+    fp32 row run as GEMVs, which need none: no lookup.)"""
+    if k <= 8192 and m <= (1 if dtype == N.F32 else 32):
+        return 0, None
+    need = max(_split_bytes(x.device, dtype, m, n, k, epilogue), 0)
+    return need, torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
 
 
 @functools.lru_cache(maxsize=4096)

@@ -37,6 +37,8 @@ SHAPES = [
     (4, 896, 4864),
     (2, 1153, 5120),
     (3, 64, 5128),
+    (2, 130, 8200),       # (bf16: two rows past the GEMVs, split over K)
+    (1, 70, 20488),
 ]
 
 
@@ -154,3 +156,40 @@ def test_linear_of_few_stages_matches_float64(m, n, k):
 @pytest.mark.parametrize("m,n,k", [(70, 1001, 104), (129, 9731, 136), (300, 901, 896), (200, 9730, 1000)])
 def test_linear_resid_of_few_stages_matches_float64(m, n, k):
     test_linear_resid_matches_float64(m, n, k)
+
+
+@pytest.mark.parametrize("room", [0, 16, 4 << 10])
+def test_linear_ws_with_less_than_the_split_workspace(room):
+    """A shape that splits over K, its workspace absent or too small: the
+    unsplit product."""
+    from minitp import _native as N
+
+    m, n, k = 40, 896, 4864
+    lib, dt = N.lib(), N.dtype_code(torch.bfloat16)
+    need = lib.minitp_linear_workspace_bytes(dt, m, n, k, N.EPI_NONE)
+    assert need > room
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=DEV) * 0.05).bfloat16()
+    ws = torch.empty(max(room, 16), dtype=torch.uint8, device=DEV)
+    y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    N.check(lib.minitp_linear_ws(N.stream(), dt, x.data_ptr(), k, w.data_ptr(), None, y.data_ptr(), n, m, n, k,
+                                 N.EPI_NONE, None, ws.data_ptr() if room else None, room), "linear")
+    ref = x.double() @ w.double().t()
+    assert ((y.double() - ref).abs() <= _bound(ref, x, w, torch.bfloat16, k)).all()
+
+
+@pytest.mark.parametrize("m,n,k,lo", [(40, 130, 264, 1), (300, 896, 520, 3), (33, 64, 4864, 2), (600, 1001, 200, 5)])
+def test_linear_into_columns_of_any_alignment(m, n, k, lo):
+    """``out`` a column slice whose base is not aligned to the four-column
+    stores: the product in the slice, its neighbours untouched."""
+    from minitp import kernels as K
+
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=DEV) * 0.05).bfloat16()
+    wide = torch.full((m, n + 12), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.linear(x, w, out=wide[:, lo:lo + n])
+    ref = x.double() @ w.double().t()
+    assert ((wide[:, lo:lo + n].double() - ref).abs() <= _bound(ref, x, w, torch.bfloat16, k)).all()
+    assert wide[:, :lo].isnan().all() and wide[:, lo + n:].isnan().all()
