@@ -111,6 +111,17 @@ int minitp_linear_ws(void* stream, int dtype, const void* x, int64_t ldx, const 
  * fused.py:102-104): minitp_linear + minitp_silu_mul in one kernel. */
 int minitp_gate_up_swiglu(void* stream, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
                           int64_t M, int64_t N, int64_t K);
+
+/* One row block of a packed projection as a product of its own (the unfused
+ * ablation forms, fused.py:63-74, 106-113): W is [N, K], N of the packed
+ * weight's `packed` rows, and y gets the bits that the call on the whole
+ * packed weight gives those outputs: minitp_linear_ws with its workspace, or
+ * (swiglu != 0, packed = 2 x its width) the gate or up rows that
+ * minitp_gate_up_swiglu rounds before SwiGLU. The workspace holds
+ * minitp_linear_workspace_bytes of the packed width (swiglu: none). */
+int minitp_linear_block(void* stream, int dtype, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
+                        int64_t ldy, int64_t M, int64_t N, int64_t K, int64_t packed, int swiglu, void* workspace,
+                        int64_t workspace_bytes);
 /* RMSNorm (layer.py:39-42) feeding a linear (the decoder layer's
  * input_layernorm -> qkv_proj and post_attention_layernorm -> gate_up_proj,
  * layer.py:60-67) in one pass over W: every block normalises the x rows it

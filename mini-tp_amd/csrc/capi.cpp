@@ -223,6 +223,24 @@ int minitp_gate_up_swiglu(void* stream, int dtype, const void* x, int64_t ldx, c
   return launch_gemm_swiglu(st, dtype, x, ldx, w, y, ldy, M, N, K);
 }
 
+int minitp_linear_block(void* stream, int dtype, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
+                        int64_t ldy, int64_t M, int64_t N, int64_t K, int64_t packed, int swiglu, void* workspace,
+                        int64_t workspace_bytes) {
+  int rc = linear_checks(dtype, x, ldx, w, bias, y, ldy, M, N, K, MINITP_EPI_NONE, nullptr);
+  if (rc || M == 0 || N == 0) return rc;
+  MINITP_CHECK_ARG(packed >= N && (!swiglu || packed % 2 == 0), "linear_block: N=%lld of %lld packed rows",
+                   (long long)N, (long long)packed);
+  const int64_t need = swiglu ? 0 : minitp_linear_workspace_bytes(dtype, M, packed, K, MINITP_EPI_NONE);
+  MINITP_CHECK_ARG(workspace_bytes >= need && (workspace != nullptr || need == 0) && aligned16(workspace),
+                   "linear_block: workspace %p of %lld bytes, %lld needed", workspace, (long long)workspace_bytes,
+                   (long long)need);
+  hipStream_t st = S(stream);
+  if (gemv_supported(dtype, M, K))
+    return launch_gemv(st, dtype, PRO_NONE, EPI_STORE, gemv_args(x, ldx, w, bias, y, ldy, M, N, K, nullptr));
+  return launch_gemm_block(st, dtype, x, ldx, w, bias, y, ldy, M, N, K, packed, swiglu != 0, need ? workspace : nullptr,
+                           need);
+}
+
 int minitp_rmsnorm_linear(void* stream, int dtype, const void* x, int64_t ldx, const void* norm_w, float eps,
                           const void* w, const void* bias, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
                           int epilogue, const void* aux) {

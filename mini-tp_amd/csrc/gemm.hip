@@ -675,6 +675,34 @@ int launch_stream(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* 
   return MINITP_OK;
 }
 
+// The tile of an unsplit product (no SwiGLU) of at most SHORT_STAGES stages, or
+// of one row tile and many blocks (TileS2w's group above): LONG_TILE for none.
+enum ShortTile { LONG_TILE, SHORT_S2W, SHORT_S2, SHORT_S4, SHORT_N3, SHORT_N4, SHORT_L3 };
+inline ShortTile short_tile(int kind, int64_t M, int64_t N, int64_t K) {
+  const int64_t stages = cdiv(K, 64), cus = device_cus();
+  const int64_t blocks = cdiv(M, TILE_COST[kind].bm) * cdiv(N, TILE_COST[kind].bn);
+  const bool few = stages <= SHORT_STAGES;
+  if (kind == KIND_S && stages <= 2) return SHORT_S2W;
+  if (kind == KIND_S && blocks > 2 * cus && (few || M <= S_NT_ROWS)) return SHORT_S2;
+  if (kind == KIND_S && few) return SHORT_S4;
+  if (kind == KIND_N && few) return blocks > cus ? SHORT_N3 : SHORT_N4;
+  if (kind == KIND_L && few) return SHORT_L3;
+  return LONG_TILE;
+}
+
+// Wave groups that share K in the tiles a plan runs on: with its splits, all
+// that the order of a product's sums depends on.
+static_assert(TileXL::WK == 2 && TileL::WK == 2 && TileN::WK == 4 && TileS::WK == 4 && TileSnt::WK == 4 &&
+                  TileXS::WK == 4 && TileS32::WK == 4 && TileXS32::WK == 4 && TileStream::WK == 1 && TileS4::WK == 1,
+              "plan_groups");
+inline int plan_groups(int dtype, const GemmPlan& p, int64_t M, int64_t N, int64_t K, bool swiglu) {
+  if (dtype == MINITP_F32 || p.kind == KIND_XS) return 4;
+  if (!swiglu && p.S == 1 &&
+      (p.kind == KIND_XL ? stream_pays(M, N, K) : short_tile(p.kind, M, N, K) != LONG_TILE))
+    return 1;
+  return p.kind == KIND_XL || p.kind == KIND_L ? 2 : 4;
+}
+
 template <typename T, int OUT>
 int launch_plan(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
                 int64_t N, int64_t K, const T* aux, const StepState* state, float* part, const GemmPlan& p) {
@@ -686,14 +714,15 @@ int launch_plan(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bi
       if (p.kind == KIND_XL && p.S == 1 && stream_pays(M, N, K))
         return launch_stream<T, TileStream>(st, x, ldx, w, bias, y, ldy, M, N, K, state);
     if constexpr (OUT == MINITP_EPI_NONE || OUT == MINITP_EPI_RESID) {
-      const int64_t stages = cdiv(K, 64), cus = device_cus();
-      const int64_t blocks = cdiv(M, TILE_COST[p.kind].bm) * cdiv(N, TILE_COST[p.kind].bn);
-      const bool shallow = stages <= SHORT_STAGES;
-      if (p.kind == KIND_S && stages <= 2) return go(TileS2w{});
-      if (p.kind == KIND_S && blocks > 2 * cus && (shallow || M <= S_NT_ROWS)) return go(TileS2{});
-      if (p.kind == KIND_S && shallow) return go(TileS4{});
-      if (p.kind == KIND_N && shallow) return blocks > cus ? go(TileN3{}) : go(TileN4{});
-      if (p.kind == KIND_L && shallow) return go(TileL3{});
+      switch (short_tile(p.kind, M, N, K)) {
+        case SHORT_S2W: return go(TileS2w{});
+        case SHORT_S2: return go(TileS2{});
+        case SHORT_S4: return go(TileS4{});
+        case SHORT_N3: return go(TileN3{});
+        case SHORT_N4: return go(TileN4{});
+        case SHORT_L3: return go(TileL3{});
+        case LONG_TILE: break;
+      }
     }
     if (p.kind == KIND_XL) return go(TileXL{});
     if (p.kind == KIND_L) return go(TileL{});
@@ -740,6 +769,35 @@ int gemm_typed(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bia
                : launch_plan<T, MINITP_EPI_NONE>(st, x, ldx, w, bias, y, ldy, M, N, K, aux, state, ws, p);
 }
 
+// One row block of a packed weight on the splits and wave groups of the whole,
+// the larger tile of those groups where it still gives every CU a block.
+template <typename T, int OUT>
+int launch_block_tile(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
+                      int64_t N, int64_t K, float* part, const GemmPlan& p, int groups) {
+  auto go = [&](auto cfg) {
+    return launch_cfg<T, decltype(cfg), OUT>(st, x, ldx, w, bias, y, ldy, M, N, K, nullptr, nullptr, part, p);
+  };
+  if constexpr (sizeof(T) == 4) {
+    return M <= XS_ROWS ? go(TileXS32{}) : go(TileS32{});
+  } else {
+    auto fills = [&](int64_t bm, int64_t bn) { return cdiv(M, bm) * cdiv(N, bn) * p.S >= device_cus(); };
+    if constexpr (OUT == MINITP_EPI_NONE)
+      if (groups == 1) return fills(128, 128) ? go(TileL3{}) : go(TileS4{});
+    if (groups == 2) return fills(256, 128) ? go(TileXL{}) : go(TileL{});
+    if (M <= XS_ROWS) return go(TileXS{});
+    return fills(64, 128) ? go(TileN{}) : M <= S_NT_ROWS ? go(TileSnt{}) : go(TileS{});
+  }
+}
+
+template <typename T>
+int launch_block(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
+                 int64_t N, int64_t K, const GemmPlan& p, int groups, float* ws) {
+  if (p.S == 1)
+    return launch_block_tile<T, MINITP_EPI_NONE>(st, x, ldx, w, bias, y, ldy, M, N, K, nullptr, p, groups);
+  const int rc = launch_block_tile<T, OUT_PARTIAL>(st, x, ldx, w, bias, y, ldy, M, N, K, ws, p, groups);
+  return rc ? rc : launch_reduce<T, MINITP_EPI_NONE>(st, ws, p.S, bias, y, ldy, nullptr, M, N, nullptr);
+}
+
 }  // namespace
 
 bool gemm_prefers_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy, bool swiglu, int64_t ws_bytes,
@@ -778,6 +836,32 @@ int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, co
                                               K, nullptr, nullptr, nullptr, p)
              : launch_plan<bf16, OUT_SWIGLU>(st, (const bf16*)x, ldx, (const bf16*)w, nullptr, (bf16*)y, ldy, M, N, K,
                                              nullptr, nullptr, nullptr, p);
+}
+
+// The 256 x 256 tiles add K in one sequence, as one wave group does.
+int launch_gemm_block(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
+                      int64_t ldy, int64_t M, int64_t N, int64_t K, int64_t packed, bool swiglu, void* ws,
+                      int64_t ws_bytes) {
+  if (M == 0 || N == 0) return MINITP_OK;
+  const int64_t es = dtype == MINITP_F32 ? 4 : 2, whole = swiglu ? packed / 2 : packed;
+  if (!gemm_operands_fit(M, N, K, ldx, es)) {
+    set_error("gemm: operands over 4 GiB (M=%lld N=%lld K=%lld)", (long long)M, (long long)N, (long long)K);
+    return MINITP_ERR_UNSUPPORTED;
+  }
+  const int64_t room = swiglu || ws == nullptr ? 0 : ws_bytes;
+  const float split_us = swiglu ? 0.f : REDUCE_US;
+  const bool tile = dtype == MINITP_BF16 && gemm_prefers_tile(M, whole, K, ldx, whole, swiglu, room, split_us);
+  const GemmPlan p = tile ? GemmPlan{KIND_S, 1, cdiv(K, 64) * 64, 0.f}
+                          : gemm_plan(dtype, M, whole, K, swiglu, room, split_us);
+  const int groups = tile ? 1 : plan_groups(dtype, p, M, whole, K, swiglu);
+  if (groups == 1 && dtype == MINITP_BF16 && aligned16(x) && aligned16(w) &&
+      gemm_tile_supported(M, N, K, ldx, ldy, false))
+    return launch_gemm_tile(st, x, ldx, w, bias, y, ldy, M, N, K, false);
+  return dtype == MINITP_F32
+             ? launch_block<float>(st, (const float*)x, ldx, (const float*)w, (const float*)bias, (float*)y, ldy, M, N,
+                                   K, p, groups, (float*)ws)
+             : launch_block<bf16>(st, (const bf16*)x, ldx, (const bf16*)w, (const bf16*)bias, (bf16*)y, ldy, M, N, K,
+                                  p, groups, (float*)ws);
 }
 
 int launch_gemm_partials(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, int64_t M, int64_t N,

@@ -159,6 +159,12 @@ int launch_gemm_partials(hipStream_t st, int dtype, const void* x, int64_t ldx, 
 // store and read them
 int launch_gemm_swiglu(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int64_t M,
                        int64_t N, int64_t K, TileTail tail = TileTail{nullptr, nullptr});
+// Rows [N] of a packed weight of `packed` rows, each sum over K added in the
+// order in which launch_gemm (swiglu: launch_gemm_swiglu) adds it for the whole
+// weight with this workspace: the same bits.
+int launch_gemm_block(hipStream_t st, int dtype, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
+                      int64_t ldy, int64_t M, int64_t N, int64_t K, int64_t packed, bool swiglu, void* ws,
+                      int64_t ws_bytes);
 // Workspace with which launch_gemm would split an M x N x K product over K
 // (0: it runs unsplit at any size); plain: MINITP_EPI_NONE, which the tile
 // kernel may serve.

@@ -46,6 +46,7 @@ SIGNATURES = {
     "minitp_linear_workspace_bytes": (_i64, [_int, _i64, _i64, _i64, _int]),
     "minitp_linear_ws": (_int, [_vp, _int, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _vp, _i64]),
     "minitp_gate_up_swiglu": (_int, [_vp, _int, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64]),
+    "minitp_linear_block": (_int, [_vp, _int, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _i64]),
     "minitp_rmsnorm_linear": (_int, [_vp, _int, _vp, _i64, _vp, _f32, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int,
                                      _vp]),
     "minitp_add_rmsnorm_linear_parts": (_int, [_vp, _int, _vp, _vp, _i32, _vp, _vp, _f32, _vp, _vp, _i64, _i64,

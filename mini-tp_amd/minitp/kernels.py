@@ -170,6 +170,25 @@ def _split_bytes(device: torch.device, dtype: int, m: int, n: int, k: int, epilo
     return _lib().minitp_linear_workspace_bytes(dtype, m, n, k, epilogue)
 
 
+def linear_block(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, packed: int,
+                 swiglu: bool = False) -> torch.Tensor:
+    """linear(x, w, bias) into ``out`` for one row block ``w`` of a packed
+    weight of ``packed`` rows: the bits that ``linear`` on the whole packed
+    weight gives these outputs (``swiglu``: those ``gate_up_swiglu`` rounds)."""
+    N.require_gpu(x, w, bias, what="linear")
+    if x.dtype != w.dtype or (bias is not None and bias.dtype != w.dtype):
+        raise TypeError(f"linear: dtype mismatch x={x.dtype} w={w.dtype}")
+    w = w.contiguous()
+    xr, m, ldx = _as_rows(x)
+    dt, k = N.dtype_code(x.dtype), w.shape[1]
+    bias = bias.contiguous() if bias is not None else None
+    need, ws = (0, None) if swiglu else _split_scratch(x, dt, m, packed, k, N.EPI_NONE)
+    N.check(_lib().minitp_linear_block(N.stream(), dt, xr.data_ptr(), ldx, w.data_ptr(), N.ptr(bias), out.data_ptr(),
+                                       out.stride(-2) if out.dim() > 1 else w.shape[0], m, w.shape[0], k, packed,
+                                       int(swiglu), N.ptr(ws), need), "linear")
+    return out
+
+
 def gate_up_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up of linear(x, w) for w = [gate; up], as ``linear`` then
     ``silu_mul`` round them, in one kernel."""

@@ -24,7 +24,8 @@ class TPQwen2MLP(nn.Module):
     def forward(self, x):
         n = self.intermediate_local
         gu = self.gate_up_proj
-        if self.use_fused_gateup and gu.bias is None and 2 * gu.weight.numel() * gu.weight.element_size() < 1 << 32:
+        one = gu.bias is None and 2 * gu.weight.numel() * gu.weight.element_size() < 1 << 32
+        if self.use_fused_gateup and one:
             return self.down_proj(K.gate_up_swiglu(x, gu.weight))
-        y = gu.project(x, fused=self.use_fused_gateup)
+        y = gu.project(x, fused=self.use_fused_gateup, swiglu=one)
         return self.down_proj(K.silu_mul(y[..., :n], y[..., n:]))

@@ -1,9 +1,10 @@
 """Packed projections: one GEMV/GEMM over [q; k; v] or [gate; up] rows
 (minitp/parallel/fused.py:26-113). The split afterwards is a zero-copy view.
 
-The unfused ablation forms run one kernel per row block, written into
-column slices of one output buffer, so the values are identical and only
-the kernel count differs (fused.py:63-74, 106-113).
+The unfused ablation forms run one product per row block, written into
+column slices of one output buffer and summed in the packed product's order,
+so the values are identical and only the kernel count differs
+(fused.py:63-74, 106-113).
 """
 
 from __future__ import annotations
@@ -48,7 +49,8 @@ class FusedQKVColumnParallelLinear(nn.Module):
         q, kv = self.q_out_local, self.kv_out_local
         b = self.bias
         for lo, hi in ((0, q), (q, q + kv), (q + kv, q + 2 * kv)):
-            K.linear(x, self.weight[lo:hi], b[lo:hi] if b is not None else None, out=y[..., lo:hi])
+            K.linear_block(x, self.weight[lo:hi], b[lo:hi] if b is not None else None, y[..., lo:hi],
+                           self.weight.shape[0])
         return y
 
     def forward(self, x: torch.Tensor):
@@ -75,14 +77,16 @@ class FusedGateUpColumnParallelLinear(nn.Module):
         if init_weights:
             nn.init.kaiming_uniform_(self.weight, a=5 ** 0.5)
 
-    def project(self, x: torch.Tensor, fused: bool = True) -> torch.Tensor:
+    def project(self, x: torch.Tensor, fused: bool = True, swiglu: bool = False) -> torch.Tensor:
+        """[gate, up] (fused: one product; else two). ``swiglu``: the unfused
+        values are those ``K.gate_up_swiglu`` rounds, not the packed product's."""
         if fused:
             return K.linear(x, self.weight, self.bias)
         n = self.intermediate_local
         y = torch.empty(*x.shape[:-1], 2 * n, dtype=x.dtype, device=x.device)
         b = self.bias
         for lo, hi in ((0, n), (n, 2 * n)):
-            K.linear(x, self.weight[lo:hi], b[lo:hi] if b is not None else None, out=y[..., lo:hi])
+            K.linear_block(x, self.weight[lo:hi], b[lo:hi] if b is not None else None, y[..., lo:hi], 2 * n, swiglu)
         return y
 
     def forward(self, x: torch.Tensor):

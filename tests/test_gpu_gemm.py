@@ -158,6 +158,40 @@ def test_linear_resid_of_few_stages_matches_float64(m, n, k):
     test_linear_resid_matches_float64(m, n, k)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden,inter,heads,kv_heads,head_dim", [(896, 4864, 14, 2, 64), (3584, 18944, 28, 4, 128),
+                                                                  (264, 136, 4, 2, 32)])
+def test_unfused_projections_give_the_packed_ones_bits(hidden, inter, heads, kv_heads, head_dim, dtype):
+    """Row blocks of the packed QKV and gate/up weights as products of their
+    own against the packed products, and the MLP with and without its fused
+    gate/up: bitwise, at row counts on every form the packed product takes."""
+    from minitp.config import ModelConfig
+    from minitp.distributed.context import ParallelContext
+    from minitp.mlp import TPQwen2MLP
+    from minitp.parallel.fused import FusedQKVColumnParallelLinear
+
+    cfg = ModelConfig(hidden, inter, 1, heads, kv_heads, head_dim, 128, 1e-6, 1e6, 64)
+    ctx = ParallelContext(0, 0, 1, 0, 1, torch.device(DEV), None)
+    g = torch.Generator(device=DEV).manual_seed(hidden)
+    with torch.device(DEV):
+        qkv = FusedQKVColumnParallelLinear(hidden, heads * head_dim, kv_heads * head_dim, ctx).to(dtype)
+        mlp = TPQwen2MLP(cfg, ctx).to(dtype)
+    with torch.no_grad():
+        for p in [*qkv.parameters(), *mlp.parameters()]:
+            p.copy_(torch.randn(p.shape, generator=g, device=DEV) * 0.02)
+        for m in (1, 2, 3, 4, 5, 32, 33, 48, 65, 100, 157, 300, 433, 512, 700, 1099, 2100, 4096):
+            if dtype == torch.float32 and m * hidden * inter > 1.2e11:
+                continue
+            x = torch.randn(m, hidden, generator=g, device=DEV).to(dtype)
+            assert torch.equal(qkv.project(x), qkv.project(x, fused=False)), ("qkv", m)
+            gu = mlp.gate_up_proj
+            assert torch.equal(gu.project(x), gu.project(x, fused=False)), ("gate_up", m)
+            outs = []
+            for mlp.use_fused_gateup in (True, False):
+                outs.append(mlp(x))
+            assert torch.equal(*outs), ("mlp", m)
+
+
 @pytest.mark.parametrize("room", [0, 16, 4 << 10])
 def test_linear_ws_with_less_than_the_split_workspace(room):
     """A shape that splits over K, its workspace absent or too small: the
