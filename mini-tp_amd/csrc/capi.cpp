@@ -188,7 +188,7 @@ int minitp_linear(void* stream, int dtype, const void* x, int64_t ldx, const voi
 int64_t minitp_linear_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int epilogue) {
   if (!dtype_ok(dtype) || M < 0 || N < 0 || K <= 0 || epilogue < MINITP_EPI_NONE || epilogue > MINITP_EPI_SWIGLU)
     return -1;
-  if (M == 0 || N == 0 || epilogue == MINITP_EPI_SWIGLU || gemv_supported(dtype, M, K)) return 0;
+  if (M == 0 || N == 0 || epilogue == MINITP_EPI_SWIGLU || gemv_serves(dtype, M, N, K)) return 0;
   return gemm_split_bytes(dtype, M, N, K, epilogue == MINITP_EPI_NONE);
 }
 
@@ -200,7 +200,7 @@ int minitp_linear_ws(void* stream, int dtype, const void* x, int64_t ldx, const 
   MINITP_CHECK_ARG(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0) && aligned16(workspace),
                    "linear: workspace %p of %lld bytes", workspace, (long long)workspace_bytes);
   hipStream_t st = S(stream);
-  if (epilogue == MINITP_EPI_SWIGLU ? gemv_entry_rows(dtype, M, K) : gemv_supported(dtype, M, K))
+  if (epilogue == MINITP_EPI_SWIGLU ? gemv_entry_rows(dtype, M, K) : gemv_serves(dtype, M, N, K))
     return launch_gemv(st, dtype, PRO_NONE, gemv_epilogue(epilogue), gemv_args(x, ldx, w, bias, y, ldy, M, N, K, aux));
   if (epilogue == MINITP_EPI_SWIGLU) {
     if (dtype == MINITP_BF16 && bias == nullptr && aligned16(x) && aligned16(w) &&
@@ -218,7 +218,7 @@ int minitp_gate_up_swiglu(void* stream, int dtype, const void* x, int64_t ldx, c
   int rc = linear_checks(dtype, x, ldx, w, nullptr, y, ldy, M, N, K, MINITP_EPI_NONE, nullptr);
   if (rc || M == 0 || N == 0) return rc;
   hipStream_t st = S(stream);
-  if (gemv_supported(dtype, M, K))
+  if (gemv_serves(dtype, M, 2 * N, K))
     return launch_gemv(st, dtype, PRO_NONE, EPI_SWIGLU, gemv_args(x, ldx, w, nullptr, y, ldy, M, N, K, nullptr));
   return launch_gemm_swiglu(st, dtype, x, ldx, w, y, ldy, M, N, K);
 }
@@ -235,7 +235,7 @@ int minitp_linear_block(void* stream, int dtype, const void* x, int64_t ldx, con
                    "linear_block: workspace %p of %lld bytes, %lld needed", workspace, (long long)workspace_bytes,
                    (long long)need);
   hipStream_t st = S(stream);
-  if (gemv_supported(dtype, M, K))
+  if (gemv_serves(dtype, M, packed, K))
     return launch_gemv(st, dtype, PRO_NONE, EPI_STORE, gemv_args(x, ldx, w, bias, y, ldy, M, N, K, nullptr));
   return launch_gemm_block(st, dtype, x, ldx, w, bias, y, ldy, M, N, K, packed, swiglu != 0, need ? workspace : nullptr,
                            need);

@@ -2104,7 +2104,7 @@ int pick_k(hipStream_t st, const GemvArgs& a) {
   if constexpr (MM == 1 && PRO == PRO_NONE && (EPI == EPI_STORE || EPI == EPI_RESID || EPI == EPI_SWIGLU))
     if (use_split<T, PRO, EPI>(a)) return launch_split<T, MM, EPI>(st, a);
   if (nchunk <= 128) return launch_reg<T, MM, 1, 2, PRO, EPI>(st, a);
-  if constexpr (MM == 4 && sizeof(T) == 4) {
+  if constexpr (MM == 4 && sizeof(T) == 4 && EPI != EPI_ARGMAX) {
     if (nchunk <= F32_NORM_CHUNKS) return launch_reg<T, MM, 2, 2, PRO, EPI>(st, a);
   }
   if constexpr (MM > 1 && sizeof(T) == 4 && PRO == PRO_NONE &&
@@ -2235,6 +2235,19 @@ bool gemv_entry_rows(int dtype, int64_t M, int64_t K) {
 bool gemv_supported(int dtype, int64_t M, int64_t K) {
   if (gemv_entry_rows(dtype, M, K)) return true;
   return dtype == MINITP_F32 && M >= 2 && M <= 4 && K % 4 == 0 && K / 4 <= F32_MAX_CHUNKS;
+}
+
+// Plain products that run as GEMVs rather than on the GEMM, for a weight of
+// `rows` rows. fp32 rows 3 and 4 of 257 to 640 chunks leave half of the register
+// form's lanes (1,280 chunks) without work, which costs more than the GEMM's
+// 32-row tile once the weight is large: K = 1,536 at 3 rows 81 us against 48
+// for 37,888 outputs and 302 against 149 (266 on the GEMM before the ring) for
+// 151,936; K = 1,028 25.5 against 17.0 for 9,728, but 9.3 against 15.7 for 2,052; K =
+// 2,048 39.5 against 41.5 for 16,388 and 45.8 against 42.4 for 18,944. K = 896 (93.6
+// against 94.1 for 151,936) and 3,584 up: within 15 % either way.
+bool gemv_serves(int dtype, int64_t M, int64_t rows, int64_t K) {
+  if (!gemv_supported(dtype, M, K)) return false;
+  return !(dtype == MINITP_F32 && M > 2 && K / 4 > F32_NORM_CHUNKS && K / 4 <= 640 && rows > 18432);
 }
 
 // The RMSNorm prologue holds a wave's whole K range: on the MFMA form that

@@ -111,6 +111,7 @@ int launch_gemv_part_swiglu(hipStream_t st, int dtype, const GemvArgs& a);
 int64_t gemv_argmax_partials(int64_t N);
 int launch_gemv(hipStream_t st, int dtype, int pro, int epi, const GemvArgs& a);
 bool gemv_supported(int dtype, int64_t M, int64_t K);
+bool gemv_serves(int dtype, int64_t M, int64_t rows, int64_t K);
 bool gemv_entry_rows(int dtype, int64_t M, int64_t K);
 // bf16 rows MF_MIN_ROWS..32 run the MFMA forms (16-row operand tiles, rows
 // past M read as zeros); fewer rows and fp32 the register forms. At 3 and 4

@@ -416,8 +416,9 @@ struct Qwen2Program {
       if ((rc = launch_gemv(st, c.dtype, PRO_NONE, EPI_RESID, d))) return rc;
     }
     // ---- final norm, LM head, greedy pick ----------------------------------------
-    // (fp32 rows past the entry forms' keep their LM head on the GEMM: 0.5B
-    // batch 3 91 us, 147 on the register GEMV)
+    // (fp32 rows past the entry forms' keep their last-position LM head on the
+    // GEMM: 0.5B batch 3 91 us, 147 on the register GEMV with its argmax; every
+    // position's logits of as few rows, below, 97 on the GEMV, 93 and a norm on the GEMM)
     if (!s.logits_all && gemv_entry_rows(c.dtype, B, H) && !gemv_mfma_rows(c.dtype, B)) {
       GemvArgs g{};
       g.x = (const char*)w.x + (T - 1) * H * es();  // last position of each row

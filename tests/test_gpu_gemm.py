@@ -37,6 +37,8 @@ SHAPES = [
     (4, 896, 4864),
     (2, 1153, 5120),
     (3, 64, 5128),
+    (3, 18433, 1032),     # (fp32: the GEMM's side of the line at 18,432 rows of the weight)
+    (4, 18432, 2560),
     (2, 130, 8200),       # (bf16: two rows past the GEMVs, split over K)
     (1, 70, 20488),
 ]
