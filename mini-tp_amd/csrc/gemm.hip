@@ -351,8 +351,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
   }
 }
 
-// The same products as gemm_kernel without a K split or wave groups, for many
-// tiles of few stages: a block walks its share of tiles and the ring of stages
+// The same products as gemm_kernel without a K split or wave groups, for one row
+// tile and many column tiles of few stages: a block walks its share of tiles and the ring of stages
 // runs on across them, so that a tile's epilogue and the next one's first
 // loads overlap (gemm_kernel drains its ring and refills it for every tile:
 // 0.5B LM head of 194 rows 107 us, 5 tiles of 14 stages a block; 97 so, bound
@@ -364,8 +364,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
 template <typename T, typename C>
 __global__ __launch_bounds__(C::THREADS) void gemm_stream_kernel(const T* __restrict__ x, int64_t ldx,
                                                                  const T* __restrict__ w, const T* __restrict__ bias,
-                                                                 T* y, int64_t ldy, int M, int N, int K, int tiles_m,
-                                                                 int tiles_n, int items, const StepState* state) {
+                                                                 T* y, int64_t ldy, int M, int N, int K, int items,
+                                                                 const StepState* state) {
   constexpr int BM = C::BM, BN = C::BN, STAGES = C::STAGES, PPW = C::PPW;
   constexpr int FM = C::FM, WN = C::WN, ROWB = C::ROWB, ES = (int)sizeof(T), V = 16 / ES, TK = KCH * V;
   static_assert(C::WK == 1, "a wave tile is one wave's");
@@ -380,30 +380,22 @@ __global__ __launch_bounds__(C::THREADS) void gemm_stream_kernel(const T* __rest
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN % C::WM, wn = wave % WN;
-  auto place = [&](int t, int& m0, int& n0) {
-    const int group = t / (8 * tiles_n), first_m = group * 8, gsz = min(tiles_m - first_m, 8);
-    const int in_group = t - group * 8 * tiles_n;
-    m0 = (first_m + in_group % gsz) * BM;
-    n0 = in_group / gsz * BN;
-  };
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   constexpr int A_BYTES = BM * ROWB;
   auto swz = [](int r) { return (r >> 1) & 7; };
 
   // ---- the load side: the tile whose stages are being issued -----------------
-  u32x4 xq, wq;
+  const uint32_t x_bytes = (uint32_t)(((int64_t)(M - 1) * ldx + K) * ES);
+  const uint32_t x_pad = x_bytes <= ROW_OOB ? ROW_OOB : (uint32_t)((int64_t)(M - 1) * ldx * ES);
+  const u32x4 xq = rsrc_span(x, x_bytes);
+  u32x4 wq;
   uint32_t voff[PPW];
   int kc[PPW];
   auto setup = [&](int t) {
-    int m0, n0;
-    place(t, m0, n0);
-    const int x_rows = min(M - m0, BM);
+    const int n0 = t * BN;
     const int64_t w_rows = min(N - n0, BN);
-    const uint32_t x_bytes = (uint32_t)(((int64_t)(x_rows - 1) * ldx + K) * ES);
     const uint32_t w_bytes = (uint32_t)(w_rows * K * ES);
-    xq = rsrc_span(x + (int64_t)m0 * ldx, x_bytes);
     wq = rsrc_span(w + (int64_t)n0 * K, w_bytes);
-    const uint32_t x_pad = x_bytes <= ROW_OOB ? ROW_OOB : (uint32_t)((int64_t)(x_rows - 1) * ldx * ES);
     const uint32_t w_pad = w_bytes <= ROW_OOB ? ROW_OOB : 0u;
 #pragma unroll
     for (int j = 0; j < PPW; ++j) {
@@ -413,7 +405,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_stream_kernel(const T* __rest
       const int c = (lane % KCH) ^ swz(r);
       kc[j] = c * V;
       if (!is_w) {
-        voff[j] = r < x_rows ? (uint32_t)(((int64_t)r * ldx + c * V) * ES) : x_pad;
+        voff[j] = r < M ? (uint32_t)(((int64_t)r * ldx + c * V) * ES) : x_pad;
       } else {
         voff[j] = n0 + r < N ? (uint32_t)(((int64_t)r * K + c * V) * ES) : w_pad;
       }
@@ -477,13 +469,12 @@ __global__ __launch_bounds__(C::THREADS) void gemm_stream_kernel(const T* __rest
       rd = rd + 1 == STAGES ? 0 : rd + 1;
       wr_stage = wr_stage + 1 == STAGES ? 0 : wr_stage + 1;
     }
-    int m0, n0;
-    place(first + li, m0, n0);
+    const int n0 = (first + li) * BN;
     const bool quads = N % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & (4 * sizeof(T) - 1)) == 0;
     const int col0 = n0 + wn * 64 + 4 * half;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int64_t row = m0 + wm * (32 * FM) + i * 32 + (lane & 31);
+      const int64_t row = wm * (32 * FM) + i * 32 + (lane & 31);
       if (row >= M) continue;
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -653,24 +644,24 @@ int launch_cfg(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bia
   return MINITP_OK;
 }
 
-// Two rounds of 256 x 128 tiles and more, of at most 32 stages: the running
+// One row tile, two rounds of 256 x 128 tiles and more, of at most 32 stages (more
+// row tiles run on the 256 x 256 ones): the running
 // ring saves about 4.5 us a tile and its eight waves lose 0.12 a stage against
 // gemm_kernel's sixteen (N = 151,936, K = 896, 14 stages: 150 rows 99.5 -> 86.5
 // us, 194 rows 107 -> 97, 250 rows 119.6 -> 105; N = 152,064, K = 3,584, 56
 // stages, 200 rows: 307 against 318).
 inline bool stream_pays(int64_t M, int64_t N, int64_t K) {
-  return cdiv(M, 256) * cdiv(N, 128) >= 2 * (int64_t)device_cus() && K <= 2048;
+  return M <= TileStream::BM && cdiv(N, TileStream::BN) >= 2 * (int64_t)device_cus() && K <= 2048;
 }
 
 template <typename T, typename C>
 int launch_stream(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bias, T* y, int64_t ldy, int64_t M,
                   int64_t N, int64_t K, const StepState* state) {
   if (const int rc = ensure_lds_limit((const void*)gemm_stream_kernel<T, C>, C::RING_BYTES)) return rc;
-  const int tiles_m = (int)cdiv(M, C::BM), tiles_n = (int)cdiv(N, C::BN);
-  const int64_t items = (int64_t)tiles_m * tiles_n;
+  const int64_t items = cdiv(N, C::BN);
   const dim3 grid((unsigned)(8 * cdiv(std::min<int64_t>(items, device_cus()), 8)));
   hipLaunchKernelGGL((gemm_stream_kernel<T, C>), grid, dim3(C::THREADS), C::RING_BYTES, st, x, ldx, w, bias, y, ldy,
-                     (int)M, (int)N, (int)K, tiles_m, tiles_n, (int)items, state);
+                     (int)M, (int)N, (int)K, (int)items, state);
   MINITP_LAUNCH_CHECK();
   return MINITP_OK;
 }

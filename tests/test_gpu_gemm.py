@@ -138,11 +138,14 @@ def test_swiglu_forms_agree_with_the_module(tokens):
         torch.testing.assert_close(a, b, atol=0.05, rtol=0.02)
 
 
-@pytest.mark.parametrize("m,n,k", [(250, 65700, 200), (194, 65665, 264), (255, 98432, 896), (300, 65664, 72)])
+@pytest.mark.parametrize("m,n,k", [(250, 65700, 200), (194, 65665, 264), (255, 98432, 896), (256, 65664, 1000),
+                                   (201, 131001, 8), (195, 80001, 72), (133, 131002, 136)])
 def test_linear_of_many_tiles_matches_float64(m, n, k):
     """Products whose blocks walk several tiles on one running ring of stages:
-    last row and column tiles not full, columns not in fours, a last round
-    that some blocks sit out; the bar of the plain products."""
+    one row tile, full and not, a last column tile not full, columns not in
+    fours, one to sixteen stages a tile (fewer than the ring's and odd counts
+    among them), a last round that some blocks sit out; the bar of the plain
+    products."""
     test_linear_matches_float64(m, n, k, torch.bfloat16)
 
 
