@@ -138,17 +138,12 @@ __global__ __launch_bounds__(C::THREADS) void gemm_kernel(const T* __restrict__ 
   const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per_xcd || item >= items) return;
   const int tiles = tiles_m * tiles_n;
-  // (no division where the quotient is known: the three take 50 to 100 ns ahead
-  // of the first load)
-  int z = 0, group = 0;
-  if (items != tiles) z = item / tiles;
-  const int t = item - z * tiles;
-  if (tiles_m > 8) group = t / (8 * tiles_n);
-  const int first_m = group * 8, gsz = min(tiles_m - first_m, 8);
+  // (straight-line divisions: branches around those whose quotient is known saved
+  // one row tile 70 ns and cost the others up to 0.7 us, 433 x 3584 x 3584 26.9 -> 27.6)
+  const int z = item / tiles, t = item - z * tiles;
+  const int group = t / (8 * tiles_n), first_m = group * 8, gsz = min(tiles_m - first_m, 8);
   const int in_group = t - group * 8 * tiles_n;
-  int tn = in_group;
-  if (gsz > 1) tn = in_group / gsz;
-  const int m0 = (first_m + in_group - tn * gsz) * BM;
+  const int m0 = (first_m + in_group % gsz) * BM, tn = in_group / gsz;
   const int kb = z * kper, ke = min(kb + kper, K);
 
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
@@ -648,8 +643,9 @@ int launch_cfg(hipStream_t st, const T* x, int64_t ldx, const T* w, const T* bia
 // row tiles run on the 256 x 256 ones): the running
 // ring saves about 4.5 us a tile and its eight waves lose 0.12 a stage against
 // gemm_kernel's sixteen (N = 151,936, K = 896, 14 stages: 150 rows 99.5 -> 86.5
-// us, 194 rows 107 -> 97, 250 rows 119.6 -> 105; N = 152,064, K = 3,584, 56
-// stages, 200 rows: 307 against 318).
+// us, 194 rows 107 -> 97, 250 rows 119.6 -> 105; N = 152,064, 200 rows: K = 1,536
+// 157 against 152, 2,048 199.5 and 196.9, 2,560 235 and 239, 3,584 307 and 321; N =
+// 98,304 crosses between 2,048 and 2,560 too).
 inline bool stream_pays(int64_t M, int64_t N, int64_t K) {
   return M <= TileStream::BM && cdiv(N, TileStream::BN) >= 2 * (int64_t)device_cus() && K <= 2048;
 }

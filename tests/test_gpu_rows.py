@@ -74,7 +74,7 @@ def test_silu_mul_matches_float64(rows, n, pad, dtype):
 
 @pytest.mark.parametrize("dtype,atol", [(torch.float32, 2e-5), (torch.bfloat16, 0.05)])
 @pytest.mark.parametrize("batch,tokens", [(2, 1), (3, 1), (31, 1), (33, 1), (48, 1), (65, 1), (1, 31), (2, 17),
-                                          (1, 70), (3, 100), (2, 400)])
+                                          (1, 70), (3, 100), (2, 400), (1, 3), (2, 2), (1, 4)])
 @pytest.mark.parametrize("shape", ["05b", "7b"])
 def test_forward_matches_the_module_path(shape, batch, tokens, dtype, atol):
     """Two layers at the model's widths on a cache already holding PAST rows.
