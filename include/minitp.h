@@ -127,7 +127,8 @@ int minitp_linear_block(void* stream, int dtype, const void* x, int64_t ldx, con
  * layer.py:60-67) in one pass over W: every block normalises the x rows it
  * needs (fp32, rounded to dtype) and streams its share of W. Arguments as
  * minitp_linear plus norm_w [K] and eps. Serves the decode shapes only
- * (M <= 4 rows, M == 1 up to K = 20480; bf16 5..32 rows up to K = 1024);
+ * (fp32 M <= 4 up to K = 512; M <= 2 up to 4096 fp32, 8192 bf16; M == 1 up
+ * to 20480; bf16 3..32 rows up to 1024);
  * others return
  * MINITP_ERR_UNSUPPORTED (use minitp_rmsnorm, then minitp_linear). The norm
  * sums x^2 in a different order than minitp_rmsnorm, so the two agree to

@@ -9,10 +9,10 @@ bits of a direct run (MINITP_PREFILL_GRAPH=0 when the program is created).
 Shapes: the 0.5B layer shape with 2 layers at batch 1 and 3 (LM-head GEMV +
 argmax) and 8 (the MFMA norm + LM-head GEMV of 5-32 rows, then argmax); the
 fused GEMV path of a short prompt (batch 1, 8 tokens); the LM-head GEMM of 40
-rows; and prompts whose products run on the 256 x 256 tile GEMM with its split
-last round (0.5B, 3 x 256 tokens) and its every-tile split (the 7B layer
-shape at 512 tokens), whose partials and arrival words live in the step
-state."""
+rows; and prompts whose products run on larger tiles (0.5B, 3 x 256 tokens; the
+7B layer shape at 512 tokens: the 256 x 256 tile GEMM, a last round split over K
+where it pays, and smaller tiles split over K), whose partials and arrival
+words live in the workspace and the step state."""
 
 import dataclasses
 
@@ -120,9 +120,9 @@ def test_prefill_graphs_of_one_shape_keep_the_attention_form_apart(shape, monkey
 def test_prefill_graph_replays_other_launch_paths_bitwise(shape, batch, tokens, monkeypatch):
     """Three prompts of one shape (direct, recorded, replayed) against direct
     runs, bitwise: the fused short-prompt GEMVs (1 x 8), the LM-head GEMM
-    that reads its logits pointer from the step state (40 rows), and the tile
-    GEMM's split last round and every-tile split (3 x 256 at 0.5B; 512 tokens
-    at 7B), which keep their arrival words and partials in the step state."""
+    that reads its logits pointer from the step state (40 rows), and the larger
+    tiles and K splits (3 x 256 at 0.5B; 512 tokens at 7B), which keep their
+    arrival words and partials in the step state and the workspace."""
     cfg, (graphed, _), (direct, _) = _models(monkeypatch, shape)
     g = torch.Generator().manual_seed(batch * 1000 + tokens)
     prompts = [torch.randint(0, cfg.vocab_size, (batch, tokens), generator=g).to(DEV) for _ in range(3)]

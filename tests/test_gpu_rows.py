@@ -2,8 +2,8 @@
 csrc/rope.hip): RMSNorm on vector pieces against float64 at the edges of what
 stays in registers, SwiGLU on ragged strides, and forwards whose products are
 split over K (their partials added by the consuming kernel) against the
-module path, whose products choose their own splits, at every row count where the tile or the
-split changes.
+module path, whose products choose their own splits, at every row count where
+the tile or the split changes.
 """
 
 import dataclasses
