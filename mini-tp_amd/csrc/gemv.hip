@@ -1366,7 +1366,9 @@ constexpr int MF_ONE = 8;
 #ifndef MINITP_MF_LOOP_STAGE
 #define MINITP_MF_LOOP_STAGE 1
 #endif
-template <int PRO, int EPI, int WAUX>
+// (TAIL: a SwiGLU width that is no multiple of a tuple. A pair count per tuple in
+// the whole-tuple form too costs the batch-32 gate/up 0.05 of its 8.35 us.)
+template <int PRO, int EPI, int WAUX, bool TAIL = false>
 __global__ __launch_bounds__(256) void gemv_mfma_loop_kernel(GemvArgs a) {
   static_assert(EPI == EPI_STORE || EPI == EPI_SWIGLU, "the tuple loop serves the store and SwiGLU epilogues");
   constexpr int MF_LOOP_PD = MINITP_MF_LOOP_PD;  // tuples whose weight loads are in flight
@@ -1521,8 +1523,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_loop_kernel(GemvArgs a) {
     // (lane nidx + 8); plain store: every lane finishes its own column
     const int p = nidx & (P16 - 1);
     const int64_t row_a = EPI == EPI_STORE ? (nidx < P16 ? ra + p : rb + p) : ra + p;
-    // (pairs of the tuple: the last one's may be fewer)
-    const int pairs = EPI == EPI_SWIGLU ? (int)std::min<int64_t>(P16, a.N - ra) : P16;
+    const int pairs = TAIL ? min(P16, (int)a.N - (int)t * P16) : P16;
     const bool oka = (EPI == EPI_STORE || nidx < pairs) && row_valid<EPI>(row_a, a);
     float bias_a = 0.f;
     if constexpr (EPI == EPI_STORE)  // a zero-length resource reads zeros
@@ -1953,6 +1954,8 @@ int launch_mfma_nt(hipStream_t st, const GemvArgs& a, int64_t ntup) {
       // stream stays non-temporal: 53 against 58 us at batch 32, kernel trace)
       auto kern = a.M > MINITP_MF_PLAIN_ROWS && EPI == EPI_SWIGLU ? gemv_mfma_loop_kernel<PRO, EPI, 0>
                                                                   : gemv_mfma_loop_kernel<PRO, EPI, AUX_NT>;
+      if constexpr (EPI == EPI_SWIGLU)
+        if (a.N % P16 != 0) kern = gemv_mfma_loop_kernel<PRO, EPI, AUX_NT, true>;
       const int lds = 4 * MF_X_STAGE;
       const int rc = ensure_lds_limit((const void*)kern, lds);
       if (rc) return rc;
