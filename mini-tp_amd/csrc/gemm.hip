@@ -2,10 +2,10 @@
 //
 // MFMA tiling for CDNA4 (wave64). A block owns a BM x BN output tile (32 x 64
 // to 256 x 128) made of 64 x 64 wave tiles (2 x 2 MFMA accumulators of
-// 32 x 32; 32 x 64 wave tiles for few rows), with WK waves sharing each wave
-// tile's K: wave group g takes every WK-th
-// 16-byte substep of a stage and the groups' sums are added in group order at
-// the end (a fixed order). Both operands are K-contiguous in memory (x rows
+// 32 x 32; 32 x 64 wave tiles for few rows; 32 x 32 and 64 x 32 ones for
+// products of few stages), with WK waves sharing each wave tile's K (one for
+// few stages): wave group g takes every WK-th 16-byte substep of a stage and
+// the groups' sums are added in group order at the end (a fixed order). Both operands are K-contiguous in memory (x rows
 // and W rows), the layout the MFMA fragments want, so nothing is transposed:
 //   bf16: v_mfma_f32_32x32x16_bf16 (8 bf16 per lane and operand, k = 8*(lane/32)+i)
 //   fp32: 4 x v_mfma_f32_32x32x2f32 per 16 bytes (lane half h holds k 4h .. 4h+3
